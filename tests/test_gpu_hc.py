@@ -291,3 +291,40 @@ def test_hc_one_launch_consecutive_and_graph(lib, H, with_inject, fused):
     assert after.value == before.value, (before.value, after.value)
     st.destroy()
     qfm.init(2560, 640, 512, 10, 1, 1)
+
+
+@pytest.mark.parametrize("H,T,with_inject,alias", [(2048, 5, True, False), (2560, 15, True, True),
+                                                   (2048, 16, False, False), (2560, 17, True, False),
+                                                   (2048, 33, True, True)])
+def test_hc_rows_token_tiles(lib, H, T, with_inject, alias):
+    """More than four rows run as 16-token MFMA tiles: row counts at the tile's edges, with
+    and without the inject matrix, and (alias) with inj_prev and inj one
+    buffer, as the engine chains the mixers. Each stage within STAGE of the
+    fp64 oracle on its own inputs (fp32 sums of at most 4H / 32 = 320 exact
+    block dots: 320 * 2^-24 = 1.9e-5 of the sum's magnitude)."""
+    _say("hc rows: H", H, "T", T, "inject", with_inject, "alias", alias)
+    qfm.init(H, H // 4, 512, 10, 1, 1)
+    rng = np.random.default_rng(H + 100 * T)
+    RS, L = 4 * H, 320
+    mats = (_Mat(rng, L, RS, 0.004), _Mat(rng, 4, RS, 0.004), _Mat(rng, RS, L, 0.02))
+    wn = (rng.uniform(-0.2, 0.2, RS).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    R0 = rng.standard_normal((T, RS)).astype(np.float32)
+    yp = rng.standard_normal((T, H)).astype(np.float32)
+    ip = rng.uniform(0, 2, (T, 4)).astype(np.float32)
+    bufs = _hc_bufs(T, H)
+    dR, dwn, dyp = qfm.DevBuf.from_array(R0), qfm.DevBuf.from_array(wn), qfm.DevBuf.from_array(yp)
+    dip = bufs["inj"] if alias else qfm.DevBuf.from_array(ip)
+    if alias:
+        dip.upload(ip)
+    st = qfm.Stream()
+    _hc_call(lib, bufs, dR, dwn, mats, dyp, dip, with_inject, T, st)
+    st.sync()
+    g = _hc_typed(bufs, T)
+    # (not asserted: the end-to-end figure. A last-bit difference ahead of an X8
+    # rounding moves a code by one, i.e. hc_d by absmax / 127, and an up row by
+    # up to 127 * 0.03 times that; how often it happens grows with the rows)
+    _check_mixer(g, dR.download(np.float32, (T, RS)), R0, wn, mats, yp, ip, True, with_inject, H)
+    bits = g["mixed"].view(np.uint32)
+    assert np.array_equal(g["xb"], ((bits + 0x7FFF + ((bits >> 16) & 1)) >> 16).astype(np.uint16))
+    st.destroy()
+    qfm.init(2560, 640, 512, 10, 1, 1)
