@@ -323,10 +323,11 @@ typedef struct {
  * across calls (the same offsets for every M, so one workspace of the largest
  * size serves calls of any M); calls that share a workspace must not overlap. */
 size_t qfm_workspace_bytes(int M);
-/* For M > 8 (prefill) logits is [M][E] of the MFMA router GEMM (the exact
- * canonical logits are computed only for the selection candidates), hidden is
- * NULL and counters points at {tokens whose candidate set overflowed and had
- * every logit recomputed, gate/up work items, down work items} (int, device
+/* For M > 8 logits is [M][E]: the exact canonical logits up to 1536 rows, the
+ * MFMA router GEMM's beyond (where the exact ones are computed only for the
+ * selection candidates); hidden is NULL and counters points at {tokens whose
+ * candidate set overflowed (more than 64 candidates for the top K), work items
+ * of the gate/up GEMM, of the down GEMM (0: the same ones)} (int, device
  * memory; NULL for M <= 8). */
 typedef struct {
     float *logits;   /* [M][E+1]: router logits; column E = <sh_gate_inp, x> */

@@ -114,6 +114,42 @@ void noalloc_prepare_current_device();
 // Resolve the one-launch pre-mixer's hand-off area for the current device (qfm_init).
 void hc_prepare_current_device();
 
+// Weights of one projection over the expert groups (prefill and middle paths).
+struct GroupW {
+    const int8_t *w;      // routed arena blob: INT8 [E][rows][K], or NVFP4 packed e2m1 [E][rows][K/2]
+    const float *s;       // INT8 routed row scales [E][rows]
+    const int8_t *w_sh;   // shared expert [rows][K] (INT8 in both formats)
+    const float *s_sh;    // shared row scales [rows]
+    const uint8_t *sc4;   // NVFP4 e4m3 block scales [E][rows][K/16]
+    const float *s2;      // NVFP4 per-expert global scales [E]
+};
+
+// The middle path (8 < T <= kMidRowsMax, qfm_mid.hip): router, selection, plan
+// and the two grouped GEMMs, up to the fp16 partials that k_pf_combine_h sums.
+constexpr int kMidRowsMax = 1536;
+struct MidArgs {
+    const float *router, *bias, *g;     // g: shared-expert gate vector or nullptr
+    const uint16_t *x;
+    int T, has_sh;
+    bool f4;
+    float *logits;                      // [T][E]
+    int *sel;
+    float *wts, *gam;
+    uint4 *x16;                         // x as fp16 scaled by 2^k per token, 2^-k in x16isc
+    float *x16isc;
+    int *ctr;                           // {selection overflows, items, ...}
+    int *p_tok, *p_slot;
+    float *p_wt;
+    int4 *items;
+    int max_items;                      // entries of items
+    uint16_t *hid;                      // [pairs][I] fp16
+    int8_t *hk;                         // [pairs][I / 64]
+    uint16_t *part;                     // [T (K + shared)][H] fp16
+    int8_t *partk;                      // [T (K + shared)][H / 64]
+    GroupW gg, gu, gd;
+};
+int launch_mid(const MidArgs &a, hipStream_t s);
+
 // Prefill (T > 8 rows): MFMA router + exact candidate selection, grouped
 // MFMA gate/up and down over the routing inversion, owned-partial combine.
 size_t prefill_ws_bytes(int T);

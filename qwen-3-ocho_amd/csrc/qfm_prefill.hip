@@ -814,15 +814,6 @@ k_pf_scatter(const int *__restrict__ sel, const float *__restrict__ wts, const f
 }
 
 // ---- grouped expert GEMMs -------------------------------------------------------------
-struct GroupW {
-    const int8_t *w;      // routed arena blob: INT8 [E][rows][K], or NVFP4 packed e2m1 [E][rows][K/2]
-    const float *s;       // INT8 routed row scales [E][rows]
-    const int8_t *w_sh;   // shared expert [rows][K] (INT8 in both formats)
-    const float *s_sh;    // shared row scales [rows]
-    const uint8_t *sc4;   // NVFP4 e4m3 block scales [E][rows][K/16]
-    const float *s2;      // NVFP4 per-expert global scales [E]
-};
-
 // MODE kAllI8: every tile INT8. kRoutedF4: routed tiles (grp < E) of an
 // NVFP4 arena (block scales staged into the bf16 B tile, the global scale s2
 // applied in the epilogue) and the shared expert's tiles, INT8 in both formats.
@@ -1177,6 +1168,27 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
     float *x16isc = static_cast<float *>(at(kPfX16isc));
 
     const float *g = (has_sh && gated) ? L->sh_gate_inp : nullptr;
+    GroupW gg, gu, gd;
+    if (f4) {
+        gg = GroupW{reinterpret_cast<const int8_t *>(a->w_gate), nullptr, L->sh_gate.w, L->sh_gate.s, a->s_gate, a->s2g_dev};
+        gu = GroupW{reinterpret_cast<const int8_t *>(a->w_up), nullptr, L->sh_up.w, L->sh_up.s, a->s_up, a->s2u_dev};
+        gd = GroupW{reinterpret_cast<const int8_t *>(a->w_down), nullptr, L->sh_down.w, L->sh_down.s, a->s_down, a->s2d_dev};
+    } else {
+        gg = GroupW{a->i8_gate, a->i8s_gate, L->sh_gate.w, L->sh_gate.s, nullptr, nullptr};
+        gu = GroupW{a->i8_up, a->i8s_up, L->sh_up.w, L->sh_up.s, nullptr, nullptr};
+        gd = GroupW{a->i8_down, a->i8s_down, L->sh_down.w, L->sh_down.s, nullptr, nullptr};
+    }
+    if (T <= kMidRowsMax) {
+        // the middle path uses the same regions (hid as scaled fp16, its
+        // exponents in the hsum region, one item list)
+        const MidArgs m{L->router, L->router_bias, g, x, T, has_sh ? 1 : 0, f4, lg, sel, wts, gam, x16, x16isc, ctr,
+                        p_tok, p_slot, p_wt, items_gu, (int)(Lw.bytes[kPfItemsGu] / sizeof(int4)), hid,
+                        reinterpret_cast<int8_t *>(hsum), part, partk, gg, gu, gd};
+        if (const int rc = launch_mid(m, s)) return rc;
+        hipLaunchKernelGGL(k_pf_combine_h, dim3((unsigned)(((size_t)T * H / 4 + 255) / 256)), dim3(256), 0, s, part,
+                           partk, T, S, H, y, y32);
+        return check_launch("prefill");
+    }
     // zero the small counters with a fill kernel (no memset node in captured graphs)
     launch_fill_f32(reinterpret_cast<float *>(ctr), 8, 0.0f, s);
     hipLaunchKernelGGL(k_pf_router_prep, dim3((unsigned)(E + (T + 3) / 4)), dim3(256), 0, s, L->router, E, H, wnorm,
@@ -1194,16 +1206,6 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
                        items_gu, items_dn, ctr + 1, (int)(max_mt * nt_gu), (int)(max_mt * nt_dn));
     hipLaunchKernelGGL(k_pf_scatter, dim3((unsigned)(nblk + (has_sh ? (T + 255) / 256 : 0))), dim3(256), 0, s, sel,
                        wts, g ? gam : nullptr, T, K, E, has_sh ? 1 : 0, off, blk, p_tok, p_slot, p_wt);
-    GroupW gg, gu, gd;
-    if (f4) {
-        gg = GroupW{reinterpret_cast<const int8_t *>(a->w_gate), nullptr, L->sh_gate.w, L->sh_gate.s, a->s_gate, a->s2g_dev};
-        gu = GroupW{reinterpret_cast<const int8_t *>(a->w_up), nullptr, L->sh_up.w, L->sh_up.s, a->s_up, a->s2u_dev};
-        gd = GroupW{reinterpret_cast<const int8_t *>(a->w_down), nullptr, L->sh_down.w, L->sh_down.s, a->s_down, a->s2d_dev};
-    } else {
-        gg = GroupW{a->i8_gate, a->i8s_gate, L->sh_gate.w, L->sh_gate.s, nullptr, nullptr};
-        gu = GroupW{a->i8_up, a->i8s_up, L->sh_up.w, L->sh_up.s, nullptr, nullptr};
-        gd = GroupW{a->i8_down, a->i8s_down, L->sh_down.w, L->sh_down.s, nullptr, nullptr};
-    }
     const dim3 g_gu((unsigned)(max_mt * nt_gu)), g_dn((unsigned)(max_mt * nt_dn)),
         nth(f4 ? ExpertEngineF4::NT : ExpertEngine::NT), nth_dn(f4 ? ExpertEngineF4::NT : DownEngineI8::NT);
     if (f4) {

@@ -155,6 +155,67 @@ def test_prefill_tile_boundaries(lib, T, fmt):
     st.destroy()
 
 
+# ------------------------------------------------------------------ middle row counts
+@pytest.mark.parametrize("hidden,inter,T,fmt,hot", [
+    (2048, 512, 9, 1, 0), (2048, 512, 16, 0, 16), (2048, 512, 33, 1, 17), (2560, 640, 31, 0, 33), (2560, 640, 17, 1, 1),
+    (2560, 640, 65, 1, 65), (2560, 640, 1300, 0, 65)])
+def test_middle_rows(lib, hidden, inter, T, fmt, hot):
+    """9 to 1536 rows run as weight-streaming items of 16 (INT8 from 24 rows an
+    expert: 64) rows per expert; 1537 rows are the first of the prefill tiles.
+    `hot` rows are copies of row 0, so that its ten experts get at least that
+    many rows: counts at and around whole items, beside experts with one row and
+    with none. Routing bit-exact, the exact logits in the workspace view, and y
+    within TOL of the grouped fp64 oracle (16-bit hidden values and partials)."""
+    _say("middle rows H", hidden, "T", T, "fmt", fmt, "hot", hot)
+    qfm.init(hidden, inter, E, K, 1, 1)
+    st = qfm.Stream()
+    seed, layer, xl = 6, 3, 60
+    L = qfm.SynthLayer(fmt, seed, layer, stream=st)
+    x = orc.fill("gauss_bf16", seed, xl, orc.T_X, 0, T * hidden).reshape(T, hidden)
+    x[:hot] = x[0]
+    dx, dy = qfm.DevBuf.from_array(x), qfm.DevBuf(T * hidden * 2)
+    wsb = lib.qfm_workspace_bytes(T)
+    ws = qfm.DevBuf(wsb)
+    for _ in range(2):                                   # the second call on a used workspace
+        qfm.check(lib.qfm_moe_forward(C.byref(L.s.layer), dx.ptr, T, dy.ptr, ws.ptr, wsb, st.h), "forward")
+    st.sync()
+    view = qfm.QfmWsView()
+    lib.qfm_workspace_view(ws.ptr, T, C.byref(view))
+    y = orc.bf16_to_f32(dy.download(np.uint16, (T, hidden)))
+    r = orc.moe_layer_grouped(hidden, inter, E, K, T, seed, layer, xl, x=x, fmt=fmt)
+    assert np.array_equal(qfm.d2h(view.sel, np.int32, (T, K)), r["sel"])
+    assert np.allclose(qfm.d2h(view.wts, np.float32, (T, K)), r["w"], rtol=2e-6, atol=1e-7)
+    W = orc.fill("gauss", seed, layer, orc.T_ROUTER, 0, E * hidden, scale=0.02).reshape(E, hidden)
+    rows = [0, T // 2, T - 1]
+    lg = qfm.d2h(view.logits, np.float32, (T, E))
+    assert np.array_equal(lg[rows].view(np.uint32), orc.router_logits(W, x[rows]).view(np.uint32))
+    rel = max(_rel(y[t], r["y"][t]) for t in range(T))
+    _say("  max rel err", rel)
+    assert rel <= TOL
+    L.destroy()
+    st.destroy()
+    qfm.init(H, I, E, K, 1, 1)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_middle_rows_upper_edge(lib, fmt):
+    """The largest middle call and the smallest prefill call on the same rows:
+    the same routing, and y rows that differ by the two paths' 16-bit roundings
+    only (hidden values 2^-9 against 2^-12, partials and y alike: well below
+    TOL of the largest value)."""
+    _say("middle rows, upper edge, fmt", fmt)
+    qfm.init(H, I, E, K, 1, 1)
+    st = qfm.Stream()
+    T = 1536
+    L = qfm.SynthLayer(fmt, 8, 2, stream=st)
+    x = orc.fill("gauss_bf16", 8, 61, orc.T_X, 0, (T + 1) * H).reshape(T + 1, H)
+    a, b = _forward(lib, L.s.layer, x[:T], st), _forward(lib, L.s.layer, x, st)
+    assert np.array_equal(a["sel"], b["sel"][:T]) and np.allclose(a["wts"], b["wts"][:T], rtol=2e-6, atol=1e-7)
+    assert max(_rel(a["y"][t], b["y"][t]) for t in range(T)) <= TOL
+    L.destroy()
+    st.destroy()
+
+
 # ------------------------------------------------------------------ fork rows sharing experts
 @pytest.mark.parametrize("M,fmt,boost", [(2, 0, 64.0), (8, 0, 64.0), (8, 1, 64.0), (8, 0, 1.5), (5, 1, 1.5)])
 def test_fork_rows_sharing_experts(lib, M, fmt, boost):
