@@ -18,6 +18,7 @@
 // failure); the void form calls it and leaves the code in the error latch.
 #include "qfm_dev.h"
 #include "qfm_internal.h"
+#include "qfm_mfma.h"
 
 namespace qfm {
 
@@ -166,94 +167,226 @@ __device__ __forceinline__ void ld_f32x16(const float *p, float *v) {
 }
 
 // ---- chunk tier gate/up: INT8 arena x X8 token rows (qf8_moe_i8.hip:196-262).
-// grid (I / RPB, n_exp_max); each lane group keeps its gate and up row in
-// registers and dots them with TX tokens at a time.
+// grid (I / 64, n_exp_max); wave w the 16 gate and 16 up rows from 64 b + 16 w,
+// the expert's pairs 16 at a time as MFMA columns: v_mfma_i32_16x16x32_i8 over
+// one 32-value X8 block (exact), scaled by the token's block scale into fp32.
+// Weights stream 16 bytes a lane, two 256-value chunks in flight, and become
+// fragments through wave-private LDS (as the middle path's gate/up); an
+// expert's further pairs read them again, from L2. Bound by the weight stream;
+// the form before it (a lane group per row, four tokens a pass) lost the
+// stream's rate to its dots from ~2 rows an expert on (2560/640, 64 / 128 / 256 /
+// 1024 rows, whole call with the down launch below: 514 / 846 / 1410 / 4704 us
+// against 317 / 420 / 503 / 1286).
+struct ChunkGuLds {
+    uint8_t w[4][32 * 256];                       // per wave: 16 gate and 16 up rows of one chunk
+    uint8_t x[2][16 * 256];                       // 16 tokens' codes, two chunks
+    float s[2][16][9];                            // and their block scales
+};
 template <int H, int I>
 __global__ void __launch_bounds__(256)
 k_cx_gateup_i8x8(const int8_t *__restrict__ Wg, const float *__restrict__ Sg, const int8_t *__restrict__ Wu,
                  const float *__restrict__ Su, const int8_t *__restrict__ xq, const float *__restrict__ xs,
                  float *__restrict__ hidden, const int *__restrict__ exp_slot, const int *__restrict__ exp_ptr,
                  const int *__restrict__ pair_tok, const int *__restrict__ n_exp_dev) {
-    constexpr int CPR = H / 16, LPR = lpr_of(CPR), NST = CPR / LPR, RPB = 256 / LPR, TX = 4;
+    constexpr int KC = 256, NCH = H / KC, NB = KC / 32;
+    static_assert(NCH % 2 == 0, "whole rounds of chunks");
+    __shared__ __align__(16) ChunkGuLds L;
+    typedef int i32x4_t __attribute__((ext_vector_type(4)));
+    typedef u32x4_t u32x4_u __attribute__((aligned(1)));      // (X8 rows need no more than their element's alignment)
+    typedef f32x4_t f32x4_u __attribute__((aligned(4)));
     const int e = blockIdx.y;
     if (e >= *n_exp_dev) return;
-    const int l = threadIdx.x % LPR, row = blockIdx.x * RPB + threadIdx.x / LPR;
     const int slot = exp_slot[e], base = exp_ptr[e], n = exp_ptr[e + 1] - base;
-    const size_t woff = ((size_t)slot * I + row) * H;
-    uint4 wg[NST], wu[NST];
+    for (int j0 = 0; j0 < n; j0 += 16) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));             // (LDS addresses hoisted out of this loop take 80 VGPRs)
+        const int lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+        const int rows = min(16, n - j0);
+        const size_t row = (size_t)slot * I + blockIdx.x * 64 + wave * 16;
+        const uint8_t *gp = reinterpret_cast<const uint8_t *>(Wg) + (row + g) * H + l16 * 16;
+        const uint8_t *up = reinterpret_cast<const uint8_t *>(Wu) + (row + g) * H + l16 * 16;
+        u32x4_t buf[2][8], xr;
+        f32x4_t sr;
+        auto wload = [&](int c, int b) __attribute__((always_inline)) {
 #pragma unroll
-    for (int st = 0; st < NST; st++) {
-        wg[st] = ld_nt16(Wg + woff + (st * LPR + l) * 16);
-        wu[st] = ld_nt16(Wu + woff + (st * LPR + l) * 16);
-    }
-    const float sg = Sg[(size_t)slot * I + row], su = Su[(size_t)slot * I + row];
-    for (int j0 = 0; j0 < n; j0 += TX) {
-        int tk[TX];
-#pragma unroll
-        for (int j = 0; j < TX; j++) tk[j] = pair_tok[base + (j0 + j < n ? j0 + j : j0)];
-        uint4 xv[TX][NST];
-        float sc[TX][NST];
-#pragma unroll
-        for (int j = 0; j < TX; j++)
-#pragma unroll
-            for (int st = 0; st < NST; st++) {
-                const int c = st * LPR + l;
-                xv[j][st] = *reinterpret_cast<const uint4 *>(xq + (size_t)tk[j] * H + c * 16);
-                sc[j][st] = xs[(size_t)tk[j] * (H / 32) + (c >> 1)];
+            for (int j = 0; j < 4; j++) {
+                buf[b][j] = ld_w<1>(gp + (size_t)j * 4 * H + c * KC);
+                buf[b][4 + j] = ld_w<1>(up + (size_t)j * 4 * H + c * KC);
             }
+        };
+        const int xt = tid >> 4, st = (tid & 31) >> 1;
+        const int8_t *xp = xq + (size_t)(xt < rows ? pair_tok[base + j0 + xt] : 0) * H + (tid & 15) * 16;
+        const bool sl = tid < 32 && st < rows;
+        const float *sp = xs + (size_t)(sl ? pair_tok[base + j0 + st] : 0) * (H / 32) + (tid & 1) * 4;
+        auto xload = [&](int c) __attribute__((always_inline)) {
+            if (xt < rows) xr = *reinterpret_cast<const u32x4_u *>(xp + c * KC);
+            if (sl) sr = *reinterpret_cast<const f32x4_u *>(sp + c * NB);
+        };
+        wload(0, 0);
+        xload(0);
+        wload(1, 1);
+        if (j0 > 0) __syncthreads();              // the previous pairs' last chunk is consumed
+        f32x4_t ag = {0.f, 0.f, 0.f, 0.f}, au = ag;
+        uint8_t *lw = L.w[wave];
+        auto step = [&](int c, int b) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < TX; j++) {
-            float ag = 0.0f, au = 0.0f;
-#pragma unroll
-            for (int st = 0; st < NST; st++) {
-                ag = fmaf((float)dot16_i8i8(wg[st], xv[j][st]), sc[j][st], ag);
-                au = fmaf((float)dot16_i8i8(wu[st], xv[j][st]), sc[j][st], au);
+            for (int j = 0; j < 4; j++) {
+                *reinterpret_cast<u32x4_t *>(lw + lds_at<KC>(j * 4 + g, l16)) = buf[b][j];
+                *reinterpret_cast<u32x4_t *>(lw + 16 * KC + lds_at<KC>(j * 4 + g, l16)) = buf[b][4 + j];
             }
-            ag = group_sum<LPR>(ag);
-            au = group_sum<LPR>(au);
-            if (l == 0 && j0 + j < n) hidden[(size_t)(base + j0 + j) * I + row] = silu(ag * sg) * (au * su);
+            if (xt < rows) *reinterpret_cast<u32x4_t *>(L.x[b] + lds_at<KC>(xt, tid & 15)) = xr;
+            if (sl)
+#pragma unroll
+                for (int i = 0; i < 4; i++) L.s[b][st][(tid & 1) * 4 + i] = sr[i];
+            if (c + 2 < NCH) wload(c + 2, b);
+            if (c + 1 < NCH) xload(c + 1);
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < NB; q++) {
+                const int f = lds_at<KC>(l16, 2 * q + (g >> 1)) + (g & 1) * 8;
+                const long xv = *reinterpret_cast<const long *>(L.x[b] + f);
+                const float s = L.s[b][l16][q];
+                const i32x4_t z = {0, 0, 0, 0};
+                const i32x4_t dg = __builtin_amdgcn_mfma_i32_16x16x32_i8(*reinterpret_cast<const long *>(lw + f), xv, z, 0, 0, 0);
+                const i32x4_t du = __builtin_amdgcn_mfma_i32_16x16x32_i8(*reinterpret_cast<const long *>(lw + 16 * KC + f), xv, z, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    ag[i] = fmaf((float)dg[i], s, ag[i]);
+                    au[i] = fmaf((float)du[i], s, au[i]);
+                }
+            }
+            wave_lds_fence();
+        };
+#pragma unroll 1
+        for (int c = 0; c < NCH; c += 2) {
+            step(c, 0);
+            step(c + 1, 1);
+        }
+        if (l16 < rows) {                         // D: pair l16, rows 4 g + i
+            const f32x4_t sg = *reinterpret_cast<const f32x4_u *>(Sg + row + 4 * g);
+            const f32x4_t su = *reinterpret_cast<const f32x4_u *>(Su + row + 4 * g);
+            f32x4_t h;
+#pragma unroll
+            for (int i = 0; i < 4; i++) h[i] = silu(ag[i] * sg[i]) * (au[i] * su[i]);
+            *reinterpret_cast<f32x4_u *>(hidden + (size_t)(base + j0 + l16) * I + blockIdx.x * 64 + wave * 16 + 4 * g) = h;
         }
     }
 }
 
 // ---- chunk tier down: owned partials part[(tok*K + k)][H] = wt * sd * <Wd, h>
 // with k the position of the expert in the token's selection
-// (qf8_moe_i8.hip:263-311). grid (H / RPB, n_exp_max).
-template <int H, int I>
-__global__ void __launch_bounds__(256)
+// (qf8_moe_i8.hip:263-311). grid (H / CW, n_exp_max), CW columns a block.
+// MFMA tiles of 16 weight rows by 16 columns (mid_dn_body), a pair's fp32 hidden row as three
+// of the columns: the value times 2^k (k per 64 values) split into three fp16
+// pieces of 11 bits, which leaves nothing of the 24 out (2^-39 of the group's
+// largest value at most), so the dots are the fp32 ones; the three sums are
+// added per row. Five pairs a token tile; an expert's further pairs read its
+// weights again (from L2). Bound by the weight stream; the form before it (a
+// lane group per weight row, each reading the pairs' rows from L2) waited for
+// those reads: 16 / 64 / 256 rows at 2048/512 132 / 344 / 625 us against 32 / 70
+// / 133, at 2560/640, 64 rows 313 against 110 (5.5 TB/s).
+template <int I, int NT>
+struct ChunkHidStage {
+    static constexpr int NTH = 64 * mid_dn_waves(I, NT), NP = 5 * NT, F4R = I / 4;   // float4s per row
+    static constexpr int NX = (NP * F4R + NTH - 1) / NTH;
+    static_assert(F4R % 16 == 0, "a group of 64 values is one 16-lane row");
+    const float *h;                                // the pairs' hidden rows (contiguous)
+    int n, tid;                                    // pairs, thread
+    f32x4_t v[NX];
+    __device__ __forceinline__ void load() {
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int c = j * NTH + tid;
+            v[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            if (c < n * F4R) v[j] = reinterpret_cast<const f32x4_t *>(h)[c];
+        }
+    }
+    __device__ __forceinline__ void store(MidDnLds<I, NT> &L) {
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int c = j * NTH + tid, t = c / F4R, f = c - t * F4R;
+            const float m = row16_max(fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
+            const int k = f16_exp(m);
+            if (c >= n * F4R) continue;
+            uint16_t o[3][4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float r = __builtin_ldexpf(v[j][i], k);
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+                    const _Float16 q = (_Float16)r;
+                    o[p][i] = __builtin_bit_cast(uint16_t, q);
+                    // (inf and NaN stay in the first piece alone)
+                    r = (__float_as_uint(r) & 0x7F800000u) == 0x7F800000u ? 0.0f : r - (float)q;
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                const int r = 3 * t + t / 5 + p;   // five pairs in columns 0..14 of a tile
+                *reinterpret_cast<u32x2_t *>(L.h + lds_at<I * 2>(r, f >> 1) + (f & 1) * 8) =
+                    u32x2_t{(uint32_t)o[p][0] | ((uint32_t)o[p][1] << 16), (uint32_t)o[p][2] | ((uint32_t)o[p][3] << 16)};
+                if ((f & 15) == 0) L.isc[r][f >> 4] = exp2i(-k);
+            }
+        }
+    }
+};
+template <int H, int I, int NT>
+__global__ void __launch_bounds__(64 * mid_dn_waves(I, NT))
 k_cx_down_part_i8(const int8_t *__restrict__ Wd, const float *__restrict__ Sd, const float *__restrict__ hidden,
                   const float *__restrict__ pair_wt, const int *__restrict__ pair_tok,
                   const int *__restrict__ exp_slot, const int *__restrict__ exp_ptr,
                   const int *__restrict__ n_exp_dev, const int *__restrict__ sel, int K, float *__restrict__ part) {
-    constexpr int CPR = I / 16, LPR = lpr_of(CPR), NST = CPR / LPR, RPB = 256 / LPR, TX = NST == 1 ? 4 : 1;
+    constexpr int CW = 64 * mid_dn_waves(I, NT), NP = 5 * NT;
+    static_assert(H % CW == 0, "whole blocks of columns");
+    __shared__ __align__(16) MidDnLds<I, NT> L;
+    __shared__ int s_k[NP];
+    typedef f32x4_t f32x4_u __attribute__((aligned(4)));
     const int e = blockIdx.y;
     if (e >= *n_exp_dev) return;
-    const int l = threadIdx.x % LPR, row = blockIdx.x * RPB + threadIdx.x / LPR;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const int slot = exp_slot[e], base = exp_ptr[e], n = exp_ptr[e + 1] - base;
-    uint4 w[NST];
+    const int c0 = blockIdx.x * CW + wave * 64;
+    const uint8_t *w = reinterpret_cast<const uint8_t *>(Wd) + ((size_t)slot * H + c0) * I;
+    f32x4_t sd[4];
 #pragma unroll
-    for (int st = 0; st < NST; st++) w[st] = ld_nt16(Wd + ((size_t)slot * H + row) * I + (st * LPR + l) * 16);
-    const float sd = Sd[(size_t)slot * H + row];
-    for (int j0 = 0; j0 < n; j0 += TX) {
-        float hv[TX][NST][16];
-#pragma unroll
-        for (int j = 0; j < TX; j++) {
-            const int pj = base + (j0 + j < n ? j0 + j : j0);
-#pragma unroll
-            for (int st = 0; st < NST; st++) ld_f32x16(hidden + (size_t)pj * I + (st * LPR + l) * 16, hv[j][st]);
+    for (int rt = 0; rt < 4; rt++)
+        sd[rt] = *reinterpret_cast<const f32x4_u *>(Sd + (size_t)slot * H + c0 + rt * 16 + 4 * g);
+    for (int j0 = 0; j0 < n; j0 += NP) {
+        const int np = min(NP, n - j0);
+        if (j0 > 0) __syncthreads();               // the previous pairs' rows are consumed
+        if (tid < np) {                            // the slot's place in the pair's selection (0 if it is not there)
+            const int tok = pair_tok[base + j0 + tid];
+            int k = 0;
+            for (int kk = K - 1; kk >= 0; kk--)
+                if (sel[(size_t)tok * K + kk] == slot) k = kk;
+            s_k[tid] = tok * K + k;
         }
+        // (an opaque copy: the body's LDS addresses hoisted out of this loop take 80 VGPRs)
+        int tl = tid;
+        asm volatile("" : "+v"(tl));
+        ChunkHidStage<I, NT> st{hidden + (size_t)(base + j0) * I, np, tl, {}};
+        f32x4_t acc[4][NT];
+        mid_dn_body<I, false, NT>(w, nullptr, NT == 1 ? 16 : 16 * ((np + 4) / 5), L, acc, st, tl);
 #pragma unroll
-        for (int j = 0; j < TX; j++) {
-            float acc = 0.0f;
+        for (int t4 = 0; t4 < NT; t4++) {
+            // columns 3 j, 3 j + 1, 3 j + 2 of the tile: pair 5 t4 + j (five pairs in
+            // 15 columns, so a tile's pieces never cross into the next tile)
+            const int j = t4 * 5 + l16 / 3;
+            const bool live = l16 % 3 == 0 && l16 < 15 && j < np;
+            const float pw = live ? pair_wt[base + j0 + j] : 0.0f;
+            float *dst = part + (size_t)(live ? s_k[j] : 0) * H + c0 + 4 * g;
 #pragma unroll
-            for (int st = 0; st < NST; st++) acc = dot16_i8f(w[st], hv[j][st], acc);
-            acc = group_sum<LPR>(acc);
-            if (l == 0 && j0 + j < n) {
-                const int pj = base + j0 + j, tok = pair_tok[pj];
-                int k = 0;
-                for (int kk = 0; kk < K; kk++)
-                    if (sel[(size_t)tok * K + kk] == slot) { k = kk; break; }
-                part[((size_t)tok * K + k) * H + row] = pair_wt[pj] * sd * acc;
+            for (int rt = 0; rt < 4; rt++) {
+                f32x4_t v;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float av = acc[rt][t4][i];   // (a bit cast of the element itself takes element 0)
+                    const int a = __builtin_bit_cast(int, av);
+                    const float m1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, a, 0x101, 0xF, 0xF, true));
+                    const float m2 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, a, 0x102, 0xF, 0xF, true));
+                    v[i] = pw * sd[rt][i] * ((av + m1) + m2);
+                }
+                if (live) *reinterpret_cast<f32x4_u *>(dst + rt * 16) = v;
             }
         }
     }
@@ -632,15 +765,23 @@ int qf8_i8_experts_chunk_ex(const Qf4ExpCache *c, const int8_t *xq, const float 
         set_error(-1, "qf8_i8_experts_chunk: bad arguments"); return -1;
     }
     const int K = g_cfg.K;
+    // token tiles (5 pairs each) of the down launch: whole call, us, 2048/512 /
+    // 2560/640, one tile against two at 2.5 pairs an expert 265 / 420 : 289 / 441,
+    // at 5 332 / 528 : 325 / 503; one against four at 20 808 / 1334 : 639 / 1286
+    const long avg = (long)T * K / n_exp_max;
+    const int nt = avg < 4 ? 1 : avg < 10 ? 2 : 4;
+#define QFM_CX_DOWN(HH, II, NT)                                                                                     \
+    hipLaunchKernelGGL((k_cx_down_part_i8<HH, II, NT>), dim3(HH / (64 * mid_dn_waves(II, NT)), n_exp_max),          \
+                       dim3(64 * mid_dn_waves(II, NT)), 0, s, c->i8_down, c->i8s_down, hidden, pair_wt, pair_tok,   \
+                       exp_slot, exp_ptr, n_exp_dev, sel, K, part)
     QFM_SHAPE_DISPATCH({
-        hipLaunchKernelGGL((k_cx_gateup_i8x8<HH, II>), dim3(II / (256 / lpr_of(HH / 16)), n_exp_max), dim3(256), 0,
+        hipLaunchKernelGGL((k_cx_gateup_i8x8<HH, II>), dim3(II / 64, n_exp_max), dim3(256), 0,
                            s, c->i8_gate, c->i8s_gate, c->i8_up, c->i8s_up, xq, xs, hidden, exp_slot, exp_ptr,
                            pair_tok, n_exp_dev);
-        hipLaunchKernelGGL((k_cx_down_part_i8<HH, II>), dim3(HH / (256 / lpr_of(II / 16)), n_exp_max), dim3(256), 0,
-                           s, c->i8_down, c->i8s_down, hidden, pair_wt, pair_tok, exp_slot, exp_ptr, n_exp_dev, sel,
-                           K, part);
+        if (nt == 1) { QFM_CX_DOWN(HH, II, 1); } else if (nt == 2) { QFM_CX_DOWN(HH, II, 2); } else { QFM_CX_DOWN(HH, II, 4); }
         hipLaunchKernelGGL(k_cx_combine, dim3((HH + 255) / 256, T), dim3(256), 0, s, part, K, HH, y);
     });
+#undef QFM_CX_DOWN
     return check_launch("qf8_i8_experts_chunk");
 }
 

@@ -31,13 +31,9 @@
 // never reaches another one, and they are not stored.
 #include "qfm_dev.h"
 #include "qfm_internal.h"
+#include "qfm_mfma.h"
 
 namespace qfm {
-
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 // ---- router ---------------------------------------------------------------------
 // Blocks [0, ceil(T / 4)): a wave per token writes x as fp16 scaled by 2^k
@@ -229,85 +225,6 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
             p_slot[TK + t] = t * S + K;
             p_wt[TK + t] = gam ? gam[t] : 1.0f;
         }
-}
-
-// ---- fragments ----------------------------------------------------------------------
-// 16 int8 codes -> 16 fp16, exact: 1024 + u (u = q + 128) by v_perm, then - 1152
-__device__ __forceinline__ void i8_to_f16(u32x4_t w, f16x8_t &a, f16x8_t &b) {
-    const f16x2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    uint32_t o[8];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const uint32_t d = w[q] ^ 0x80808080u;
-        o[2 * q] = __builtin_bit_cast(uint32_t, as_h2(__builtin_amdgcn_perm(0x64646464u, d, 0x04010400u)) - off);
-        o[2 * q + 1] = __builtin_bit_cast(uint32_t, as_h2(__builtin_amdgcn_perm(0x64646464u, d, 0x04030402u)) - off);
-    }
-    a = __builtin_bit_cast(f16x8_t, u32x4_t{o[0], o[1], o[2], o[3]});
-    b = __builtin_bit_cast(f16x8_t, u32x4_t{o[4], o[5], o[6], o[7]});
-}
-// 8 e2m1 codes (one dword) times a block scale < 0x7F -> fp16, exact
-__device__ __forceinline__ f16x8_t f4_to_f16(uint32_t w, f16x2_t s) {
-    const u32x4_t o = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * s),
-                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1) * s),
-                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * s),
-                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * s)};
-    return __builtin_bit_cast(f16x8_t, o);
-}
-// the same with any scale byte (0x7F: +inf, >= 0x80: up to 2^24) as bf16, exact;
-// the activations follow as bf16 (they were bf16 rows times a power of two, or
-// are rounded to 8 bits: k_mid_down's hidden rows, as the prefill path holds them)
-__device__ __forceinline__ uint32_t pack_bf16_hi(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ __forceinline__ bf16x8_t f4_to_bf16x8(uint32_t w, float s) {
-    const f32x2_t a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1),
-                  c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
-    const u32x4_t o = {pack_bf16_hi(a.x * s, a.y * s), pack_bf16_hi(b.x * s, b.y * s), pack_bf16_hi(c.x * s, c.y * s),
-                       pack_bf16_hi(d.x * s, d.y * s)};
-    return __builtin_bit_cast(bf16x8_t, o);
-}
-__device__ __forceinline__ bf16x8_t f16_to_bf16x8(f16x8_t h) {
-    uint32_t o[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        o[i] = (uint32_t)f32_to_bf16((float)h[2 * i]) | ((uint32_t)f32_to_bf16((float)h[2 * i + 1]) << 16);
-    return __builtin_bit_cast(bf16x8_t, u32x4_t{o[0], o[1], o[2], o[3]});
-}
-__device__ __forceinline__ f32x4_t mfma_f16(f16x8_t a, f16x8_t b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4_t mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-// LDS rows of STRIDE bytes: 16-byte chunk c of row r at chunk position c ^
-// lds_rot(r), so that the 16 rows of a fragment read spread over the 64 banks
-template <int STRIDE>
-__device__ __forceinline__ int lds_rot(int r) {
-    static_assert(STRIDE % 256 == 0 || STRIDE % 256 == 128 || STRIDE % 256 == 64, "row strides in use");
-    return STRIDE % 256 == 0 ? r & 15 : STRIDE % 256 == 128 ? r & 7 : (r >> 2) & 3;
-}
-template <int STRIDE>
-__device__ __forceinline__ int lds_at(int r, int c) { return r * STRIDE + ((c ^ lds_rot<STRIDE>(r)) << 4); }
-// orders this wave's LDS accesses across its lanes (LDS serves one wave in order)
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-// 2^k scaling of a group whose largest magnitude is m into [2^14, 2^15)
-__device__ __forceinline__ int f16_exp(float m) {
-    return m == 0.0f ? 0 : min(113, max(-113, 141 - (int)(__float_as_uint(m) >> 23)));
-}
-__device__ __forceinline__ float exp2i(int k) { return __uint_as_float((uint32_t)(127 + k) << 23); }
-
-// 16 bytes of weights. With one token tile an item (nearly) every byte is read
-// once: nontemporal (INT8 gate/up + down at 37 / 300 rows 154 -> 136 / 288 ->
-// 262 us, 6.4 TB/s; at 700 rows no difference). With four the tiles of a large
-// expert read them again.
-template <int NT>
-__device__ __forceinline__ u32x4_t ld_w(const uint8_t *p) {
-    const u32x4_t *v = reinterpret_cast<const u32x4_t *>(p);
-    if constexpr (NT == 1) return __builtin_nontemporal_load(v);
-    else return *v;
 }
 
 // ---- gate/up ------------------------------------------------------------------------
@@ -514,110 +431,31 @@ k_mid_gateup(const int4 *__restrict__ items, const int *__restrict__ n_items, co
 }
 
 // ---- down ---------------------------------------------------------------------------
-constexpr int mid_dn_waves(int I, int nt) { return nt == 1 || I * nt > 2048 ? 4 : 8; }
+// The item's hidden rows (contiguous fp16 rows, exponents hk) into LDS.
 template <int I, int NT>
-struct MidDnLds {
-    uint8_t h[16 * NT * I * 2];                   // the item's hidden rows (whole K)
-    uint8_t w[mid_dn_waves(I, NT)][16 * I];          // per wave: one tile of 16 weight rows (NVFP4: codes, then scales)
-    float isc[16 * NT][I / 64 + 1];               // 2^-k of each row and 64 hidden values
+struct MidHidStage {
+    static constexpr int NTH = 64 * mid_dn_waves(I, NT), HS = I * 2, HC = HS / 16, NG = I / 64, NX = 16 * NT * HC / NTH;
+    static_assert(NX * NTH == 16 * NT * HC, "whole loads per thread");
+    const uint16_t *hid;
+    const int8_t *hk;
+    int rows;
+    u32x4_t hr[NX];
+    __device__ __forceinline__ void load() {
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int c = j * NTH + (int)threadIdx.x;
+            if (c < rows * HC) hr[j] = reinterpret_cast<const u32x4_t *>(hid)[c];
+        }
+    }
+    __device__ __forceinline__ void store(MidDnLds<I, NT> &L) {
+        for (int i = threadIdx.x; i < rows * NG; i += NTH) L.isc[i / NG][i % NG] = exp2i(-(int)hk[i]);
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int c = j * NTH + (int)threadIdx.x;
+            if (c < rows * HC) *reinterpret_cast<u32x4_t *>(L.h + lds_at<HS>(c / HC, c % HC)) = hr[j];
+        }
+    }
 };
-// One item, 64 output columns per wave: wave w the columns c0 .. c0 + 63 as four tiles
-// of 16 weight rows; acc[rt][n]: D[row 4 g + i][token l16].
-template <int H, int I, bool F4, int NT>
-__device__ __forceinline__ void mid_dn_body(const uint8_t *__restrict__ wd, const uint8_t *__restrict__ bd,
-                                            const uint16_t *__restrict__ hid, const int8_t *__restrict__ hk, int rows,
-                                            MidDnLds<I, NT> &L, f32x4_t (&acc)[4][NT]) {
-    constexpr int MT = 16 * NT, NG = I / 64, RT = 4;
-    constexpr int ROWB = F4 ? I / 2 : I, CPR = ROWB / 16, NL = 16 * CPR / 64;   // bytes, chunks per row, loads per tile
-    constexpr int SB = I / 16, SL = 16 * SB / 16;                                // NVFP4 scale bytes per row, 16-byte loads per tile
-    constexpr int D = F4 ? 4 : 2;                                                // tiles in flight
-    constexpr int NTH = 64 * mid_dn_waves(I, NT);                                   // threads
-    constexpr int HS = I * 2, HC = HS / 16, NX = MT * HC / NTH;
-    static_assert(NL * 64 == 16 * CPR && NX * NTH == MT * HC && SL <= 64, "whole loads per tile");
-    static_assert(!F4 || 16 * ROWB + 16 * SB <= 16 * I, "an NVFP4 tile and its scales fit the INT8 tile's LDS");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
-    u32x4_t buf[D][NL], sc[F4 ? D : 1], hr[NX];
-#pragma unroll
-    for (int j = 0; j < NX; j++) {                // the hidden rows are contiguous (and in L2): first
-        const int c = j * NTH + tid;
-        if (c < rows * HC) hr[j] = reinterpret_cast<const u32x4_t *>(hid)[c];
-    }
-    auto wload = [&](int rt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < NL; j++)
-            buf[rt % D][j] = ld_w<NT>(wd + (size_t)rt * 16 * ROWB + (j * 64 + lane) * 16);
-        if constexpr (F4)
-            if (lane < SL) sc[rt % D] = *reinterpret_cast<const u32x4_t *>(bd + (size_t)rt * 16 * SB + lane * 16);
-    };
-#pragma unroll
-    for (int rt = 0; rt < D; rt++) wload(rt);
-    for (int i = tid; i < rows * NG; i += NTH) L.isc[i / NG][i % NG] = exp2i(-(int)hk[i]);
-#pragma unroll
-    for (int j = 0; j < NX; j++) {
-        const int c = j * NTH + tid;
-        if (c < rows * HC) *reinterpret_cast<u32x4_t *>(L.h + lds_at<HS>(c / HC, c % HC)) = hr[j];
-    }
-    __syncthreads();
-    uint8_t *lw = L.w[wave];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
-#pragma unroll
-        for (int j = 0; j < NL; j++) {
-            const int c = j * 64 + lane;
-            *reinterpret_cast<u32x4_t *>(lw + lds_at<ROWB>(c / CPR, c % CPR)) = buf[rt % D][j];
-        }
-        if constexpr (F4)
-            if (lane < SL) *reinterpret_cast<u32x4_t *>(lw + 16 * ROWB + lane * 16) = sc[rt % D];
-        if (rt + D < RT) wload(rt + D);
-        wave_lds_fence();
-#pragma unroll
-        for (int n = 0; n < NT; n++) acc[rt][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (int kg = 0; kg < NG; kg++) {
-            // hidden values 64 kg + 16 g .. + 15 of token l16, weights of row l16
-            auto hfrag = [&](int n, int h) __attribute__((always_inline)) {
-                return *reinterpret_cast<const f16x8_t *>(L.h + lds_at<HS>(n * 16 + l16, 8 * kg + 2 * g + h));
-            };
-            auto add = [&](int n, f32x4_t d) __attribute__((always_inline)) {
-                const float s = L.isc[n * 16 + l16][kg];
-#pragma unroll
-                for (int i = 0; i < 4; i++) acc[rt][n][i] = fmaf(d[i], s, acc[rt][n][i]);
-            };
-            const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (!F4) {
-                f16x8_t w0, w1;
-                i8_to_f16(*reinterpret_cast<const u32x4_t *>(lw + lds_at<ROWB>(l16, 4 * kg + g)), w0, w1);
-#pragma unroll
-                for (int n = 0; n < NT; n++) {
-                    if (NT > 1 && n * 16 >= rows) continue;
-                    add(n, mfma_f16(w1, hfrag(n, 1), mfma_f16(w0, hfrag(n, 0), z)));
-                }
-            } else {
-                const u32x2_t w = *reinterpret_cast<const u32x2_t *>(lw + lds_at<ROWB>(l16, 2 * kg + (g >> 1)) + (g & 1) * 8);
-                const uint32_t b = lw[16 * ROWB + l16 * SB + 4 * kg + g];
-                if (__builtin_amdgcn_ballot_w64(b >= 0x7Fu) == 0) {
-                    const f32x2_t f = __builtin_amdgcn_cvt_pk_f32_fp8(b, false);
-                    const f16x2_t s = {(_Float16)f.x, (_Float16)f.x};
-                    const f16x8_t w0 = f4_to_f16(w[0], s), w1 = f4_to_f16(w[1], s);
-#pragma unroll
-                    for (int n = 0; n < NT; n++) {
-                        if (NT > 1 && n * 16 >= rows) continue;
-                        add(n, mfma_f16(w1, hfrag(n, 1), mfma_f16(w0, hfrag(n, 0), z)));
-                    }
-                } else {
-                    const float s = e4m3_scale(b);
-                    const bf16x8_t w0 = f4_to_bf16x8(w[0], s), w1 = f4_to_bf16x8(w[1], s);
-#pragma unroll
-                    for (int n = 0; n < NT; n++) {
-                        if (NT > 1 && n * 16 >= rows) continue;
-                        add(n, mfma_bf16(w1, f16_to_bf16x8(hfrag(n, 1)), mfma_bf16(w0, f16_to_bf16x8(hfrag(n, 0)), z)));
-                    }
-                }
-            }
-        }
-        wave_lds_fence();
-    }
-}
 
 template <int H, int I, bool F4, int NT>
 __global__ void __launch_bounds__(64 * mid_dn_waves(I, NT))
@@ -635,23 +473,22 @@ k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, cons
     const int grp = it.x, pb = it.y, rows = it.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const int c0 = cb * CW + wave * 64;
-    const uint16_t *hp = hid + (size_t)pb * I;
-    const int8_t *kp = hk + (size_t)pb * (I / 64);
+    MidHidStage<I, NT> st{hid + (size_t)pb * I, hk + (size_t)pb * (I / 64), rows, {}};
     f32x4_t acc[4][NT], sd[4];
     if (F4 && grp < E) {
         const size_t row = (size_t)grp * H + c0;
         const float a = gd.s2[grp];
 #pragma unroll
         for (int rt = 0; rt < 4; rt++) sd[rt] = f32x4_t{a, a, a, a};
-        mid_dn_body<H, I, true, NT>(reinterpret_cast<const uint8_t *>(gd.w) + row * (I / 2), gd.sc4 + row * (I / 16), hp,
-                                    kp, rows, L, acc);
+        mid_dn_body<I, true, NT>(reinterpret_cast<const uint8_t *>(gd.w) + row * (I / 2), gd.sc4 + row * (I / 16), rows,
+                                 L, acc, st, tid);
     } else {
         const size_t row = grp < E ? (size_t)grp * H + c0 : (size_t)c0;
 #pragma unroll
         for (int rt = 0; rt < 4; rt++)
             sd[rt] = *reinterpret_cast<const f32x4_t *>((grp < E ? gd.s : gd.s_sh) + row + rt * 16 + 4 * g);
-        mid_dn_body<H, I, false, NT>(reinterpret_cast<const uint8_t *>(grp < E ? gd.w : gd.w_sh) + row * I, nullptr, hp,
-                                     kp, rows, L, acc);
+        mid_dn_body<I, false, NT>(reinterpret_cast<const uint8_t *>(grp < E ? gd.w : gd.w_sh) + row * I, nullptr, rows,
+                                  L, acc, st, tid);
     }
     // the wave's 64 columns of each token as fp16 scaled by 2^k (k from the
     // largest finite magnitude; inf and NaN pass through), k to partk

@@ -157,6 +157,43 @@ def test_experts_chunk(lib, T):
     L.destroy()
 
 
+@pytest.mark.parametrize("T,n_exp_max", [(5, 50), (6, 60), (16, 160), (17, 170), (4, 10), (9, 10), (10, 10), (21, 10), (41, 10)])
+def test_experts_chunk_pair_tiles(lib, T, n_exp_max):
+    """Every token selects the same ten experts, so each has T pairs: counts at
+    and past the gate/up launch's 16 rows and the down launch's 5, 10 and 20 pairs
+    a pass (the pairs per expert bound choose between them). fp32 throughout:
+    integer block dots of 32 values exact, at most H / 32 + I / 64 + K = 82 fp32
+    roundings of 2^-24 along a sum, and SiLU by hardware exp and reciprocal
+    (2^-21): within 1e-5 of the largest value. Token 0 is 2^20 times smaller than
+    the others (each row keeps its own scale)."""
+    seed, layer = 2, 6
+    _say("experts chunk pair tiles", T, n_exp_max)
+    sel = np.tile(RNG.choice(E, K, replace=False).astype(np.int32), (T, 1))
+    for t in range(T):
+        RNG.shuffle(sel[t])
+    wt = (RNG.random((T, K)) + 0.1).astype(np.float32)
+    q, s, xhat = _x8_rows(T)
+    s[0] *= np.float32(2.0 ** -20)
+    xhat[0] = xhat[0] * 2.0 ** -20
+    L = qfm.SynthLayer(qfm.QFM_FMT_INT8, seed, layer)
+    P = T * K
+    dsel, dwt, dq, ds = _dev(sel), _dev(wt), _dev(q), _dev(s)
+    d_slot, d_ptr, d_tok, d_pw, d_cnt = (qfm.DevBuf(E * 4), qfm.DevBuf((E + 1) * 4), qfm.DevBuf(P * 4),
+                                         qfm.DevBuf(P * 4), qfm.DevBuf(8))
+    hid, part, y = qfm.DevBuf(P * I * 4), qfm.DevBuf(P * H * 4), qfm.DevBuf(T * H * 4)
+    qfm.check(lib.qf8_i8_csr_build_ex(dsel.ptr, dwt.ptr, T, d_slot.ptr, d_ptr.ptr, d_tok.ptr, d_pw.ptr, d_cnt.ptr, None))
+    qfm.check(lib.qf8_i8_experts_chunk_ex(C.byref(L.s.arena), dq.ptr, ds.ptr, hid.ptr, None, None, d_slot.ptr, d_ptr.ptr,
+                                          d_tok.ptr, d_pw.ptr, d_cnt.ptr, n_exp_max, P, dsel.ptr, part.ptr, T, y.ptr,
+                                          None))
+    _sync(lib)
+    got = y.download(np.float32, (T, H))
+    w = {int(e): _i8_expert_w(seed, layer, int(e)) for e in sel[0]}
+    for t in range(T):
+        ref = sum(float(wt[t, k]) * orc.i8_expert(xhat[t], *w[int(sel[t, k])])[1] for k in range(K))
+        assert _rel(got[t], ref) <= 1e-5, t
+    L.destroy()
+
+
 # ------------------------------------------------------------------ NVFP4 M=1
 def test_nvfp4_m1_entry_points(lib):
     seed, layer = 3, 5
