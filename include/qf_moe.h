@@ -323,7 +323,7 @@ typedef struct {
  * across calls (the same offsets for every M, so one workspace of the largest
  * size serves calls of any M); calls that share a workspace must not overlap. */
 size_t qfm_workspace_bytes(int M);
-/* For M > 8 logits is [M][E]: the exact canonical logits up to 1536 rows, the
+/* For M > 8 logits is [M][E]: the exact canonical logits up to 600 rows, the
  * MFMA router GEMM's beyond (where the exact ones are computed only for the
  * selection candidates); hidden is NULL and counters points at {tokens whose
  * candidate set overflowed (more than 64 candidates for the top K), work items

@@ -210,8 +210,8 @@ k_cx_gateup_i8x8(const int8_t *__restrict__ Wg, const float *__restrict__ Sg, co
         auto wload = [&](int c, int b) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                buf[b][j] = ld_w<1>(gp + (size_t)j * 4 * H + c * KC);
-                buf[b][4 + j] = ld_w<1>(up + (size_t)j * 4 * H + c * KC);
+                buf[b][j] = ld_w<true>(gp + (size_t)j * 4 * H + c * KC);
+                buf[b][4 + j] = ld_w<true>(up + (size_t)j * 4 * H + c * KC);
             }
         };
         const int xt = tid >> 4, st = (tid & 31) >> 1;
@@ -366,7 +366,7 @@ k_cx_down_part_i8(const int8_t *__restrict__ Wd, const float *__restrict__ Sd, c
         asm volatile("" : "+v"(tl));
         ChunkHidStage<I, NT> st{hidden + (size_t)(base + j0) * I, np, tl, {}};
         f32x4_t acc[4][NT];
-        mid_dn_body<I, false, NT>(w, nullptr, NT == 1 ? 16 : 16 * ((np + 4) / 5), L, acc, st, tl);
+        mid_dn_body<I, false, NT, NT == 1>(w, nullptr, NT == 1 ? 16 : 16 * ((np + 4) / 5), L, acc, st, tl);
 #pragma unroll
         for (int t4 = 0; t4 < NT; t4++) {
             // columns 3 j, 3 j + 1, 3 j + 2 of the tile: pair 5 t4 + j (five pairs in

@@ -124,9 +124,17 @@ struct GroupW {
     const float *s2;      // NVFP4 per-expert global scales [E]
 };
 
-// The middle path (8 < T <= kMidRowsMax, qfm_mid.hip): router, selection, plan
+// The middle path (8 < T <= mid_rows_max, qfm_mid.hip): router, selection, plan
 // and the two grouped GEMMs, up to the fp16 partials that k_pf_combine_h sums.
-constexpr int kMidRowsMax = 1536;
+// Where it ends against the prefill's 128-row tiles, us per layer, here / tiles:
+// 2048/512 INT8 1500 rows 507 / 620, 2560/640 INT8 1500 rows 841 / 932, NVFP4
+// 2048/512 458 / 686, 2560/640 723 / 991; it grows by 0.13, 0.30, 0.19 and 0.28
+// us a row, the tiles by 0.04 to 0.07.
+constexpr int mid_rows_max(int I, bool f4) { return I <= 512 ? 2800 : f4 ? 2500 : 1800; }
+// up to here the exact router of every expert (k_mid_router), beyond it
+// k_pf_select's candidates: 300 / 450 / 1021 rows 23 / 32 / 66 us, with the
+// selection 28 / 37 / 71, against 44 at 450 rows and 50 at 1021
+constexpr int kMidExactRows = 600;
 struct MidArgs {
     const float *router, *bias, *g;     // g: shared-expert gate vector or nullptr
     const uint16_t *x;
@@ -138,8 +146,7 @@ struct MidArgs {
     uint4 *x16;                         // x as fp16 scaled by 2^k per token, 2^-k in x16isc
     float *x16isc;
     int *ctr;                           // {selection overflows, items, ...}
-    int *p_tok, *p_slot;
-    float *p_wt;
+    int2 *pairs;                        // [T (K + shared)] {partial slot, weight}
     int4 *items;
     int max_items;                      // entries of items
     uint16_t *hid;                      // [pairs][I] fp16

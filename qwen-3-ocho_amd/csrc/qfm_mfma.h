@@ -79,14 +79,15 @@ __device__ __forceinline__ int f16_exp(float m) {
 }
 __device__ __forceinline__ float exp2i(int k) { return __uint_as_float((uint32_t)(127 + k) << 23); }
 
-// 16 bytes of weights. With one token tile an item (nearly) every byte is read
-// once: nontemporal (INT8 gate/up + down at 37 / 300 rows 154 -> 136 / 288 ->
-// 262 us, 6.4 TB/s; at 700 rows no difference). With four the tiles of a large
-// expert read them again.
-template <int NT>
+// 16 bytes of weights: nontemporal where (nearly) every byte is read ONCE (INT8
+// gate/up + down at 37 / 300 rows 154 -> 136 / 288 -> 262 us, 6.4 TB/s), plain
+// where an expert's further items read them again (1021 rows: 264 + 167 us
+// nontemporal, 244 + 144 plain; NVFP4 at 2560/640 395 + 255 against 304 + 240;
+// at 700 rows no difference).
+template <bool ONCE>
 __device__ __forceinline__ u32x4_t ld_w(const uint8_t *p) {
     const u32x4_t *v = reinterpret_cast<const u32x4_t *>(p);
-    if constexpr (NT == 1) return __builtin_nontemporal_load(v);
+    if constexpr (ONCE) return __builtin_nontemporal_load(v);
     else return *v;
 }
 
@@ -102,7 +103,7 @@ struct MidDnLds {
 // wave's first row and its block scales) against `rows` activation rows, which
 // stage.load() requests and stage.store(L) puts into L.h (fp16, lds_at rows)
 // and L.isc; acc[rt][n]: D[row 4 g + i][activation row l16].
-template <int I, bool F4, int NT, class STAGE>
+template <int I, bool F4, int NT, bool ONCE, class STAGE>
 __device__ __forceinline__ void mid_dn_body(const uint8_t *__restrict__ wd, const uint8_t *__restrict__ bd, int rows,
                                             MidDnLds<I, NT> &L, f32x4_t (&acc)[4][NT], STAGE &&stage, int tid) {
     constexpr int NG = I / 64, RT = 4, HS = I * 2;
@@ -117,7 +118,7 @@ __device__ __forceinline__ void mid_dn_body(const uint8_t *__restrict__ wd, cons
     auto wload = [&](int rt) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NL; j++)
-            buf[rt % D][j] = ld_w<NT>(wd + (size_t)rt * 16 * ROWB + (j * 64 + lane) * 16);
+            buf[rt % D][j] = ld_w<ONCE>(wd + (size_t)rt * 16 * ROWB + (j * 64 + lane) * 16);
         if constexpr (F4)
             if (lane < SL) sc[rt % D] = *reinterpret_cast<const u32x4_t *>(bd + (size_t)rt * 16 * SB + lane * 16);
     };

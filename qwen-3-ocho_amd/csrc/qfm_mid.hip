@@ -1,4 +1,4 @@
-// qfm_mid.hip -- the forward at a middle number of rows (8 < T <= kMidRowsMax):
+// qfm_mid.hip -- the forward at a middle number of rows (8 < T <= mid_rows_max):
 // weight-streaming grouped MFMA GEMMs.
 //
 // Reference behaviour: the chunk path (ocho/amd_server/qf8_moe_i8.hip:196-395)
@@ -180,19 +180,30 @@ k_mid_topk(const float *__restrict__ logits, int T, int K, int renorm, int *__re
 }
 
 // ---- plan -------------------------------------------------------------------------
+// A pair is {partial slot t (K + shared) + k, weight bits}: its token is slot / S.
 // One block of 1024 threads: pair counts per expert (LDS), offsets, the pairs
 // scattered into expert order (the order inside a group is unspecified, as in
 // k_pf_scatter), the shared expert's pairs (group E) in token order, and the
-// items: the shared group's first, then the experts' in ascending order.
+// items: the shared group's first, then the experts' in ascending order. The
+// selection is read in batches of 16 a thread, and a pair leaves as one 8-byte
+// store (scattered stores of three arrays and loads one at a time took 29 us at
+// 1021 rows).
+constexpr int kPlanBatch = 16;
 __global__ void __launch_bounds__(1024)
 k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const float *__restrict__ gam, int T, int K,
-           int E, int has_sh, int mt, int *__restrict__ p_tok, int *__restrict__ p_slot, float *__restrict__ p_wt,
-           int4 *__restrict__ items, int *__restrict__ n_items) {
+           int E, int has_sh, int mt, int2 *__restrict__ pairs, int4 *__restrict__ items, int *__restrict__ n_items) {
     __shared__ int cnt[1024], sa[1024], sb[1024];
     const int g = threadIdx.x, S = K + has_sh, TK = T * K;
     cnt[g] = 0;
     __syncthreads();
-    for (int p = g; p < TK; p += 1024) atomicAdd(&cnt[sel[p]], 1);
+    int v[kPlanBatch];
+    for (int p0 = g; p0 < TK; p0 += 1024 * kPlanBatch) {
+#pragma unroll
+        for (int i = 0; i < kPlanBatch; i++) v[i] = p0 + i * 1024 < TK ? sel[p0 + i * 1024] : -1;
+#pragma unroll
+        for (int i = 0; i < kPlanBatch; i++)
+            if (v[i] >= 0) atomicAdd(&cnt[v[i]], 1);
+    }
     __syncthreads();
     const int c = g < E ? cnt[g] : 0;
     const int mi = (c + mt - 1) / mt;
@@ -213,18 +224,33 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
     for (int i = g; i < shi; i += 1024) items[i] = make_int4(E, TK + i * mt, min(mt, T - i * mt), 0);
     if (g == E - 1) n_items[0] = shi + sb[g];
     __syncthreads();
-    for (int p = g; p < TK; p += 1024) {
-        const int t = p / K, pos = atomicAdd(&cnt[sel[p]], 1);
-        p_tok[pos] = t;
-        p_slot[pos] = t * S + p - t * K;
-        p_wt[pos] = wts[p];
+    const bool one = TK <= 1024 * kPlanBatch;                  // v still holds every id
+    for (int p0 = g; p0 < TK; p0 += 1024 * kPlanBatch) {
+        float w[kPlanBatch];
+#pragma unroll
+        for (int i = 0; i < kPlanBatch; i++) {
+            const int p = p0 + i * 1024;
+            w[i] = p < TK ? wts[p] : 0.0f;
+            if (!one) v[i] = p < TK ? sel[p] : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < kPlanBatch; i++)
+            if (v[i] >= 0) {
+                const int p = p0 + i * 1024, t = p / K;
+                pairs[atomicAdd(&cnt[v[i]], 1)] = make_int2(t * S + p - t * K, __float_as_int(w[i]));
+            }
     }
     if (has_sh)
-        for (int t = g; t < T; t += 1024) {
-            p_tok[TK + t] = t;
-            p_slot[TK + t] = t * S + K;
-            p_wt[TK + t] = gam ? gam[t] : 1.0f;
-        }
+        for (int t = g; t < T; t += 1024) pairs[TK + t] = make_int2(t * S + K, __float_as_int(gam ? gam[t] : 1.0f));
+}
+
+// Block b's unit of work of n: the blocks go to the 8 XCDs round-robin (b & 7),
+// and each XCD takes a contiguous range of units, so that the items of one
+// expert, which read the same weights, share an L2 (2560/640, 1021 rows, where
+// ten row blocks an item had spread them: figures at the launcher). -1: none.
+__device__ __forceinline__ int xcd_unit(int b, int n) {
+    const int c = (n + 7) >> 3, u = (b & 7) * c + (b >> 3);
+    return (b >> 3) < c && u < n ? u : -1;
 }
 
 // ---- gate/up ------------------------------------------------------------------------
@@ -237,10 +263,10 @@ struct MidGuLds {
 };
 // One item, 64 intermediate rows: wave w rows o0 = 64 rb + 16 w .. + 15 of gate
 // and up. ag / au: D[row 4 g + i][token l16] per token tile.
-template <int H, int I, bool F4, int NT>
+template <int H, int I, bool F4, int NT, bool ONCE>
 __device__ __forceinline__ void mid_gu_body(const uint8_t *__restrict__ wg, const uint8_t *__restrict__ wu,
                                             const uint8_t *__restrict__ bg, const uint8_t *__restrict__ bu,
-                                            const uint16_t *__restrict__ x16, const int *__restrict__ p_tok, int rows,
+                                            const uint16_t *__restrict__ x16, const int2 *__restrict__ pairs, int S, int rows,
                                             MidGuLds<NT> &L, f32x4_t (&ag)[NT], f32x4_t (&au)[NT]) {
     constexpr int KC = mid_kc(NT), NCH = H / KC, MT = 16 * NT;
     constexpr int ROWB = F4 ? H / 2 : H, CB = F4 ? KC / 2 : KC;        // bytes per row, per row and chunk
@@ -260,8 +286,8 @@ __device__ __forceinline__ void mid_gu_body(const uint8_t *__restrict__ wg, cons
     auto wload = [&](int c, int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NI; j++) {
-            buf[b][j] = ld_w<NT>(gp + (size_t)j * RPI * ROWB + c * CB);
-            buf[b][NI + j] = ld_w<NT>(up + (size_t)j * RPI * ROWB + c * CB);
+            buf[b][j] = ld_w<ONCE>(gp + (size_t)j * RPI * ROWB + c * CB);
+            buf[b][NI + j] = ld_w<ONCE>(up + (size_t)j * RPI * ROWB + c * CB);
         }
         if constexpr (F4)
             if (lane < 32) sc[b] = *reinterpret_cast<const scv_t *>(sp + c * SB);
@@ -270,7 +296,7 @@ __device__ __forceinline__ void mid_gu_body(const uint8_t *__restrict__ wg, cons
 #pragma unroll
     for (int j = 0; j < NX; j++) {
         const int t = tid / XC + XR * j;
-        xp[j] = x16 + (size_t)(t < rows ? p_tok[t] : 0) * H + (tid % XC) * 8;
+        xp[j] = x16 + (size_t)(t < rows ? pairs[t].x / S : 0) * H + (tid % XC) * 8;
     }
     auto xload = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
@@ -365,18 +391,17 @@ __device__ __forceinline__ void mid_gu_body(const uint8_t *__restrict__ wg, cons
     }
 }
 
-template <int H, int I, bool F4, int NT>
+template <int H, int I, bool F4, int NT, bool ONCE>
 __global__ void __launch_bounds__(256)
-k_mid_gateup(const int4 *__restrict__ items, const int *__restrict__ n_items, const int *__restrict__ p_tok,
+k_mid_gateup(const int4 *__restrict__ items, const int *__restrict__ n_items, const int2 *__restrict__ pairs, int S,
              const uint16_t *__restrict__ x16, const float *__restrict__ x16isc, GroupW g0, GroupW g1, int E,
              uint16_t *__restrict__ hid, int8_t *__restrict__ hk) {
     constexpr int NRB = I / 64;
     __shared__ __align__(16) MidGuLds<NT> L;
-    const int item = (int)blockIdx.x / NRB, rb = (int)blockIdx.x - item * NRB;
-    const int nit = n_items[0];
-    const int4 it = items[item];                  // (items holds at least gridDim / NRB entries)
-    args_now(nit, it.x, it.y, it.z);
-    if (item >= nit) return;
+    const int u = xcd_unit(blockIdx.x, n_items[0] * NRB);
+    if (u < 0) return;
+    const int item = u / NRB, rb = u - item * NRB;
+    const int4 it = items[item];
     const int grp = it.x, pb = it.y, rows = it.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const int o0 = rb * 64 + wave * 16;
@@ -387,16 +412,16 @@ k_mid_gateup(const int4 *__restrict__ items, const int *__restrict__ n_items, co
         const float a = g0.s2[grp], b = g1.s2[grp];
         sg = f32x4_t{a, a, a, a};
         su = f32x4_t{b, b, b, b};
-        mid_gu_body<H, I, true, NT>(reinterpret_cast<const uint8_t *>(g0.w) + row * (H / 2),
+        mid_gu_body<H, I, true, NT, ONCE>(reinterpret_cast<const uint8_t *>(g0.w) + row * (H / 2),
                                     reinterpret_cast<const uint8_t *>(g1.w) + row * (H / 2), g0.sc4 + row * (H / 16),
-                                    g1.sc4 + row * (H / 16), x16, p_tok + pb, rows, L, ag, au);
+                                    g1.sc4 + row * (H / 16), x16, pairs + pb, S, rows, L, ag, au);
     } else {
         const size_t row = grp < E ? (size_t)grp * I + o0 : (size_t)o0;
         sg = *reinterpret_cast<const f32x4_t *>((grp < E ? g0.s : g0.s_sh) + row + 4 * g);
         su = *reinterpret_cast<const f32x4_t *>((grp < E ? g1.s : g1.s_sh) + row + 4 * g);
-        mid_gu_body<H, I, false, NT>(reinterpret_cast<const uint8_t *>(grp < E ? g0.w : g0.w_sh) + row * H,
+        mid_gu_body<H, I, false, NT, ONCE>(reinterpret_cast<const uint8_t *>(grp < E ? g0.w : g0.w_sh) + row * H,
                                      reinterpret_cast<const uint8_t *>(grp < E ? g1.w : g1.w_sh) + row * H, nullptr,
-                                     nullptr, x16, p_tok + pb, rows, L, ag, au);
+                                     nullptr, x16, pairs + pb, S, rows, L, ag, au);
     }
     // hidden = silu(g) * u, then fp16 scaled by the power of two of the block's
     // 64 rows of each token
@@ -404,7 +429,7 @@ k_mid_gateup(const int4 *__restrict__ items, const int *__restrict__ n_items, co
 #pragma unroll
     for (int n = 0; n < NT; n++) {
         const int t = n * 16 + l16;
-        const float isc = t < rows ? x16isc[p_tok[pb + t]] : 0.0f;
+        const float isc = t < rows ? x16isc[pairs[pb + t].x / S] : 0.0f;
         m[n] = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -457,19 +482,18 @@ struct MidHidStage {
     }
 };
 
-template <int H, int I, bool F4, int NT>
+template <int H, int I, bool F4, int NT, bool ONCE>
 __global__ void __launch_bounds__(64 * mid_dn_waves(I, NT))
-k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, const int *__restrict__ p_slot,
-           const float *__restrict__ p_wt, const uint16_t *__restrict__ hid, const int8_t *__restrict__ hk, GroupW gd,
+k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, const int2 *__restrict__ pairs,
+           const uint16_t *__restrict__ hid, const int8_t *__restrict__ hk, GroupW gd,
            int E, uint16_t *__restrict__ part, int8_t *__restrict__ partk) {
     constexpr int CW = 64 * mid_dn_waves(I, NT), NCB = H / CW;    // columns per block, blocks per item
     static_assert(NCB * CW == H, "whole blocks of columns");
     __shared__ __align__(16) MidDnLds<I, NT> L;
-    const int item = (int)blockIdx.x / NCB, cb = (int)blockIdx.x - item * NCB;
-    const int nit = n_items[0];
+    const int u = xcd_unit(blockIdx.x, n_items[0] * NCB);
+    if (u < 0) return;
+    const int item = u / NCB, cb = u - item * NCB;
     const int4 it = items[item];
-    args_now(nit, it.x, it.y, it.z);
-    if (item >= nit) return;
     const int grp = it.x, pb = it.y, rows = it.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const int c0 = cb * CW + wave * 64;
@@ -480,14 +504,14 @@ k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, cons
         const float a = gd.s2[grp];
 #pragma unroll
         for (int rt = 0; rt < 4; rt++) sd[rt] = f32x4_t{a, a, a, a};
-        mid_dn_body<I, true, NT>(reinterpret_cast<const uint8_t *>(gd.w) + row * (I / 2), gd.sc4 + row * (I / 16), rows,
+        mid_dn_body<I, true, NT, ONCE>(reinterpret_cast<const uint8_t *>(gd.w) + row * (I / 2), gd.sc4 + row * (I / 16), rows,
                                  L, acc, st, tid);
     } else {
         const size_t row = grp < E ? (size_t)grp * H + c0 : (size_t)c0;
 #pragma unroll
         for (int rt = 0; rt < 4; rt++)
             sd[rt] = *reinterpret_cast<const f32x4_t *>((grp < E ? gd.s : gd.s_sh) + row + rt * 16 + 4 * g);
-        mid_dn_body<I, false, NT>(reinterpret_cast<const uint8_t *>(grp < E ? gd.w : gd.w_sh) + row * I, nullptr, rows,
+        mid_dn_body<I, false, NT, ONCE>(reinterpret_cast<const uint8_t *>(grp < E ? gd.w : gd.w_sh) + row * I, nullptr, rows,
                                   L, acc, st, tid);
     }
     // the wave's 64 columns of each token as fp16 scaled by 2^k (k from the
@@ -496,8 +520,9 @@ k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, cons
     for (int n = 0; n < NT; n++) {
         const int t = n * 16 + l16;
         const bool live = t < rows;
-        const float w = live ? p_wt[pb + t] : 0.0f;
-        const int slot = live ? p_slot[pb + t] : 0;
+        const int2 pr = live ? pairs[pb + t] : make_int2(0, 0);
+        const float w = __int_as_float(pr.y);
+        const int slot = pr.x;
         float m = 0.0f;
 #pragma unroll
         for (int rt = 0; rt < 4; rt++)
@@ -528,16 +553,18 @@ k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, cons
 int launch_mid(const MidArgs &a, hipStream_t s) {
     const Cfg &c = g_cfg;
     const int T = a.T, E = c.E, K = c.K, H = c.H, I = c.I;
-    const int ng = (T + 7) / 8, nx = E / 8 + (a.g ? 1 : 0);
-    const int tg = max(1, ng * nx / 1536);                     // token groups per router block: ~1536 blocks
-    const unsigned g_r = (unsigned)((T + 3) / 4 + nx * ((ng + tg - 1) / tg));
-    if (H == 2048)
-        hipLaunchKernelGGL(k_mid_router<8>, dim3(g_r), dim3(256), 0, s, a.router, a.bias, a.g, a.x, T, E, tg, a.logits,
-                           a.gam, a.x16, a.x16isc, a.ctr);
-    else
-        hipLaunchKernelGGL(k_mid_router<10>, dim3(g_r), dim3(256), 0, s, a.router, a.bias, a.g, a.x, T, E, tg, a.logits,
-                           a.gam, a.x16, a.x16isc, a.ctr);
-    hipLaunchKernelGGL(k_mid_topk<8>, dim3((T + 3) / 4), dim3(256), 0, s, a.logits, T, K, c.renorm, a.sel, a.wts, a.ctr);
+    if (T <= kMidExactRows) {                                  // (beyond: the caller has launched router and selection)
+        const int ng = (T + 7) / 8, nx = E / 8 + (a.g ? 1 : 0);
+        const int tg = max(1, ng * nx / 1536);                     // token groups per router block: ~1536 blocks
+        const unsigned g_r = (unsigned)((T + 3) / 4 + nx * ((ng + tg - 1) / tg));
+        if (H == 2048)
+            hipLaunchKernelGGL(k_mid_router<8>, dim3(g_r), dim3(256), 0, s, a.router, a.bias, a.g, a.x, T, E, tg, a.logits,
+                               a.gam, a.x16, a.x16isc, a.ctr);
+        else
+            hipLaunchKernelGGL(k_mid_router<10>, dim3(g_r), dim3(256), 0, s, a.router, a.bias, a.g, a.x, T, E, tg, a.logits,
+                               a.gam, a.x16, a.x16isc, a.ctr);
+        hipLaunchKernelGGL(k_mid_topk<8>, dim3((T + 3) / 4), dim3(256), 0, s, a.logits, T, K, c.renorm, a.sel, a.wts, a.ctr);
+    }
     // token tiles per item. One (16 rows) keeps three blocks on a CU, which
     // streams best, and an expert's further items find its weights in L2:
     // gate/up + down, us, at 300 / 1021 / 1500 / 2000 rows with one, two and
@@ -545,24 +572,29 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
     // 425 / 462; NVFP4 198 / 345 / 422 / 500, 278 / 386 / 462 / 580, 436 / 526 /
     // 599 / 688. Four are taken for INT8 from 24 rows an expert.
     const int avg = T * K / E;
-    const int nt = avg < 24 || a.f4 ? 1 : 4, mt = 16 * nt;
+    const int nt = avg < 24 || a.f4 || I > 512 ? 1 : 4, mt = 16 * nt;
     hipLaunchKernelGGL(k_mid_plan, dim3(1), dim3(1024), 0, s, a.sel, a.wts, a.g ? a.gam : nullptr, T, K, E, a.has_sh, mt,
-                       a.p_tok, a.p_slot, a.p_wt, a.items, a.ctr + 1);
+                       a.pairs, a.items, a.ctr + 1);
     // items: one per distinct expert, one more per full mt rows, the shared group's
     const int max_items = min(E, T * K) + T * K / mt + (a.has_sh ? (T + mt - 1) / mt : 0);
     if (max_items > a.max_items) { set_error(-2, "mid path: %d items, room for %d", max_items, a.max_items); return -2; }
     const int dw = 64 * mid_dn_waves(I, nt);                      // columns, and threads, per down block
-    const dim3 g_gu((unsigned)(max_items * (I / 64))), g_dn((unsigned)(max_items * (H / dw))), b(256), bd((unsigned)dw);
-#define QFM_MID(HH, II, F4, NT)                                                                                     \
-    hipLaunchKernelGGL((k_mid_gateup<HH, II, F4, NT>), g_gu, b, 0, s, a.items, a.ctr + 1, a.p_tok,                  \
-                       reinterpret_cast<const uint16_t *>(a.x16), a.x16isc, a.gg, a.gu, E, a.hid, a.hk);            \
-    hipLaunchKernelGGL((k_mid_down<HH, II, F4, NT>), g_dn, bd, 0, s, a.items, a.ctr + 1, a.p_slot, a.p_wt, a.hid,    \
+    // (xcd_unit wants eight times the largest range: a multiple of 8)
+    const dim3 g_gu((unsigned)((max_items * (I / 64) + 7) / 8 * 8)), g_dn((unsigned)((max_items * (H / dw) + 7) / 8 * 8)), b(256), bd((unsigned)dw);
+#define QFM_MID(HH, II, F4, NT, ONCE)                                                                               \
+    hipLaunchKernelGGL((k_mid_gateup<HH, II, F4, NT, ONCE>), g_gu, b, 0, s, a.items, a.ctr + 1, a.pairs,            \
+                       K + a.has_sh, reinterpret_cast<const uint16_t *>(a.x16), a.x16isc, a.gg, a.gu, E, a.hid,     \
+                       a.hk);                                                                                       \
+    hipLaunchKernelGGL((k_mid_down<HH, II, F4, NT, ONCE>), g_dn, bd, 0, s, a.items, a.ctr + 1, a.pairs, a.hid,      \
                        a.hk, a.gd, E, a.part, a.partk)
+#define QFM_MID_ONCE(HH, II, F4)                                                                                    \
+    if (avg < (F4 ? 8 : 12)) { QFM_MID(HH, II, F4, 1, true); } else { QFM_MID(HH, II, F4, 1, false); }
     if (shape_2048()) {
-        if (a.f4) { QFM_MID(2048, 512, true, 1); } else if (nt == 1) { QFM_MID(2048, 512, false, 1); } else { QFM_MID(2048, 512, false, 4); }
+        if (a.f4) { QFM_MID_ONCE(2048, 512, true) } else if (nt == 1) { QFM_MID_ONCE(2048, 512, false) } else { QFM_MID(2048, 512, false, 4, false); }
     } else {
-        if (a.f4) { QFM_MID(2560, 640, true, 1); } else if (nt == 1) { QFM_MID(2560, 640, false, 1); } else { QFM_MID(2560, 640, false, 4); }
+        if (a.f4) { QFM_MID_ONCE(2560, 640, true) } else { QFM_MID_ONCE(2560, 640, false) }
     }
+#undef QFM_MID_ONCE
 #undef QFM_MID
     return 0;
 }

@@ -433,9 +433,11 @@ struct TileEngine {
 
 // router GEMM: 128 x 128 tiles, 2 x 2 waves; grouped expert GEMMs: 128 x 256, 2 x 4 waves
 using RouterEngine = TileEngine<kB_BF16, 2, 2, 4, 2>;
-// router GEMM slices along H, summed in slice order by k_pf_select (2 measured
-// 5% slower than 1 at T = 8038: the 63 m-tiles x 4 n-tiles already fill the chip)
+// router GEMM slices along H the workspace counts for its logits region; more
+// slices borrow another region (launch_prefill)
 constexpr int kRouterKS = 1;
+// up to here four waves select a token's experts, beyond it one (k_pf_select)
+constexpr int kSelectSplitRows = 1100;
 // INT8 tiles: 128 x 256 in 8 waves of 64 x 64 (two waves per SIMD). Four
 // waves of 128 x 64 (MW = 8: one wave per SIMD, accumulators in AGPRs, 25%
 // fewer LDS reads per MFMA) measured 1343 / 1149 us against 797 / 719 us.
@@ -491,7 +493,7 @@ k_pf_router_mfma(const uint16_t *__restrict__ x, int T, int H, const uint16_t *_
     __shared__ int arow[BM];
     __shared__ const char *bptr[BN];
     int mt, et;
-    const int ks = blockIdx.y, Hk = H / kRouterKS, k0 = ks * Hk;     // this block's slice of H
+    const int ks = blockIdx.y, Hk = H / (int)gridDim.y, k0 = ks * Hk;   // this block's slice of H
     xcd_tile(blockIdx.x, E / BN, mt, et);
     if (mt * BM >= T) return;
     const int t0 = mt * BM, e0 = et * BN;
@@ -564,64 +566,75 @@ __device__ __forceinline__ float bound_coeff(int H) {
     return 2.0f * (0x1p-9f + (float)(2 * H) * 0x1p-24f + (float)(H / 64 + 8) * 0x1p-24f);
 }
 
-// one wave per token: candidates, exact logits, exact top-K, shared gate
-template <int NJ, int EPL>
+// Candidates, exact logits, exact top-K and the shared gate, WPT waves per
+// token. lg_part: the router GEMM's nks partial logits [nks][T][E], summed in
+// slice order; their sum goes to lg. Every wave of a token forms the bounds and
+// the candidate list itself (no barrier) and recomputes every WPT-th candidate;
+// the first wave ranks them. tau, a lower bound of the K-th largest logit, is
+// the K-th largest of the 64 lane maxima of the lower bounds (K distinct
+// experts reach it): one rank pass instead of K wave-wide maxima, for about one
+// candidate more. One wave per token is bound by its chain of L2 round trips
+// while the tokens do not fill the chip: four waves take up to kSelectSplitRows
+// (450 / 1021 / 1500 rows 19 / 23 / 36 us; K wave-wide maxima and one wave a
+// token: 25 / 30 / 31 us; 8038 rows one wave 76 -> 68 us).
+template <int NJ, int WPT>
 __global__ void __launch_bounds__(256)
 k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, const float *__restrict__ bias,
-            const float *__restrict__ g, float *__restrict__ lg_approx, const float *__restrict__ xnorm,
-            const float *__restrict__ wnorm, int K, int renorm, int *__restrict__ sel, float *__restrict__ wts,
-            float *__restrict__ gam, int *__restrict__ n_fallback) {
-    constexpr int H = NJ * 256, E = EPL * 64;
+            const float *__restrict__ g, const float *__restrict__ lg_part, int nks, float *__restrict__ lg,
+            const float *__restrict__ xnorm, const float *__restrict__ wnorm, int K, int renorm,
+            int *__restrict__ sel, float *__restrict__ wts, float *__restrict__ gam, int *__restrict__ n_fallback) {
+    constexpr int H = NJ * 256, EPL = 8, E = EPL * 64, TPB = 4 / WPT;
+    __shared__ __align__(16) uint32_t s_lm[4][64];
     __shared__ int s_cand[4][kCandMax];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t = blockIdx.x * 4 + wave;
-    if (t >= T) return;
+    __shared__ __align__(16) unsigned long long s_key[TPB][kCandMax], s_top[TPB][16];
+    __shared__ float s_lg[TPB][E];                       // every logit exact (overflow, or no renormalization)
+    __shared__ __align__(16) unsigned long long s_tk[TPB][kTopkLds];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, tb = wave / WPT, w = wave % WPT;
+    const int t = blockIdx.x * TPB + tb;
+    if (t >= T) return;                                  // (WPT == 4: block-uniform)
     const uint16_t *xt = x + (size_t)t * H;
     const float cB = bound_coeff(H) * xnorm[t];
-    float lo[EPL], hi[EPL];
+    float l[EPL], hi[EPL];
+#pragma unroll
+    for (int i = 0; i < EPL; i++) l[i] = 0.0f;
+    for (int q = 0; q < nks; q++)
+#pragma unroll
+        for (int i = 0; i < EPL; i++) {
+            const float *p = lg_part + ((size_t)q * T + t) * E + i * 64 + lane;
+            l[i] += WPT == 1 ? __builtin_nontemporal_load(p) : *p;
+        }
+    uint32_t mx = 0u;                                    // the lane's largest lower bound (sortable bits)
 #pragma unroll
     for (int i = 0; i < EPL; i++) {
         const int e = i * 64 + lane;
-        float l = 0.0f;
-#pragma unroll
-        for (int q = 0; q < kRouterKS; q++) l += __builtin_nontemporal_load(&lg_approx[((size_t)q * T + t) * E + e]);   // slice order
-        if (bias) l += bias[e];
-        // the approximate logits, the x row and their write-back are touched once per
-        // token: nontemporal, so the router rows of the candidates stay in L2
-        __builtin_nontemporal_store(l, &lg_approx[(size_t)t * E + e]);          // the view's approximate logits
-        const float b = cB * wnorm[e] + 1e-6f * (fabsf(l) + (bias ? fabsf(bias[e]) : 0.0f) + 1.0f);
-        lo[i] = l - b;
-        hi[i] = l + b;
+        const float be = bias ? bias[e] : 0.0f;
+        if (bias) l[i] += be;
+        // the logits and x are touched once per token: nontemporal, so the router rows of the candidates stay in L2
+        if (w == 0) __builtin_nontemporal_store(l[i], &lg[(size_t)t * E + e]);
+        const float b = cB * wnorm[e] + 1e-6f * (fabsf(l[i]) + fabsf(be) + 1.0f);
+        hi[i] = l[i] + b;
+        mx = max(mx, (uint32_t)(topk_key(l[i] - b, 0) >> 32));
     }
-    // tau = K-th largest lower bound (K rounds of a wave-wide maximum)
-    float tau;
-    {
-        // K-th largest of lo[] by repeated wave max (K <= 16, values need not be distinct)
-        unsigned long long kk[EPL];
+    s_lm[wave][lane] = mx;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    int rank = 0;
 #pragma unroll
-        for (int i = 0; i < EPL; i++) kk[i] = topk_key(lo[i], i * 64 + lane);
-        unsigned long long b = 0;
-        for (int k = 0; k < K; k++) {
-            b = 0;
+    for (int q = 0; q < 16; q++) {
+        const uint4 p = reinterpret_cast<const uint4 *>(s_lm[wave])[q];
+        const uint32_t d[4] = {p.x, p.y, p.z, p.w};
 #pragma unroll
-            for (int i = 0; i < EPL; i++) b = kk[i] > b ? kk[i] : b;
-            b = __ockl_wfred_max_u64(b);
-#pragma unroll
-            for (int i = 0; i < EPL; i++) kk[i] = kk[i] == b ? 0ull : kk[i];
-        }
-        tau = topk_key_value(b);
+        for (int u = 0; u < 4; u++) rank += (d[u] > mx || (d[u] == mx && 4 * q + u < lane)) ? 1 : 0;
     }
-    // candidates: hi >= tau
-    int cnt = 0;
+    const uint32_t tk = (uint32_t)__builtin_amdgcn_readlane((int)mx, __builtin_ctzll(__ballot(rank == K - 1)));
+    const float tau = topk_key_value((unsigned long long)tk << 32);
+    // candidates: not below tau (a NaN bound makes every expert one)
+    unsigned long long cb[EPL];
+    int total = 0, pos[EPL];
 #pragma unroll
-    for (int i = 0; i < EPL; i++) cnt += hi[i] >= tau ? 1 : 0;
-    const unsigned long long ltm = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    int off = 0, total = 0;
-#pragma unroll
-    for (int bt = 0; bt < 5; bt++) {
-        const unsigned long long bb = __ballot((cnt >> bt) & 1);
-        off += __popcll(bb & ltm) << bt;
-        total += __popcll(bb) << bt;
+    for (int i = 0; i < EPL; i++) {
+        cb[i] = __ballot(!(hi[i] < tau));
+        pos[i] = __builtin_amdgcn_mbcnt_hi((uint32_t)(cb[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cb[i], (uint32_t)total));
+        total += __popcll(cb[i]);
     }
     // Without renormalization the weights divide by the softmax denominator over
     // all E logits, so every logit is recomputed exactly (the M <= 8 path's
@@ -631,70 +644,69 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
     if (!full) {
 #pragma unroll
         for (int i = 0; i < EPL; i++)
-            if (hi[i] >= tau) s_cand[wave][off++] = i * 64 + lane;
-    } else if (overflow && lane == 0) {
-        atomicAdd(n_fallback, 1);
+            if ((cb[i] >> lane) & 1ull) s_cand[wave][pos[i]] = i * 64 + lane;
     }
+    if (overflow && renorm && w == 0 && lane == 0) atomicAdd(n_fallback, 1);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const int nc = full ? E : total;
-    // exact logits of the candidates (all E on overflow) -> 64-bit keys; lane k < K
-    // keeps the k-th best key so far (descending), maintained by insertion
-    unsigned long long best = 0;
-    float xv[NJ][4];                                // this token's x slice, canonical lane layout
+    float xv[NJ][4];                                     // this token's x slice, canonical lane layout
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const u32x2_t p = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t *>(xt + j * 256 + lane * 4));
         xv[j][0] = bf16_lo(p.x); xv[j][1] = bf16_hi(p.x); xv[j][2] = bf16_lo(p.y); xv[j][3] = bf16_hi(p.y);
     }
-    constexpr int CB = 4;                           // candidates per batch of loads
-    float exl[EPL];                                 // full: exact logit of expert i * 64 + lane
-#pragma unroll
-    for (int i = 0; i < EPL; i++) exl[i] = 0.0f;
-    for (int c0 = 0; c0 < nc; c0 += CB) {
+    constexpr int CB = 4;                                // candidates per batch of loads
+    for (int c0 = w; c0 < nc; c0 += CB * WPT) {
         int eb[CB];
 #pragma unroll
         for (int q = 0; q < CB; q++) {
-            const int c = c0 + q < nc ? c0 + q : c0;  // past the end: repeat a candidate, result dropped
+            const int c = c0 + q * WPT < nc ? c0 + q * WPT : c0;   // past the end: repeat a candidate, result dropped
             eb[q] = full ? c : s_cand[wave][c];
         }
         float lb[CB];
         canon_dot_wave_batch<NJ, CB>(W, H, eb, xv, lane, lb);
 #pragma unroll
         for (int q = 0; q < CB; q++) {
-            if (c0 + q >= nc) break;
-            float l = lb[q];
-            if (bias) l = __fadd_rn(l, bias[eb[q]]);
-            if (full) {                             // keep it in the lane that owns expert eb[q]
-#pragma unroll
-                for (int i = 0; i < EPL; i++)
-                    if (eb[q] == i * 64 + lane) exl[i] = l;
+            const int c = c0 + q * WPT;
+            if (c >= nc) break;
+            const float v = bias ? __fadd_rn(lb[q], bias[eb[q]]) : lb[q];
+            if (lane == 0) {
+                if (full) s_lg[tb][c] = v;
+                else s_key[tb][c] = topk_key(v, eb[q]);
             }
-            const unsigned long long key = topk_key(l, eb[q]);
-            // insert into the sorted lane list: lanes with a smaller key shift down
-            const unsigned long long prev = __shfl_up(best, 1, WAVE);
-            const bool ge_prev = lane == 0 || prev > key;
-            if (lane < K && best < key) best = ge_prev ? key : prev;
         }
     }
-    const float mx = topk_key_value(__shfl(best, 0, WAVE));
-    const float ek = lane < K ? __expf(topk_key_value(best) - mx) : 0.0f;
-    float denom = __ockl_wfred_add_f32(ek);
-    if (!renorm) {                                  // every logit is exact here (full)
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < EPL; i++) s += __expf(exl[i] - mx);
-        denom = __ockl_wfred_add_f32(s);
-    }
-    if (lane < K) {
-        sel[(size_t)t * K + lane] = topk_key_index(best);
-        wts[(size_t)t * K + lane] = ek / denom;
-    }
-    if (g) {
+    if (g && w == WPT - 1) {
         const int e0[1] = {0};
         float gdv[1];
         canon_dot_wave_batch<NJ, 1>(g, H, e0, xv, lane, gdv);   // x from registers
-        const float gd = gdv[0];
-        if (lane == 0) gam[t] = sigmoid(gd);
+        if (lane == 0) gam[t] = sigmoid(gdv[0]);
+    }
+    if constexpr (WPT > 1) __syncthreads();
+    else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (w != 0) return;
+    int my_i;
+    float my_w;
+    if (full) {
+        float v[EPL];
+#pragma unroll
+        for (int i = 0; i < EPL; i++) v[i] = s_lg[tb][i * 64 + lane];
+        wave_topk_regs<EPL>(v, K, renorm, lane, s_tk[tb], my_i, my_w);
+    } else {                                             // K <= total <= 64 candidates, one per lane
+        const unsigned long long key = lane < total ? s_key[tb][lane] : 0ull;
+        int r = 0;
+        for (int c = 0; c < total; c++) r += s_key[tb][c] > key ? 1 : 0;
+        if (lane < total && r < K) s_top[tb][r] = key;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const unsigned long long mine = lane < K ? s_top[tb][lane] : 0ull;
+        const float mxv = topk_key_value(s_top[tb][0]);
+        const float ek = lane < K ? __expf(topk_key_value(mine) - mxv) : 0.0f;
+        my_i = topk_key_index(mine);
+        my_w = ek / __ockl_wfred_add_f32(ek);
+    }
+    if (lane < K) {
+        sel[(size_t)t * K + lane] = my_i;
+        wts[(size_t)t * K + lane] = my_w;
     }
 }
 
@@ -1178,29 +1190,45 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
         gu = GroupW{a->i8_up, a->i8s_up, L->sh_up.w, L->sh_up.s, nullptr, nullptr};
         gd = GroupW{a->i8_down, a->i8s_down, L->sh_down.w, L->sh_down.s, nullptr, nullptr};
     }
-    if (T <= kMidRowsMax) {
+    // router and selection: exact logits of every expert up to kMidExactRows
+    // rows (launch_mid), the bf16 MFMA GEMM with exact candidates beyond
+    const bool mid = T <= mid_rows_max(I, f4);
+    if (!mid || T > kMidExactRows) {
+        // zero the small counters with a fill kernel (no memset node in captured graphs)
+        launch_fill_f32(reinterpret_cast<float *>(ctr), 8, 0.0f, s);
+        hipLaunchKernelGGL(k_pf_router_prep, dim3((unsigned)(E + (T + 3) / 4)), dim3(256), 0, s, L->router, E, H, wnorm,
+                           wb16, x, T, xnorm, xsum, mid || !f4 ? x16 : nullptr, x16sum, x16isc);
+        // few m-tiles: K in slices until the chip is full (their partial logits lie
+        // in the region of the partials, which the down GEMM writes later; that
+        // has room for two at top_k 1 without a shared expert): 1021 rows 31 -> 13 us
+        const size_t room = Lw.bytes[kPfPart] / ((size_t)T * E * sizeof(float));
+        const int nks = T <= 2048 && room >= 4 ? 4 : T <= 4096 && room >= 2 ? 2 : 1;
+        float *lgp = nks > 1 ? reinterpret_cast<float *>(part) : lg;
+        const int mt_router = ((T + BM - 1) / BM + 7) / 8 * 8;
+        hipLaunchKernelGGL(k_pf_router_mfma, dim3(mt_router * (E / BN), nks), dim3(256), 0, s, x, T, H, wb16, E, lgp);
+#define QFM_PF_SELECT(NJ, WPT)                                                                                      \
+    hipLaunchKernelGGL((k_pf_select<NJ, WPT>), dim3((unsigned)((T * WPT + 3) / 4)), dim3(256), 0, s, x, T,          \
+                       L->router, L->router_bias, g, lgp, nks, lg, xnorm, wnorm, K, c.renorm, sel, wts, gam, ctr)
+        if (H == 2048) {
+            if (T <= kSelectSplitRows) { QFM_PF_SELECT(8, 4); } else { QFM_PF_SELECT(8, 1); }
+        } else {
+            if (T <= kSelectSplitRows) { QFM_PF_SELECT(10, 4); } else { QFM_PF_SELECT(10, 1); }
+        }
+#undef QFM_PF_SELECT
+    }
+    if (mid) {
         // the middle path uses the same regions (hid as scaled fp16, its
-        // exponents in the hsum region, one item list)
+        // exponents in the hsum region, one item list, 8-byte pairs over the
+        // token and slot regions)
+        static_assert(kPfSlot == kPfTok + 1, "the pairs span two adjacent regions");
         const MidArgs m{L->router, L->router_bias, g, x, T, has_sh ? 1 : 0, f4, lg, sel, wts, gam, x16, x16isc, ctr,
-                        p_tok, p_slot, p_wt, items_gu, (int)(Lw.bytes[kPfItemsGu] / sizeof(int4)), hid,
+                        reinterpret_cast<int2 *>(p_tok), items_gu, (int)(Lw.bytes[kPfItemsGu] / sizeof(int4)), hid,
                         reinterpret_cast<int8_t *>(hsum), part, partk, gg, gu, gd};
         if (const int rc = launch_mid(m, s)) return rc;
         hipLaunchKernelGGL(k_pf_combine_h, dim3((unsigned)(((size_t)T * H / 4 + 255) / 256)), dim3(256), 0, s, part,
                            partk, T, S, H, y, y32);
         return check_launch("prefill");
     }
-    // zero the small counters with a fill kernel (no memset node in captured graphs)
-    launch_fill_f32(reinterpret_cast<float *>(ctr), 8, 0.0f, s);
-    hipLaunchKernelGGL(k_pf_router_prep, dim3((unsigned)(E + (T + 3) / 4)), dim3(256), 0, s, L->router, E, H, wnorm,
-                       wb16, x, T, xnorm, xsum, f4 ? nullptr : x16, x16sum, x16isc);
-    const int mt_router = ((T + BM - 1) / BM + 7) / 8 * 8;
-    hipLaunchKernelGGL(k_pf_router_mfma, dim3(mt_router * (E / BN), kRouterKS), dim3(256), 0, s, x, T, H, wb16, E, lg);
-    if (H == 2048)
-        hipLaunchKernelGGL((k_pf_select<8, 8>), dim3((T + 3) / 4), dim3(256), 0, s, x, T, L->router, L->router_bias,
-                           g, lg, xnorm, wnorm, K, c.renorm, sel, wts, gam, ctr);
-    else
-        hipLaunchKernelGGL((k_pf_select<10, 8>), dim3((T + 3) / 4), dim3(256), 0, s, x, T, L->router, L->router_bias,
-                           g, lg, xnorm, wnorm, K, c.renorm, sel, wts, gam, ctr);
     hipLaunchKernelGGL(k_pf_count, dim3(nblk), dim3(256), 0, s, sel, T * K, E, blk);
     hipLaunchKernelGGL(k_pf_plan, dim3(1), dim3(1024), 0, s, blk, nblk, E, has_sh ? 1 : 0, T, nt_gu, nt_dn, off,
                        items_gu, items_dn, ctr + 1, (int)(max_mt * nt_gu), (int)(max_mt * nt_dn));

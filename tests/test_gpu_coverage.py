@@ -158,10 +158,10 @@ def test_prefill_tile_boundaries(lib, T, fmt):
 # ------------------------------------------------------------------ middle row counts
 @pytest.mark.parametrize("hidden,inter,T,fmt,hot", [
     (2048, 512, 9, 1, 0), (2048, 512, 16, 0, 16), (2048, 512, 33, 1, 17), (2560, 640, 31, 0, 33), (2560, 640, 17, 1, 1),
-    (2560, 640, 65, 1, 65), (2560, 640, 1300, 0, 65)])
+    (2560, 640, 65, 1, 65), (2560, 640, 601, 0, 65), (2048, 512, 1300, 0, 65)])
 def test_middle_rows(lib, hidden, inter, T, fmt, hot):
-    """9 to 1536 rows run as weight-streaming items of 16 (INT8 from 24 rows an
-    expert: 64) rows per expert; 1537 rows are the first of the prefill tiles.
+    """9 to 2800 rows (2560/640: 1800 INT8, 2500 NVFP4) run as weight-streaming
+    items of 16 (2048/512 INT8 from 24 rows an expert: 64) rows per expert.
     `hot` rows are copies of row 0, so that its ten experts get at least that
     many rows: counts at and around whole items, beside experts with one row and
     with none. Routing bit-exact, the exact logits in the workspace view, and y
@@ -185,10 +185,11 @@ def test_middle_rows(lib, hidden, inter, T, fmt, hot):
     r = orc.moe_layer_grouped(hidden, inter, E, K, T, seed, layer, xl, x=x, fmt=fmt)
     assert np.array_equal(qfm.d2h(view.sel, np.int32, (T, K)), r["sel"])
     assert np.allclose(qfm.d2h(view.wts, np.float32, (T, K)), r["w"], rtol=2e-6, atol=1e-7)
-    W = orc.fill("gauss", seed, layer, orc.T_ROUTER, 0, E * hidden, scale=0.02).reshape(E, hidden)
-    rows = [0, T // 2, T - 1]
-    lg = qfm.d2h(view.logits, np.float32, (T, E))
-    assert np.array_equal(lg[rows].view(np.uint32), orc.router_logits(W, x[rows]).view(np.uint32))
+    if T <= 600:                                         # (beyond: approximate logits, exact ones for the candidates)
+        W = orc.fill("gauss", seed, layer, orc.T_ROUTER, 0, E * hidden, scale=0.02).reshape(E, hidden)
+        rows = [0, T // 2, T - 1]
+        lg = qfm.d2h(view.logits, np.float32, (T, E))
+        assert np.array_equal(lg[rows].view(np.uint32), orc.router_logits(W, x[rows]).view(np.uint32))
     rel = max(_rel(y[t], r["y"][t]) for t in range(T))
     _say("  max rel err", rel)
     assert rel <= TOL
@@ -206,7 +207,7 @@ def test_middle_rows_upper_edge(lib, fmt):
     _say("middle rows, upper edge, fmt", fmt)
     qfm.init(H, I, E, K, 1, 1)
     st = qfm.Stream()
-    T = 1536
+    T = 2800
     L = qfm.SynthLayer(fmt, 8, 2, stream=st)
     x = orc.fill("gauss_bf16", 8, 61, orc.T_X, 0, (T + 1) * H).reshape(T + 1, H)
     a, b = _forward(lib, L.s.layer, x[:T], st), _forward(lib, L.s.layer, x, st)
