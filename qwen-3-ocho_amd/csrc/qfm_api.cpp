@@ -390,6 +390,13 @@ static int forward_impl(const qfm_layer *L, const uint16_t *x, int M, uint16_t *
         if (marks) { pm[3] = prof_event(s); g_prof.marks.push_back(pm); }
         return rc;
     }
+    if (M == 1 && L->fmt == QFM_FMT_NVFP4 && !shape_shard()) {
+        // the same three launches on the NVFP4 arena (hidden: K routed rows, then the shared one)
+        int rc = launch_router_shared(L->router, L->router_bias, g, nullptr, x, 1, logits, ld, hidden, c.I, s);
+        if (!rc) rc = launch_f4_m1(L->arena, sp, x, logits, g ? logits + c.E : nullptr, sel, wts, hidden,
+                                   reinterpret_cast<uint32_t *>(b + w.ctl), y32, y, s);
+        return rc;
+    }
     if (M <= 8) {
         float *hsh = hidden + (size_t)M * c.K * c.I;
         // the router launch also ranks every row (its selection tail) and, for

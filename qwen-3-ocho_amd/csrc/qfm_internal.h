@@ -85,6 +85,13 @@ int launch_x8(const float *x, int8_t *q, float *sc, int n, hipStream_t s);
 int launch_i8_down_m1(const Qf4ExpCache *c, const float *hidden, const float *wts, const int *sel,
                       int nexp, const ShPtrs *sh, const float *gdot, float *y32, uint16_t *ybf, hipStream_t s);
 
+// NVFP4 M = 1, after launch_router_shared (no tail, no shared rows): the top-K
+// in the gate/up launch, whose last job is the shared expert (hidden row K),
+// then down + combine into y32 or ybf. Advances ctl[0], as every NVFP4 call of
+// the M <= 8 forward does.
+int launch_f4_m1(const Qf4ExpCache *a, const ShPtrs *sh, const uint16_t *x, const float *logits, const float *gdot,
+                 int *sel, float *wts, float *hidden, uint32_t *ctl, float *y32, uint16_t *ybf, hipStream_t s);
+
 // Multi-row decode (1 <= M <= 8), after launch_router_shared with its selection
 // tail (sel/wts [M][K], INT8: the fp16 activation chunks in xh16): gate/up
 // keyed by pair (k_csr_gateup: the first pair of each distinct expert reads
