@@ -59,6 +59,15 @@ __device__ __forceinline__ f32x4_t mfma_f16(f16x8_t a, f16x8_t b, f32x4_t c) {
 __device__ __forceinline__ f32x4_t mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+// no block-scale byte of the vector is 0x7F or more (a carry into a byte can only
+// make this false)
+template <class V>
+__device__ __forceinline__ bool f4_scales_hw(V s) {
+    uint32_t bad = 0u;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(V) / 4); i++) bad |= s[i] | (s[i] + 0x01010101u);
+    return (bad & 0x80808080u) == 0u;
+}
 // LDS rows of STRIDE bytes: 16-byte chunk c of row r at chunk position c ^
 // lds_rot(r), so that the 16 rows of a fragment read spread over the 64 banks
 template <int STRIDE>
@@ -134,51 +143,67 @@ __device__ __forceinline__ void mid_dn_body(const uint8_t *__restrict__ wd, cons
             const int c = j * 64 + lane;
             *reinterpret_cast<u32x4_t *>(lw + lds_at<ROWB>(c / CPR, c % CPR)) = buf[rt % D][j];
         }
-        if constexpr (F4)
+        // NVFP4: whether every block scale of the tile is below 0x7F (one test, and
+        // one branch, per tile: tested per 64 values the branches kept the
+        // fragments' LDS reads and conversions from overlapping)
+        bool hw = true;
+        if constexpr (F4) {
             if (lane < SL) *reinterpret_cast<u32x4_t *>(lw + 16 * ROWB + lane * 16) = sc[rt % D];
+            hw = __builtin_amdgcn_ballot_w64(lane < SL && !f4_scales_hw(sc[rt % D])) == 0;
+        }
         if (rt + D < RT) wload(rt + D);
         wave_lds_fence();
 #pragma unroll
         for (int n = 0; n < NT; n++) acc[rt][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (int kg = 0; kg < NG; kg++) {
-            // hidden values 64 kg + 16 g .. + 15 of token l16, weights of row l16
-            auto hfrag = [&](int n, int h) __attribute__((always_inline)) {
-                return *reinterpret_cast<const f16x8_t *>(L.h + lds_at<HS>(n * 16 + l16, 8 * kg + 2 * g + h));
-            };
-            auto add = [&](int n, f32x4_t d) __attribute__((always_inline)) {
-                const float s = L.isc[n * 16 + l16][kg];
+        // 64 values kg: hidden values 64 kg + 16 g .. + 15 of activation row l16, weights of row l16
+        auto hfrag = [&](int n, int kg, int h) __attribute__((always_inline)) {
+            return *reinterpret_cast<const f16x8_t *>(L.h + lds_at<HS>(n * 16 + l16, 8 * kg + 2 * g + h));
+        };
+        auto add = [&](int n, int kg, f32x4_t d) __attribute__((always_inline)) {
+            const float s = L.isc[n * 16 + l16][kg];
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[rt][n][i] = fmaf(d[i], s, acc[rt][n][i]);
-            };
-            const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (!F4) {
+            for (int i = 0; i < 4; i++) acc[rt][n][i] = fmaf(d[i], s, acc[rt][n][i]);
+        };
+        const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (!F4) {
+#pragma unroll 2
+            for (int kg = 0; kg < NG; kg++) {
                 f16x8_t w0, w1;
                 i8_to_f16(*reinterpret_cast<const u32x4_t *>(lw + lds_at<ROWB>(l16, 4 * kg + g)), w0, w1);
 #pragma unroll
                 for (int n = 0; n < NT; n++) {
                     if (NT > 1 && n * 16 >= rows) continue;
-                    add(n, mfma_f16(w1, hfrag(n, 1), mfma_f16(w0, hfrag(n, 0), z)));
+                    add(n, kg, mfma_f16(w1, hfrag(n, kg, 1), mfma_f16(w0, hfrag(n, kg, 0), z)));
                 }
-            } else {
-                const u32x2_t w = *reinterpret_cast<const u32x2_t *>(lw + lds_at<ROWB>(l16, 2 * kg + (g >> 1)) + (g & 1) * 8);
-                const uint32_t b = lw[16 * ROWB + l16 * SB + 4 * kg + g];
-                if (__builtin_amdgcn_ballot_w64(b >= 0x7Fu) == 0) {
-                    const f32x2_t f = __builtin_amdgcn_cvt_pk_f32_fp8(b, false);
+            }
+        } else {
+            auto wfrag = [&](int kg) __attribute__((always_inline)) {
+                return *reinterpret_cast<const u32x2_t *>(lw + lds_at<ROWB>(l16, 2 * kg + (g >> 1)) + (g & 1) * 8);
+            };
+            if (hw) {
+#pragma unroll
+                for (int kg = 0; kg < NG; kg++) {
+                    const u32x2_t w = wfrag(kg);
+                    const f32x2_t f = __builtin_amdgcn_cvt_pk_f32_fp8(lw[16 * ROWB + l16 * SB + 4 * kg + g], false);
                     const f16x2_t s = {(_Float16)f.x, (_Float16)f.x};
                     const f16x8_t w0 = f4_to_f16(w[0], s), w1 = f4_to_f16(w[1], s);
 #pragma unroll
                     for (int n = 0; n < NT; n++) {
                         if (NT > 1 && n * 16 >= rows) continue;
-                        add(n, mfma_f16(w1, hfrag(n, 1), mfma_f16(w0, hfrag(n, 0), z)));
+                        add(n, kg, mfma_f16(w1, hfrag(n, kg, 1), mfma_f16(w0, hfrag(n, kg, 0), z)));
                     }
-                } else {
-                    const float s = e4m3_scale(b);
+                }
+            } else {
+#pragma unroll 1
+                for (int kg = 0; kg < NG; kg++) {
+                    const u32x2_t w = wfrag(kg);
+                    const float s = e4m3_scale(lw[16 * ROWB + l16 * SB + 4 * kg + g]);
                     const bf16x8_t w0 = f4_to_bf16x8(w[0], s), w1 = f4_to_bf16x8(w[1], s);
 #pragma unroll
                     for (int n = 0; n < NT; n++) {
                         if (NT > 1 && n * 16 >= rows) continue;
-                        add(n, mfma_bf16(w1, f16_to_bf16x8(hfrag(n, 1)), mfma_bf16(w0, f16_to_bf16x8(hfrag(n, 0)), z)));
+                        add(n, kg, mfma_bf16(w1, f16_to_bf16x8(hfrag(n, kg, 1)),
+                                             mfma_bf16(w0, f16_to_bf16x8(hfrag(n, kg, 0)), z)));
                     }
                 }
             }

@@ -315,8 +315,11 @@ __device__ __forceinline__ void mid_gu_body(const uint8_t *__restrict__ wg, cons
             *reinterpret_cast<u32x4_t *>(lw + lds_at<CB>(j * RPI + lr, lc)) = buf[b][j];
             *reinterpret_cast<u32x4_t *>(lw + 16 * CB + lds_at<CB>(j * RPI + lr, lc)) = buf[b][NI + j];
         }
-        if constexpr (F4)
+        bool hw = true;                           // every block scale of the chunk below 0x7F
+        if constexpr (F4) {
             if (lane < 32) *reinterpret_cast<scv_t *>(lw + 32 * CB + lane * SB) = sc[b];
+            hw = __builtin_amdgcn_ballot_w64(lane < 32 && !f4_scales_hw(sc[b])) == 0;
+        }
         uint8_t *lx = L.x[b];
 #pragma unroll
         for (int j = 0; j < NX; j++)
@@ -344,38 +347,47 @@ __device__ __forceinline__ void mid_gu_body(const uint8_t *__restrict__ wg, cons
                 }
             }
         } else {
+            auto codes = [&](int m, int q) __attribute__((always_inline)) {
+                return *reinterpret_cast<const u32x4_t *>(lw + m * 16 * CB + lds_at<CB>(l16, 4 * q + g));
+            };
+            auto scales = [&](int m, int q) __attribute__((always_inline)) {
+                return (uint32_t)*reinterpret_cast<const uint16_t *>(lw + 32 * CB + (m * 16 + l16) * SB + 8 * q + 2 * g);
+            };
+            if (hw) {
 #pragma unroll
-            for (int q = 0; q < KC / 128; q++) {
-                const u32x4_t cg = *reinterpret_cast<const u32x4_t *>(lw + lds_at<CB>(l16, 4 * q + g));
-                const u32x4_t cu = *reinterpret_cast<const u32x4_t *>(lw + 16 * CB + lds_at<CB>(l16, 4 * q + g));
-                const uint32_t pg = *reinterpret_cast<const uint16_t *>(lw + 32 * CB + l16 * SB + 8 * q + 2 * g);
-                const uint32_t pu = *reinterpret_cast<const uint16_t *>(lw + 32 * CB + 16 * SB + l16 * SB + 8 * q + 2 * g);
-                if (__builtin_amdgcn_ballot_w64(!(e4m3_pair_hw_ok(pg) && e4m3_pair_hw_ok(pu))) == 0) {
-                    const f32x2_t fg = __builtin_amdgcn_cvt_pk_f32_fp8(pg, false), fu = __builtin_amdgcn_cvt_pk_f32_fp8(pu, false);
+                for (int q = 0; q < KC / 128; q++) {
+                    const u32x4_t cg = codes(0, q), cu = codes(1, q);
+                    const f32x2_t fg = __builtin_amdgcn_cvt_pk_f32_fp8(scales(0, q), false);
+                    const f32x2_t fu = __builtin_amdgcn_cvt_pk_f32_fp8(scales(1, q), false);
                     const f16x2_t hg[2] = {{(_Float16)fg.x, (_Float16)fg.x}, {(_Float16)fg.y, (_Float16)fg.y}};
                     const f16x2_t hu[2] = {{(_Float16)fu.x, (_Float16)fu.x}, {(_Float16)fu.y, (_Float16)fu.y}};
 #pragma unroll
                     for (int m = 0; m < 4; m++) {
-                        const f16x8_t a = f4_to_f16(cg[m], hg[m >> 1]), b = f4_to_f16(cu[m], hu[m >> 1]);
+                        const f16x8_t a = f4_to_f16(cg[m], hg[m >> 1]), b2 = f4_to_f16(cu[m], hu[m >> 1]);
 #pragma unroll
                         for (int n = 0; n < NT; n++) {
                             if (NT > 1 && n * 16 >= rows) continue;
                             const f16x8_t xf = xfrag(n, 16 * q + 4 * g + m);
                             ag[n] = mfma_f16(a, xf, ag[n]);
-                            au[n] = mfma_f16(b, xf, au[n]);
+                            au[n] = mfma_f16(b2, xf, au[n]);
                         }
                     }
-                } else {                          // a block scale outside the fp16 range: bf16, as the prefill path
+                }
+            } else {                              // a block scale outside the fp16 range: bf16, as the prefill path
+#pragma unroll 1
+                for (int q = 0; q < KC / 128; q++) {
+                    const u32x4_t cg = codes(0, q), cu = codes(1, q);
+                    const uint32_t pg = scales(0, q), pu = scales(1, q);
 #pragma unroll
                     for (int m = 0; m < 4; m++) {
                         const bf16x8_t a = f4_to_bf16x8(cg[m], e4m3_scale(m < 2 ? pg & 0xFFu : pg >> 8));
-                        const bf16x8_t b = f4_to_bf16x8(cu[m], e4m3_scale(m < 2 ? pu & 0xFFu : pu >> 8));
+                        const bf16x8_t b2 = f4_to_bf16x8(cu[m], e4m3_scale(m < 2 ? pu & 0xFFu : pu >> 8));
 #pragma unroll
                         for (int n = 0; n < NT; n++) {
                             if (NT > 1 && n * 16 >= rows) continue;
                             const bf16x8_t xf = f16_to_bf16x8(xfrag(n, 16 * q + 4 * g + m));
                             ag[n] = mfma_bf16(a, xf, ag[n]);
-                            au[n] = mfma_bf16(b, xf, au[n]);
+                            au[n] = mfma_bf16(b2, xf, au[n]);
                         }
                         asm volatile("" ::: "memory");
                     }
