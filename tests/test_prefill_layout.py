@@ -146,6 +146,36 @@ def test_plan_fits_the_bounds(shim, H, I, gu, dn):
                         assert 0 < rows <= BM and row0 + rows <= groups[g] and 0 <= n < nt
 
 
+@pytest.mark.parametrize("H,I,f4,top", [(2048, 512, 0, 2800), (2048, 512, 1, 2800), (2560, 640, 0, 1800),
+                                        (2560, 640, 1, 2500)])
+def test_middle_rows_fit_the_regions(shim, H, I, f4, top):
+    """Calls of 9 to `top` rows (mid_rows_max) keep their own contents in the
+    same regions: one item list whose bound (one item per distinct expert, one
+    more per full mt rows, the shared expert's) launch_mid refuses to exceed,
+    8-byte pairs over the token and slot regions, an int8 exponent per 64 hidden
+    values in the row-sum region, and beyond 600 rows the K slices of the router
+    logits in the partials' region (room for four but
+    at top_k 1 without a shared expert)."""
+    E = 512
+    for K in (1, 2, 9, 10, 16):
+        for has_sh in (True, False):
+            for T in [9, 10, 31, 32, 33, 127, 128, 129, 600, 601, 819, 820, 1229, 1230, 2047, 2048, top - 1, top]:
+                if T > top:
+                    continue
+                off, by, m = layout(shim, T, H, I, E, K, has_sh, GU_F4 if f4 else GU_I8, GU_F4 if f4 else DN_I8)
+                r = dict(zip(NAMES, zip(off, by)))
+                P = T * (K + has_sh)
+                mt = 16 if T * K // E < 24 or f4 or I > 512 else 64
+                items = min(E, T * K) + T * K // mt + (-(-T // mt) if has_sh else 0)
+                assert items * 16 <= r["items_gu"][1], (K, has_sh, T)
+                assert r["p_tok"][0] + 8 * P <= r["p_slot"][0] + r["p_slot"][1] and r["p_tok"][0] % 8 == 0
+                assert P * (I // 64) <= r["hsum"][1]
+                room = r["part"][1] // (T * E * 4)
+                slices = 4 if T <= 2048 and room >= 4 else 2 if T <= 4096 and room >= 2 else 1
+                assert slices == 1 or slices * T * E * 4 <= r["part"][1]
+                assert room >= (4 if K + has_sh > 1 else 2)
+
+
 def test_library_sizes_match_the_layout(shim):
     """qfm_workspace_bytes (M > 8) = the workspace's tag header (256 bytes of row
     tags, 8 rows x E 8-byte logit words and 8 rows x (K + 1) slots x H 8-byte
