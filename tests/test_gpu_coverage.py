@@ -155,6 +155,46 @@ def test_prefill_tile_boundaries(lib, T, fmt):
     st.destroy()
 
 
+# ------------------------------------------------------------------ NVFP4, one row
+@pytest.mark.parametrize("hidden,inter,k,shared,gated,f32", [
+    (2048, 512, 1, True, 1, False), (2048, 512, 4, False, 1, True), (2048, 512, 5, True, 0, True),
+    (2048, 512, 16, True, 1, False), (2560, 640, 3, True, 1, True), (2560, 640, 4, False, 1, False),
+    (2560, 640, 13, True, 0, False), (2560, 640, 16, True, 1, True)])
+def test_nvfp4_one_row_steps(lib, hidden, inter, k, shared, gated, f32):
+    """One NVFP4 row: the down launch deals the k experts' I / 32 chunks to 64
+    lanes in 1 to 5 steps (k around whole steps: 4 x 16 chunks fill one exactly,
+    3 and 4 x 20 lie either side of it, 16 x 20 fill five), with the shared expert
+    gated, ungated and absent, into bf16 and fp32 rows. Routing bit-exact; y within TOL of the fp64 oracle (hidden values
+    and x enter the dots as scaled fp16, 2^-12 each; bf16 result 2^-9)."""
+    _say("nvfp4 one row H", hidden, "K", k, "shared", shared, "gated", gated, "f32", f32)
+    qfm.init(hidden, inter, E, k, 1, gated)
+    st = qfm.Stream()
+    seed, layer, xl = 9, 5, 70
+    L = qfm.SynthLayer(qfm.QFM_FMT_NVFP4, seed, layer, stream=st)
+    lay = qfm.QfmLayer.from_buffer_copy(L.s.layer)
+    if not shared:
+        lay.sh_gate, lay.sh_up, lay.sh_down, lay.sh_gate_inp = qfm.Qf8I8Mat(), qfm.Qf8I8Mat(), qfm.Qf8I8Mat(), None
+    x = orc.fill("gauss_bf16", seed, xl, orc.T_X, 0, hidden).reshape(1, hidden)
+    dx, dy = qfm.DevBuf.from_array(x), qfm.DevBuf(hidden * 4)
+    wsb = lib.qfm_workspace_bytes(1)
+    ws = qfm.DevBuf(wsb)
+    fwd = lib.qfm_moe_forward_f32 if f32 else lib.qfm_moe_forward
+    for _ in range(2):                                   # the second call on a used workspace
+        qfm.check(fwd(C.byref(lay), dx.ptr, 1, dy.ptr, ws.ptr, wsb, st.h), "forward")
+    st.sync()
+    view = qfm.QfmWsView()
+    lib.qfm_workspace_view(ws.ptr, 1, C.byref(view))
+    y = dy.download(np.float32, (hidden,)) if f32 else orc.bf16_to_f32(dy.download(np.uint16, (hidden,)))
+    zero = None if shared else (np.zeros((inter, hidden)), np.zeros((inter, hidden)), np.zeros((hidden, inter)))
+    r = orc.moe_layer_grouped(hidden, inter, E, k, 1, seed, layer, xl, x=x, fmt=1, gated=gated, shared=zero)
+    assert np.array_equal(qfm.d2h(view.sel, np.int32, (1, k)), r["sel"])
+    assert np.allclose(qfm.d2h(view.wts, np.float32, (1, k)), r["w"], rtol=2e-6, atol=1e-7)
+    assert _rel(y, r["y"][0]) <= TOL
+    L.destroy()
+    st.destroy()
+    qfm.init(H, I, E, K, 1, 1)
+
+
 # ------------------------------------------------------------------ middle row counts
 @pytest.mark.parametrize("hidden,inter,T,fmt,hot", [
     (2048, 512, 9, 1, 0), (2048, 512, 16, 0, 16), (2048, 512, 33, 1, 17), (2560, 640, 31, 0, 33), (2560, 640, 17, 1, 1),
