@@ -1,4 +1,4 @@
-// qfm_csr.hip -- multi-row decode (M <= 8 "Ocho" fork rows): weight-once-per-
+// qfm_csr.hip -- multi-row decode (2 to 8 "Ocho" fork rows): weight-once-per-
 // distinct-expert gate/up and down keyed by pair, INT8 and NVFP4 arenas.
 //
 // Reference behaviour: the M=8 CSR tier k_m8_build_csr / k_m8_gateup /
@@ -565,8 +565,8 @@ int launch_csr_forward(const Qf4ExpCache *a, int fmt, const ShPtrs *sh, const ui
                        int4 *pdsc, void *xh16, unsigned long long *pw, uint32_t *ctl, uint16_t *y, float *y32,
                        hipStream_t s) {
     const int K = g_cfg.K, E = g_cfg.E, P = M * K;
-    if (M < 1 || M > kMaxRows || P > kMaxPairs || E != 512) {
-        set_error(-2, "csr path: needs 1 <= M <= %d, M*top_k <= %d, 512 experts", kMaxRows, kMaxPairs); return -2;
+    if (M < 2 || M > kMaxRows || P > kMaxPairs || E != 512) {
+        set_error(-2, "csr path: needs 2 <= M <= %d, M*top_k <= %d, 512 experts", kMaxRows, kMaxPairs); return -2;
     }
     if (!pdsc || !pw || !ctl || K > 16) {
         set_error(-1, "csr path: needs the pair descriptors, partial words and tags, top_k <= 16"); return -1;

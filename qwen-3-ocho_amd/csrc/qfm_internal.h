@@ -41,7 +41,7 @@ struct ShPtrs { const int8_t *qg, *qu, *qd; const float *sg, *su, *sd; };
 // and, when sh != nullptr, the shared-expert hidden hsh[m * ld_hsh + r], in one launch.
 // With x16 != nullptr (M = 1) the launch also writes x as scaled fp16 (H / 8
 // 16-byte words) followed by a float2 (sum of the scaled values, 2^-k).
-// With tail != nullptr (1 <= M <= kTailRows, E = 512, no x16) the launch also
+// With tail != nullptr (2 <= M <= kTailRows, E = 512, no x16) the launch also
 // ranks every row (k_router_shared's selection tail): sel/wts [M][K], and for
 // INT8 fork rows x as scaled fp16 chunks (xh [M][H] fp16, xci [M][H/16]).
 // lw: [M][E] 64-bit words; ctl: kTailRows + 1 words (per-row tags, then the
@@ -92,7 +92,7 @@ int launch_i8_down_m1(const Qf4ExpCache *c, const float *hidden, const float *wt
 int launch_f4_m1(const Qf4ExpCache *a, const ShPtrs *sh, const uint16_t *x, const float *logits, const float *gdot,
                  int *sel, float *wts, float *hidden, uint32_t *ctl, float *y32, uint16_t *ybf, hipStream_t s);
 
-// Multi-row decode (1 <= M <= 8), after launch_router_shared with its selection
+// Multi-row decode (2 <= M <= 8), after launch_router_shared with its selection
 // tail (sel/wts [M][K], INT8: the fp16 activation chunks in xh16): gate/up
 // keyed by pair (k_csr_gateup: the first pair of each distinct expert reads
 // the expert's rows once for all its pairs; hidden row = pair id), down

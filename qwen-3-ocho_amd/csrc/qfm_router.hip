@@ -50,7 +50,7 @@ __device__ __forceinline__ float canon_reduce_row(const float4 (&w)[NJ], const f
 // With x16 != nullptr one more block (the first) writes x row 0 as scaled
 // fp16 with its (sum, 2^-k) for the M = 1 gate/up kernel.
 //
-// With TAIL (the M <= 8 forward; tail.lw != nullptr) the launch also selects: each
+// With TAIL (the forward of 2 to 8 rows; tail.lw != nullptr) the launch also selects: each
 // router row's logits go out a second time as 64-bit words (fp32 bits | tag <<
 // 32, stored at agent scope), tag = next_tag(ctl[m]) for row m; the grid's last
 // blocks are then (INT8) x as scaled fp16 chunks (chunk16_to_f16, the fork
@@ -69,6 +69,7 @@ k_router_shared(const float *__restrict__ W, const float *__restrict__ bias, con
                 ShPtrs sh, const uint16_t *__restrict__ x, int M, int E, float *__restrict__ logits, int ld,
                 float *__restrict__ hsh, int ldh, uint4 *__restrict__ x16, float2 *__restrict__ x16i,
                 RouteTail tail, int tail0) {
+    static_assert(!TAIL || MR > 1, "one row is selected by the gate/up launch");
     constexpr int H = NJ * 256;
     const int lane = threadIdx.x;
     args_now(W, bias, g, sh.qg, sh.qu, sh.sg, sh.su, x, M, E, logits, ld, hsh, ldh, x16, x16i);
@@ -171,10 +172,7 @@ k_router_shared(const float *__restrict__ W, const float *__restrict__ bias, con
             if constexpr (MR == 1) {
                 float v = canon_butterfly(a[0]);
                 if (bias && !is_g) v = __fadd_rn(v, bb);
-                if (lane == 0 && m0 < M) {
-                    logits[(size_t)m0 * ld + b] = v;
-                    if (TAIL && !is_g) st_agent_u64(tail.lw + (size_t)m0 * E + b, __float_as_uint(v) | ((unsigned long long)tgl << 32));
-                }
+                if (lane == 0 && m0 < M) logits[(size_t)m0 * ld + b] = v;
             } else {
                 // lane r < MR ends with row m0 + r (the same addition tree per row)
                 float v = canon_reduce_rows<MR>(a, lane);
@@ -297,6 +295,12 @@ int launch_router_shared(const float *W, const float *bias, const float *g, cons
         tl = *tail;
         nblk += (tl.xh ? (M * (g_cfg.H / 16) + 63) / 64 : 0) + M;
     }
+    if (M == 1 && tail && (shape_2048() || shape_2560())) {
+        set_error(-1, "router: one row takes no selection tail"); return -1;
+    }
+#define QFM_ROUTER1(NJ, II)                                                                                    \
+    hipLaunchKernelGGL((k_router_shared<NJ, II, 1, false>), dim3(nblk), dim3(64), 0, s, W, bias, g, sp, x, M, E,   \
+                       logits, ld, hsh, ldh, xh, xi, tl, tail0)
 #define QFM_ROUTER(NJ, II, MR)                                                                                 \
     if (tail)                                                                                                  \
         hipLaunchKernelGGL((k_router_shared<NJ, II, MR, true>), dim3(nblk), dim3(64), 0, s, W, bias, g, sp, x, M, E, \
@@ -305,19 +309,19 @@ int launch_router_shared(const float *W, const float *bias, const float *g, cons
         hipLaunchKernelGGL((k_router_shared<NJ, II, MR, false>), dim3(nblk), dim3(64), 0, s, W, bias, g, sp, x, M, E, \
                            logits, ld, hsh, ldh, xh, xi, tl, tail0)
     if (shape_2048()) {
-        if (M == 1) { QFM_ROUTER(8, 512, 1); }
+        if (M == 1) { QFM_ROUTER1(8, 512); }
         else if (M <= 4) { QFM_ROUTER(8, 512, 4); }
         else { QFM_ROUTER(8, 512, 8); }
     } else if (shape_shard() && M == 1 && !sh && !tail) {
-        hipLaunchKernelGGL((k_router_shared<8, 64, 1, false>), dim3(nblk), dim3(64), 0, s, W, bias, g, sp, x, M, E,
-                           logits, ld, hsh, ldh, xh, xi, tl, tail0);
+        QFM_ROUTER1(8, 64);
     } else if (shape_2560()) {
-        if (M == 1) { QFM_ROUTER(10, 640, 1); }
+        if (M == 1) { QFM_ROUTER1(10, 640); }
         else { QFM_ROUTER(10, 640, 4); }
     } else {
         set_error(-2, "router: unsupported shape"); return -2;
     }
 #undef QFM_ROUTER
+#undef QFM_ROUTER1
     return check_launch("router_shared");
 }
 
