@@ -436,8 +436,6 @@ using RouterEngine = TileEngine<kB_BF16, 2, 2, 4, 2>;
 // router GEMM slices along H the workspace counts for its logits region; more
 // slices borrow another region (launch_prefill)
 constexpr int kRouterKS = 1;
-// up to here four waves select a token's experts, beyond it one (k_pf_select)
-constexpr int kSelectSplitRows = 1100;
 // INT8 tiles: 128 x 256 in 8 waves of 64 x 64 (two waves per SIMD). Four
 // waves of 128 x 64 (MW = 8: one wave per SIMD, accumulators in AGPRs, 25%
 // fewer LDS reads per MFMA) measured 1343 / 1149 us against 797 / 719 us.
@@ -568,7 +566,8 @@ __device__ __forceinline__ float bound_coeff(int H) {
 
 // Candidates, exact logits, exact top-K and the shared gate, WPT waves per
 // token. lg_part: the router GEMM's nks partial logits [nks][T][E], summed in
-// slice order; their sum goes to lg. Every wave of a token forms the bounds and
+// slice order; their sum goes to lg, which may be lg_part itself where nks and
+// WPT are 1 (pf_select_split): neither is __restrict__. Every wave of a token forms the bounds and
 // the candidate list itself (no barrier) and recomputes every WPT-th candidate;
 // the first wave ranks them. tau, a lower bound of the K-th largest logit, is
 // the K-th largest of the 64 lane maxima of the lower bounds (K distinct
@@ -580,9 +579,9 @@ __device__ __forceinline__ float bound_coeff(int H) {
 template <int NJ, int WPT>
 __global__ void __launch_bounds__(256)
 k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, const float *__restrict__ bias,
-            const float *__restrict__ g, const float *__restrict__ lg_part, int nks, float *__restrict__ lg,
-            const float *__restrict__ xnorm, const float *__restrict__ wnorm, int K, int renorm,
-            int *__restrict__ sel, float *__restrict__ wts, float *__restrict__ gam, int *__restrict__ n_fallback) {
+            const float *__restrict__ g, const float *lg_part, int nks, float *lg, const float *__restrict__ xnorm,
+            const float *__restrict__ wnorm, int K, int renorm, int *__restrict__ sel, float *__restrict__ wts,
+            float *__restrict__ gam, int *__restrict__ n_fallback) {
     constexpr int H = NJ * 256, EPL = 8, E = EPL * 64, TPB = 4 / WPT;
     __shared__ __align__(16) uint32_t s_lm[4][64];
     __shared__ int s_cand[4][kCandMax];
@@ -1198,11 +1197,8 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
         launch_fill_f32(reinterpret_cast<float *>(ctr), 8, 0.0f, s);
         hipLaunchKernelGGL(k_pf_router_prep, dim3((unsigned)(E + (T + 3) / 4)), dim3(256), 0, s, L->router, E, H, wnorm,
                            wb16, x, T, xnorm, xsum, mid || !f4 ? x16 : nullptr, x16sum, x16isc);
-        // few m-tiles: K in slices until the chip is full (their partial logits lie
-        // in the region of the partials, which the down GEMM writes later; that
-        // has room for two at top_k 1 without a shared expert): 1021 rows 31 -> 13 us
-        const size_t room = Lw.bytes[kPfPart] / ((size_t)T * E * sizeof(float));
-        const int nks = T <= 2048 && room >= 4 ? 4 : T <= 4096 && room >= 2 ? 2 : 1;
+        const int nks = pf_router_slices(T, E, Lw.bytes[kPfPart]);
+        const bool split = pf_select_split(T, nks);
         float *lgp = nks > 1 ? reinterpret_cast<float *>(part) : lg;
         const int mt_router = ((T + BM - 1) / BM + 7) / 8 * 8;
         hipLaunchKernelGGL(k_pf_router_mfma, dim3(mt_router * (E / BN), nks), dim3(256), 0, s, x, T, H, wb16, E, lgp);
@@ -1210,9 +1206,9 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
     hipLaunchKernelGGL((k_pf_select<NJ, WPT>), dim3((unsigned)((T * WPT + 3) / 4)), dim3(256), 0, s, x, T,          \
                        L->router, L->router_bias, g, lgp, nks, lg, xnorm, wnorm, K, c.renorm, sel, wts, gam, ctr)
         if (H == 2048) {
-            if (T <= kSelectSplitRows) { QFM_PF_SELECT(8, 4); } else { QFM_PF_SELECT(8, 1); }
+            if (split) { QFM_PF_SELECT(8, 4); } else { QFM_PF_SELECT(8, 1); }
         } else {
-            if (T <= kSelectSplitRows) { QFM_PF_SELECT(10, 4); } else { QFM_PF_SELECT(10, 1); }
+            if (split) { QFM_PF_SELECT(10, 4); } else { QFM_PF_SELECT(10, 1); }
         }
 #undef QFM_PF_SELECT
     }

@@ -78,4 +78,20 @@ inline PfLayout pf_layout(int T, int H, int I, int E, int K, bool has_sh, int gu
     return L;
 }
 
+// Slices of H in the router GEMM. Few m-tiles do not fill the chip, so K is cut
+// (1021 rows: 31 -> 13 us in four). One slice writes the logits' own region;
+// more lie in the partials' region (part_bytes), which the down GEMM writes
+// later and which has room for four, at top_k 1 without a shared expert for two.
+inline int pf_router_slices(int T, int E, size_t part_bytes) {
+    const size_t room = part_bytes / ((size_t)T * E * 4);
+    return T <= 2048 && room >= 4 ? 4 : T <= 4096 && room >= 2 ? 2 : 1;
+}
+
+// Four waves a token in k_pf_select, else one: up to kSelectSplitRows rows (the
+// figures are there), and only where its input and output logits are two
+// buffers: with one slice they are the same, and a wave would read logits that
+// another wave of its token has already stored with the bias added.
+constexpr int kSelectSplitRows = 1100;
+inline bool pf_select_split(int T, int slices) { return T <= kSelectSplitRows && slices > 1; }
+
 }  // namespace qfm

@@ -14,3 +14,8 @@ extern "C" int pf_layout_c(int T, int H, int I, int E, int K, int has_sh, int gu
     meta[3] = (unsigned long long)L.nt_gu; meta[4] = (unsigned long long)L.nt_dn; meta[5] = (unsigned long long)L.nblk;
     return qfm::kPfCount;
 }
+
+extern "C" int pf_router_slices_c(int T, int E, unsigned long long part_bytes) {
+    return qfm::pf_router_slices(T, E, part_bytes);
+}
+extern "C" int pf_select_split_c(int T, int slices) { return qfm::pf_select_split(T, slices); }

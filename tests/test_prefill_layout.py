@@ -176,6 +176,24 @@ def test_middle_rows_fit_the_regions(shim, H, I, f4, top):
                 assert room >= (4 if K + has_sh > 1 else 2)
 
 
+@pytest.mark.parametrize("H,I,f4", [(2048, 512, 0), (2048, 512, 1), (2560, 640, 0), (2560, 640, 1)])
+def test_selection_waves_never_share_a_logits_buffer(shim, H, I, f4):
+    """k_pf_select reads the router GEMM's slices and stores their sum plus the
+    bias. One slice lies in the output's own region, where a second wave of the
+    same token would race with the first one's stores: four waves a token only
+    over two or more slices, and those fit the region that they borrow."""
+    E = 512
+    assert not any(shim.pf_select_split_c(T, 1) for T in range(9, 2000))
+    for K in (1, 2, 9, 10, 16):
+        for has_sh in (True, False):
+            for T in [9, 600, 601, 1023, 1024, 1025, 1100, 1101, 2047, 2048, 2049, 4095, 4096, 4097, 16384]:
+                off, by, m = layout(shim, T, H, I, E, K, has_sh, GU_F4 if f4 else GU_I8, GU_F4 if f4 else DN_I8)
+                part, lg = by[NAMES.index("part")], by[NAMES.index("lg")]
+                n = shim.pf_router_slices_c(T, E, C.c_ulonglong(int(part)))
+                assert n in (1, 2, 4) and n * T * E * 4 <= (part if n > 1 else lg)
+                assert not shim.pf_select_split_c(T, n) or n > 1
+
+
 def test_library_sizes_match_the_layout(shim):
     """qfm_workspace_bytes (M > 8) = the workspace's tag header (256 bytes of row
     tags, 8 rows x E 8-byte logit words and 8 rows x (K + 1) slots x H 8-byte
