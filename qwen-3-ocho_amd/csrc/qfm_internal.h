@@ -155,7 +155,7 @@ struct MidArgs {
     int *ctr;                           // {selection overflows, items, ...}
     int2 *pairs;                        // [T (K + shared)] {partial slot, weight}
     int4 *items;
-    int max_items;                      // entries of items
+    int max_items;                      // entries of items; mid_items_bound checked against it by the caller
     uint16_t *hid;                      // [pairs][I] fp16
     int8_t *hk;                         // [pairs][I / 64]
     uint16_t *part;                     // [T (K + shared)][H] fp16

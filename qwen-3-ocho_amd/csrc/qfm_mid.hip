@@ -32,6 +32,7 @@
 #include "qfm_dev.h"
 #include "qfm_internal.h"
 #include "qfm_mfma.h"
+#include "qfm_prefill_layout.h"
 
 namespace qfm {
 
@@ -191,7 +192,8 @@ k_mid_topk(const float *__restrict__ logits, int T, int K, int renorm, int *__re
 constexpr int kPlanBatch = 16;
 __global__ void __launch_bounds__(1024)
 k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const float *__restrict__ gam, int T, int K,
-           int E, int has_sh, int mt, int2 *__restrict__ pairs, int4 *__restrict__ items, int *__restrict__ n_items) {
+           int E, int has_sh, int mt, int2 *__restrict__ pairs, int4 *__restrict__ items, int max_items,
+           int *__restrict__ n_items) {
     __shared__ int cnt[1024], sa[1024], sb[1024];
     const int g = threadIdx.x, S = K + has_sh, TK = T * K;
     cnt[g] = 0;
@@ -219,10 +221,13 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
     }
     const int off = sa[g] - c, shi = has_sh ? (T + mt - 1) / mt : 0;
     cnt[g] = off;                                              // the group's next free pair
+    auto item = [&](int i, int grp, int first, int rows) __attribute__((always_inline)) {
+        if (i < max_items) items[i] = make_int4(grp, first, rows, 0);   // (the host's bound lies below max_items)
+    };
     if (g < E)
-        for (int i = 0; i < mi; i++) items[shi + sb[g] - mi + i] = make_int4(g, off + i * mt, min(mt, c - i * mt), 0);
-    for (int i = g; i < shi; i += 1024) items[i] = make_int4(E, TK + i * mt, min(mt, T - i * mt), 0);
-    if (g == E - 1) n_items[0] = shi + sb[g];
+        for (int i = 0; i < mi; i++) item(shi + sb[g] - mi + i, g, off + i * mt, min(mt, c - i * mt));
+    for (int i = g; i < shi; i += 1024) item(i, E, TK + i * mt, min(mt, T - i * mt));
+    if (g == E - 1) n_items[0] = min(shi + sb[g], max_items);
     __syncthreads();
     const bool one = TK <= 1024 * kPlanBatch;                  // v still holds every id
     for (int p0 = g; p0 < TK; p0 += 1024 * kPlanBatch) {
@@ -565,6 +570,7 @@ k_mid_down(const int4 *__restrict__ items, const int *__restrict__ n_items, cons
 int launch_mid(const MidArgs &a, hipStream_t s) {
     const Cfg &c = g_cfg;
     const int T = a.T, E = c.E, K = c.K, H = c.H, I = c.I;
+    const int nt = mid_token_tiles(T, E, K, I, a.f4), mt = 16 * nt, max_items = mid_items_bound(T, E, K, a.has_sh, nt);
     if (T <= kMidExactRows) {                                  // (beyond: the caller has launched router and selection)
         const int ng = (T + 7) / 8, nx = E / 8 + (a.g ? 1 : 0);
         const int tg = max(1, ng * nx / 1536);                     // token groups per router block: ~1536 blocks
@@ -584,12 +590,8 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
     // 425 / 462; NVFP4 198 / 345 / 422 / 500, 278 / 386 / 462 / 580, 436 / 526 /
     // 599 / 688. Four are taken for INT8 from 24 rows an expert.
     const int avg = T * K / E;
-    const int nt = avg < 24 || a.f4 || I > 512 ? 1 : 4, mt = 16 * nt;
     hipLaunchKernelGGL(k_mid_plan, dim3(1), dim3(1024), 0, s, a.sel, a.wts, a.g ? a.gam : nullptr, T, K, E, a.has_sh, mt,
-                       a.pairs, a.items, a.ctr + 1);
-    // items: one per distinct expert, one more per full mt rows, the shared group's
-    const int max_items = min(E, T * K) + T * K / mt + (a.has_sh ? (T + mt - 1) / mt : 0);
-    if (max_items > a.max_items) { set_error(-2, "mid path: %d items, room for %d", max_items, a.max_items); return -2; }
+                       a.pairs, a.items, a.max_items, a.ctr + 1);
     const int dw = 64 * mid_dn_waves(I, nt);                      // columns, and threads, per down block
     // (xcd_unit wants eight times the largest range: a multiple of 8)
     const dim3 g_gu((unsigned)((max_items * (I / 64) + 7) / 8 * 8)), g_dn((unsigned)((max_items * (H / dw) + 7) / 8 * 8)), b(256), bd((unsigned)dw);

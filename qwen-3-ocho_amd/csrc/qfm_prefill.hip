@@ -1192,6 +1192,11 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
     // router and selection: exact logits of every expert up to kMidExactRows
     // rows (launch_mid), the bf16 MFMA GEMM with exact candidates beyond
     const bool mid = T <= mid_rows_max(I, f4);
+    const int room = (int)(Lw.bytes[kPfItemsGu] / sizeof(int4));
+    if (mid) {
+        const int need = mid_items_bound(T, E, K, has_sh, mid_token_tiles(T, E, K, I, f4));
+        if (need > room) { set_error(-2, "mid path: %d items, room for %d", need, room); return -2; }
+    }
     if (!mid || T > kMidExactRows) {
         // zero the small counters with a fill kernel (no memset node in captured graphs)
         launch_fill_f32(reinterpret_cast<float *>(ctr), 8, 0.0f, s);
@@ -1218,7 +1223,7 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
         // token and slot regions)
         static_assert(kPfSlot == kPfTok + 1, "the pairs span two adjacent regions");
         const MidArgs m{L->router, L->router_bias, g, x, T, has_sh ? 1 : 0, f4, lg, sel, wts, gam, x16, x16isc, ctr,
-                        reinterpret_cast<int2 *>(p_tok), items_gu, (int)(Lw.bytes[kPfItemsGu] / sizeof(int4)), hid,
+                        reinterpret_cast<int2 *>(p_tok), items_gu, room, hid,
                         reinterpret_cast<int8_t *>(hsum), part, partk, gg, gu, gd};
         if (const int rc = launch_mid(m, s)) return rc;
         hipLaunchKernelGGL(k_pf_combine_h, dim3((unsigned)(((size_t)T * H / 4 + 255) / 256)), dim3(256), 0, s, part,

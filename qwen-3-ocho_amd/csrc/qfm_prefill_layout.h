@@ -78,6 +78,17 @@ inline PfLayout pf_layout(int T, int H, int I, int E, int K, bool has_sh, int gu
     return L;
 }
 
+// The middle path's work items: an expert's rows, 16 mid_token_tiles at a time
+// (the figures are at launch_mid), and the most that T rows can make: one per
+// distinct expert, one more per full item, the shared expert's. The launcher
+// refuses a call whose bound exceeds the item region before it launches
+// anything, and the plan kernel stores none beyond the region.
+inline int mid_token_tiles(int T, int E, int K, int I, bool f4) { return T * K / E < 24 || f4 || I > 512 ? 1 : 4; }
+inline int mid_items_bound(int T, int E, int K, bool has_sh, int token_tiles) {
+    const int mt = 16 * token_tiles, tk = T * K;
+    return (E < tk ? E : tk) + tk / mt + (has_sh ? (T + mt - 1) / mt : 0);
+}
+
 // Slices of H in the router GEMM. Few m-tiles do not fill the chip, so K is cut
 // (1021 rows: 31 -> 13 us in four). One slice writes the logits' own region;
 // more lie in the partials' region (part_bytes), which the down GEMM writes

@@ -176,6 +176,39 @@ def test_middle_rows_fit_the_regions(shim, H, I, f4, top):
                 assert room >= (4 if K + has_sh > 1 else 2)
 
 
+@pytest.mark.parametrize("H,I,f4,top", [(2048, 512, 0, 2800), (2048, 512, 1, 2800), (2560, 640, 0, 1800),
+                                        (2560, 640, 1, 2500)])
+def test_middle_items_never_exceed_their_bound(shim, H, I, f4, top):
+    """The item bound that the launcher checks before its first launch holds for
+    every routing (uniform, skewed, all rows on one expert, one row more than
+    whole items on as many experts as possible), and lies within the region that
+    the plan kernel is given as its limit."""
+    E = 512
+    rng = np.random.default_rng(6)
+    for K in (1, 10, 16):
+        for T in (9, 16, 17, 129, 600, 1229, top):
+            if T > top:
+                continue
+            for has_sh in (True, False):
+                by = layout(shim, T, H, I, E, K, has_sh, GU_F4 if f4 else GU_I8, GU_F4 if f4 else DN_I8)[1]
+                nt = shim.mid_token_tiles_c(T, E, K, I, f4)
+                bound = shim.mid_items_bound_c(T, E, K, int(has_sh), nt)
+                assert bound <= by[NAMES.index("items_gu")] // 16
+                mt = 16 * nt
+                routings = _routings(T, K, E, rng) if K > 1 else []
+                one = np.zeros(E, np.int64)
+                one[:K] = T
+                spread = np.zeros(E, np.int64)                 # a row over whole items wherever rows are left
+                left = T * K
+                for e in range(E):
+                    spread[e] = min(T, mt + 1 if left >= mt + 1 + (E - 1 - e) else 1, left)
+                    left -= spread[e]
+                spread[:K] += left // K
+                for cnt in routings + [one, spread]:
+                    items = int(((cnt + mt - 1) // mt).sum()) + (-(-T // mt) if has_sh else 0)
+                    assert items <= bound, (K, T, has_sh, items, bound)
+
+
 @pytest.mark.parametrize("H,I,f4", [(2048, 512, 0), (2048, 512, 1), (2560, 640, 0), (2560, 640, 1)])
 def test_selection_waves_never_share_a_logits_buffer(shim, H, I, f4):
     """k_pf_select reads the router GEMM's slices and stores their sum plus the
