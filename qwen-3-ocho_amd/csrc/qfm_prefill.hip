@@ -564,15 +564,56 @@ __device__ __forceinline__ float bound_coeff(int H) {
     return 2.0f * (0x1p-9f + (float)(2 * H) * 0x1p-24f + (float)(H / 64 + 8) * 0x1p-24f);
 }
 
+// The K-th largest of a wave's EPL x 64 keys, of which the n in the ballots rb
+// reach a lower bound of it. Up to 64 of them are ranked through lds (64 words
+// of wave-private LDS); more are searched bit by bit.
+template <int EPL>
+__device__ __forceinline__ uint32_t wave_kth_key(const uint32_t (&key)[EPL], const unsigned long long (&rb)[EPL], int n,
+                                                 int K, int lane, uint32_t *lds) {
+    if (n > 64) {
+        uint32_t v = 0u;
+        for (uint32_t bit = 1u << 31; bit; bit >>= 1) {
+            int c = 0;
+#pragma unroll
+            for (int i = 0; i < EPL; i++) c += __popcll(__ballot(key[i] >= (v | bit)));
+            if (c >= K) v |= bit;
+        }
+        return v;
+    }
+    int base = 0;
+#pragma unroll
+    for (int i = 0; i < EPL; i++) {
+        const int pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(rb[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)rb[i], (uint32_t)base));
+        if ((rb[i] >> lane) & 1ull) lds[pos] = key[i];
+        base += __popcll(rb[i]);
+    }
+    if (lane >= n) lds[lane] = 0u;                       // (higher lanes: never ahead of a key)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const uint32_t mine = lds[lane];
+    int rank = 0;
+    for (int q = 0; q < (n + 3) >> 2; q++) {
+        const uint4 p = reinterpret_cast<const uint4 *>(lds)[q];
+        const uint32_t d[4] = {p.x, p.y, p.z, p.w};
+#pragma unroll
+        for (int u = 0; u < 4; u++) rank += (d[u] > mine || (d[u] == mine && 4 * q + u < lane)) ? 1 : 0;
+    }
+    return (uint32_t)__builtin_amdgcn_readlane((int)mine, __builtin_ctzll(__ballot(lane < n && rank == K - 1)));
+}
+
 // Candidates, exact logits, exact top-K and the shared gate, WPT waves per
 // token. lg_part: the router GEMM's nks partial logits [nks][T][E], summed in
 // slice order; their sum goes to lg, which may be lg_part itself where nks and
 // WPT are 1 (pf_select_split): neither is __restrict__. Every wave of a token forms the bounds and
 // the candidate list itself (no barrier) and recomputes every WPT-th candidate;
 // the first wave ranks them. tau, a lower bound of the K-th largest logit, is
-// the K-th largest of the 64 lane maxima of the lower bounds (K distinct
-// experts reach it): one rank pass instead of K wave-wide maxima, for about one
-// candidate more. One wave per token is bound by its chain of L2 round trips
+// the K-th largest lower bound: first the K-th largest of the 64 lane maxima
+// (one rank pass instead of K wave-wide maxima; K distinct experts reach it),
+// then, where more than K experts reach that, the K-th largest among those.
+// The second pass matters where a router's hot experts agree modulo 64 (a lane
+// holds experts e, e + 64, ..): every candidate is a router row of 8 or 10 KiB,
+// and past 64 of them a token recomputes all 512 (32 hot experts in four lanes,
+// top-16: 2048/512 INT8 8038 rows 1909 -> 1386 us a call, 2560/640 NVFP4 4000
+// rows 1581 -> 1086; evenly spread experts the same with and without). One wave per token is bound by its chain of L2 round trips
 // while the tokens do not fill the chip: four waves take up to kSelectSplitRows
 // (450 / 1021 / 1500 rows 19 / 23 / 36 us; K wave-wide maxima and one wave a
 // token: 25 / 30 / 31 us; 8038 rows one wave 76 -> 68 us).
@@ -602,7 +643,7 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
             const float *p = lg_part + ((size_t)q * T + t) * E + i * 64 + lane;
             l[i] += WPT == 1 ? __builtin_nontemporal_load(p) : *p;
         }
-    uint32_t mx = 0u;                                    // the lane's largest lower bound (sortable bits)
+    uint32_t lk[EPL], mx = 0u;                           // lower bounds (sortable bits), the lane's largest
 #pragma unroll
     for (int i = 0; i < EPL; i++) {
         const int e = i * 64 + lane;
@@ -612,7 +653,8 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
         if (w == 0) __builtin_nontemporal_store(l[i], &lg[(size_t)t * E + e]);
         const float b = cB * wnorm[e] + 1e-6f * (fabsf(l[i]) + fabsf(be) + 1.0f);
         hi[i] = l[i] + b;
-        mx = max(mx, (uint32_t)(topk_key(l[i] - b, 0) >> 32));
+        lk[i] = (uint32_t)(topk_key(l[i] - b, 0) >> 32);
+        mx = max(mx, lk[i]);
     }
     s_lm[wave][lane] = mx;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -624,7 +666,15 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
 #pragma unroll
         for (int u = 0; u < 4; u++) rank += (d[u] > mx || (d[u] == mx && 4 * q + u < lane)) ? 1 : 0;
     }
-    const uint32_t tk = (uint32_t)__builtin_amdgcn_readlane((int)mx, __builtin_ctzll(__ballot(rank == K - 1)));
+    uint32_t tk = (uint32_t)__builtin_amdgcn_readlane((int)mx, __builtin_ctzll(__ballot(rank == K - 1)));
+    unsigned long long rb[EPL];
+    int nr = 0;                                          // experts whose lower bound reaches tk
+#pragma unroll
+    for (int i = 0; i < EPL; i++) {
+        rb[i] = __ballot(lk[i] >= tk);
+        nr += __popcll(rb[i]);
+    }
+    if (nr > K) tk = wave_kth_key<EPL>(lk, rb, nr, K, lane, s_lm[wave]);   // wave-uniform
     const float tau = topk_key_value((unsigned long long)tk << 32);
     // candidates: not below tau (a NaN bound makes every expert one)
     unsigned long long cb[EPL];

@@ -1,0 +1,88 @@
+"""GPU routing beyond the exact router's rows (601 and more): the bf16 MFMA
+router, its candidates and their exact recomputation (k_pf_router_mfma,
+k_pf_select), four waves a token and one, over the K slices of the router GEMM.
+
+Selection bit-exact and weights against the CPU oracle's router and top-K; the
+workspace counter says how many tokens had more than 64 candidates.
+"""
+import ctypes as C
+import sys
+
+import numpy as np
+import pytest
+
+import _oracle as orc
+import qfm
+
+pytestmark = pytest.mark.gpu
+
+E = 512
+SHAPES = {2048: 512, 2560: 640}
+
+
+def _say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def lib():
+    L = qfm.load()
+    assert qfm.device_info()["arch"].startswith("gfx950")
+    yield L
+    qfm.init(2048, 512, E, 10, 1, 1)
+
+
+def _route(lib, H, T, K, bias=None, renorm=1, x=None, router=None, fmt=qfm.QFM_FMT_NVFP4):
+    """qfm_moe_forward's routing of T rows and the oracle's: got, ref (sel, wts), counters."""
+    seed, layer = 12, 7
+    _say("routing H", H, "T", T, "K", K, "bias", bias is not None, "renorm", renorm)
+    qfm.init(H, SHAPES[H], E, K, renorm, 1)
+    st = qfm.Stream()
+    L = qfm.SynthLayer(fmt, seed, layer, stream=st)
+    st.sync()                            # generated on st; the router and bias are the test's own
+    W = orc.fill("gauss", seed, layer, orc.T_ROUTER, 0, E * H, 0.02).reshape(E, H) if router is None else router
+    if x is None:
+        x = orc.fill("gauss_bf16", seed, 40, orc.T_X, 0, T * H).reshape(T, H)
+    lay = qfm.QfmLayer.from_buffer_copy(L.s.layer)
+    dW, dx, dy = qfm.DevBuf.from_array(W), qfm.DevBuf.from_array(x), qfm.DevBuf(T * H * 2)
+    db = None if bias is None else qfm.DevBuf.from_array(np.ascontiguousarray(bias, np.float32))
+    lay.router, lay.router_bias = dW.ptr, db.ptr if db else None
+    wsb = lib.qfm_workspace_bytes(T)
+    ws = qfm.DevBuf(wsb)
+    qfm.check(lib.qfm_moe_forward(C.byref(lay), dx.ptr, T, dy.ptr, ws.ptr, wsb, st.h), "forward")
+    st.sync()
+    view = qfm.QfmWsView()
+    lib.qfm_workspace_view(ws.ptr, T, C.byref(view))
+    got = qfm.d2h(view.sel, np.int32, (T, K)), qfm.d2h(view.wts, np.float32, (T, K))
+    counters = qfm.d2h(view.counters, np.int32, 3)
+    sel, w, _ = orc.topk(orc.router_logits(W, x, bias), K, renorm)
+    for b in (dW, dx, dy, ws) + ((db,) if db else ()):
+        b.free()
+    L.destroy()
+    st.destroy()
+    _say("  tokens with more than 64 candidates", int(counters[0]))
+    return got, (sel, w), counters
+
+
+def _check(got, ref):
+    assert np.array_equal(got[0], ref[0])
+    assert np.allclose(got[1], ref[1], rtol=2e-6, atol=1e-7)
+
+
+# ------------------------------------------------------------------ candidates
+@pytest.mark.parametrize("H,T,K,per", [(2048, 601, 16, 4), (2048, 1200, 16, 4), (2560, 601, 16, 4), (2560, 1500, 10, 3),
+                                       (2048, 601, 16, 10), (2560, 1200, 16, 10)])
+def test_hot_experts_in_few_lanes(lib, H, T, K, per):
+    """A lane of the selecting wave holds the experts that agree modulo 64. A
+    bias of +6 on experts 64 j + {0 .. per - 1} puts the hot experts into `per`
+    lanes, fewer than top_k. The candidate bound must be the K-th largest lower
+    bound all the same, not a cold expert's as the K-th largest lane maximum is:
+    no token then has more than 64 candidates. With per = 10 more than 64
+    experts (80 hot ones) lie above that lane maximum."""
+    bias = np.zeros(E, np.float32)
+    for j in range(8):
+        bias[64 * j:64 * j + per] = 6.0
+    got, ref, counters = _route(lib, H, T, K, bias)
+    _check(got, ref)
+    assert counters[0] == 0
