@@ -651,8 +651,11 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
         if (bias) l[i] += be;
         // the logits and x are touched once per token: nontemporal, so the router rows of the candidates stay in L2
         if (w == 0) __builtin_nontemporal_store(l[i], &lg[(size_t)t * E + e]);
-        const float b = cB * wnorm[e] + 1e-6f * (fabsf(l[i]) + fabsf(be) + 1.0f);
-        hi[i] = l[i] + b;
+        const float dB = cB * wnorm[e], b = dB + 1e-6f * (fabsf(l[i]) + fabsf(be) + 1.0f);
+        // a bias of -inf (a masked expert): the exact logit is -inf as well, as no
+        // sum of the dot can overflow here (dB is 2^-9 of ||w|| ||x|| or more), and
+        // -inf + b would be NaN, a candidate
+        hi[i] = be == -__builtin_inff() && dB < 0x1p100f ? be : l[i] + b;
         lk[i] = (uint32_t)(topk_key(l[i] - b, 0) >> 32);
         mx = max(mx, lk[i]);
     }

@@ -86,3 +86,21 @@ def test_hot_experts_in_few_lanes(lib, H, T, K, per):
     got, ref, counters = _route(lib, H, T, K, bias)
     _check(got, ref)
     assert counters[0] == 0
+
+
+@pytest.mark.parametrize("H,T,K,finite", [(2048, 601, 10, 212), (2048, 1200, 16, 212), (2560, 1200, 10, 212),
+                                          (2048, 601, 10, 10), (2048, 4100, 10, 300), (2560, 601, 10, 6)])
+def test_masked_experts(lib, H, T, K, finite):
+    """Experts masked by a router bias of -inf are no candidates while top_k
+    others are left (their bounds are not NaN), and none is selected. With fewer
+    than top_k left every expert is a candidate, and the masked ones follow in
+    index order with weight 0."""
+    keep = np.random.default_rng(3).permutation(E)[:finite]
+    bias = np.full(E, -np.inf, np.float32)
+    bias[keep] = 0.0
+    got, ref, counters = _route(lib, H, T, K, bias)
+    _check(got, ref)
+    if finite >= K:
+        assert counters[0] == 0 and np.isin(got[0], keep).all()
+    else:
+        assert counters[0] == T and not got[1][:, finite:].any()
