@@ -326,15 +326,16 @@ size_t qfm_workspace_bytes(int M);
 /* For M > 8 logits is [M][E]: the exact canonical logits up to 600 rows, the
  * MFMA router GEMM's beyond (where the exact ones are computed only for the
  * selection candidates); hidden is NULL and counters points at {tokens whose
- * candidate set overflowed (more than 64 candidates for the top K), work items
- * of the gate/up GEMM, of the down GEMM (0: the same ones)} (int, device
- * memory; NULL for M <= 8). */
+ * candidate set overflowed (more than 64 candidates for the top K; beyond 600
+ * rows these recompute every logit), work items of the gate/up GEMM, work items
+ * of the down GEMM} (int, device memory; NULL for M <= 8). A work item is what
+ * one block computes: some rows of one expert times a part of its weights. */
 typedef struct {
     float *logits;   /* [M][E+1]: router logits; column E = <sh_gate_inp, x> */
     int   *sel;      /* [M][K] */
     float *wts;      /* [M][K] */
     float *hidden;   /* routed / shared intermediate activations */
-    int   *counters; /* prefill: {n_fallback, n_items_gateup, n_items_down}; else NULL */
+    int   *counters; /* M > 8: {n_overflow, n_items_gateup, n_items_down}; else NULL */
 } qfm_ws_view;
 int qfm_workspace_view(void *ws, int M, qfm_ws_view *v);
 

@@ -370,7 +370,7 @@ constexpr int kTopkLds = 16 + 256 + 64 + 64;   // results, candidates, junk slot
 // (LOAD false: v[] already holds the logits, v[i] = logit i * 64 + lane; lr unused)
 template <int EPL, bool LOAD = true>
 __device__ __forceinline__ int topk_candidates(const float *lr, int K, int lane, unsigned long long *lds,
-                                               float (&v)[EPL]) {
+                                               float (&v)[EPL], bool *over = nullptr) {
     static_assert(EPL >= 1 && EPL <= 16, "E = 64 * EPL, EPL <= 16");
     constexpr int E = 64 * EPL;
     constexpr int IB = E <= 64 ? 6 : E <= 128 ? 7 : E <= 256 ? 8 : E <= 512 ? 9 : 10;   // index bits
@@ -411,6 +411,7 @@ __device__ __forceinline__ int topk_candidates(const float *lr, int K, int lane,
     for (int i = 0; i < EPL; i++) b[i] = __ballot(k31[i] >= P);
 #pragma unroll
     for (int i = 0; i < EPL; i++) { base[i] = tot; tot += __popcll(b[i]); }
+    if (over) *over = tot > 64;
     if (tot > 64) {
         // exact bound: 64-bit lane maxima (wave-uniform branch)
         unsigned long long m64 = key[0];
@@ -466,8 +467,8 @@ __device__ __forceinline__ int topk_cand_rank(const unsigned long long *cand, in
 // denom, denom = sum over the K selected (renorm) or over all E (plain softmax).
 template <int EPL, bool LOAD>
 __device__ __forceinline__ void wave_topk_v(float (&v)[EPL], const float *lr, int K, int renorm, int lane,
-                                            unsigned long long *lds, int &my_i, float &my_w) {
-    const int n = topk_candidates<EPL, LOAD>(lr, K, lane, lds, v);
+                                            unsigned long long *lds, int &my_i, float &my_w, bool *over = nullptr) {
+    const int n = topk_candidates<EPL, LOAD>(lr, K, lane, lds, v, over);
     const unsigned long long *cand = lds + 16;
     for (int j = lane; j < n; j += 64) {
         const unsigned long long cj = cand[j];
@@ -497,11 +498,12 @@ __device__ __forceinline__ void wave_topk(const float *lr, int K, int renorm, in
     float v[EPL];
     wave_topk_v<EPL, true>(v, lr, K, renorm, lane, lds, my_i, my_w);
 }
-// The same from logits held in registers (v[i] = logit i * 64 + lane)
+// The same from logits held in registers (v[i] = logit i * 64 + lane); over:
+// whether more than 64 experts shared the prefix bound (the exact form ran)
 template <int EPL>
 __device__ __forceinline__ void wave_topk_regs(float (&v)[EPL], int K, int renorm, int lane,
-                                               unsigned long long *lds, int &my_i, float &my_w) {
-    wave_topk_v<EPL, false>(v, nullptr, K, renorm, lane, lds, my_i, my_w);
+                                               unsigned long long *lds, int &my_i, float &my_w, bool *over = nullptr) {
+    wave_topk_v<EPL, false>(v, nullptr, K, renorm, lane, lds, my_i, my_w, over);
 }
 // The expert id of rank `job` (< K) only (wave-uniform result): same candidate
 // set and ranks as wave_topk, no permutation through LDS and no softmax.

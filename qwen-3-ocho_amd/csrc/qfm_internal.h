@@ -152,7 +152,7 @@ struct MidArgs {
     float *wts, *gam;
     uint4 *x16;                         // x as fp16 scaled by 2^k per token, 2^-k in x16isc
     float *x16isc;
-    int *ctr;                           // {selection overflows, items, ...}
+    int *ctr;                           // {tokens with more than 64 candidates, gate/up blocks, down blocks, items, ...}
     int2 *pairs;                        // [T (K + shared)] {partial slot, weight}
     int4 *items;
     int max_items;                      // entries of items; mid_items_bound checked against it by the caller

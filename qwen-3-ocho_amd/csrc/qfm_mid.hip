@@ -151,9 +151,8 @@ k_mid_router(const float *__restrict__ W, const float *__restrict__ bias, const 
     }
 }
 
-// One wave per token (wave_topk). n_over counts the tokens of which more than
-// 64 experts share the leading 22 value bits of the K-th selected one or lie
-// above it (the candidates of the wave's ranking overflow there).
+// One wave per token (wave_topk). n_over counts the tokens with more than 64
+// candidates (the exact form of topk_candidates' bound).
 template <int EPL>
 __global__ void __launch_bounds__(256)
 k_mid_topk(const float *__restrict__ logits, int T, int K, int renorm, int *__restrict__ sel, float *__restrict__ wts,
@@ -168,16 +167,13 @@ k_mid_topk(const float *__restrict__ logits, int T, int K, int renorm, int *__re
     for (int i = 0; i < EPL; i++) v[i] = logits[(size_t)t * E + i * 64 + lane];
     int my_i;
     float my_w;
-    wave_topk_regs<EPL>(v, K, renorm, lane, s_tk[wave], my_i, my_w);
+    bool over;
+    wave_topk_regs<EPL>(v, K, renorm, lane, s_tk[wave], my_i, my_w, &over);
     if (lane < K) {
         sel[(size_t)t * K + lane] = my_i;
         wts[(size_t)t * K + lane] = my_w;
     }
-    const uint32_t kth = (uint32_t)(s_tk[wave][K - 1] >> 42);  // leading 22 bits of the K-th key
-    int n = 0;
-#pragma unroll
-    for (int i = 0; i < EPL; i++) n += __popcll(__ballot((uint32_t)(topk_key(v[i], 0) >> 42) >= kth));
-    if (n > 64 && lane == 0) atomicAdd(n_over, 1);
+    if (over && lane == 0) atomicAdd(n_over, 1);
 }
 
 // ---- plan -------------------------------------------------------------------------
@@ -188,12 +184,13 @@ k_mid_topk(const float *__restrict__ logits, int T, int K, int renorm, int *__re
 // items: the shared group's first, then the experts' in ascending order. The
 // selection is read in batches of 16 a thread, and a pair leaves as one 8-byte
 // store (scattered stores of three arrays and loads one at a time took 29 us at
-// 1021 rows).
+// 1021 rows). ctr[3] is the number of items, ctr[1] and ctr[2] the blocks that
+// gate/up (nrb an item) and down (ncb) work with (the workspace view's counters).
 constexpr int kPlanBatch = 16;
 __global__ void __launch_bounds__(1024)
 k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const float *__restrict__ gam, int T, int K,
            int E, int has_sh, int mt, int2 *__restrict__ pairs, int4 *__restrict__ items, int max_items,
-           int *__restrict__ n_items) {
+           int nrb, int ncb, int *__restrict__ ctr) {
     __shared__ int cnt[1024], sa[1024], sb[1024];
     const int g = threadIdx.x, S = K + has_sh, TK = T * K;
     cnt[g] = 0;
@@ -227,7 +224,12 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
     if (g < E)
         for (int i = 0; i < mi; i++) item(shi + sb[g] - mi + i, g, off + i * mt, min(mt, c - i * mt));
     for (int i = g; i < shi; i += 1024) item(i, E, TK + i * mt, min(mt, T - i * mt));
-    if (g == E - 1) n_items[0] = min(shi + sb[g], max_items);
+    if (g == E - 1) {
+        const int n = min(shi + sb[g], max_items);
+        ctr[1] = n * nrb;
+        ctr[2] = n * ncb;
+        ctr[3] = n;
+    }
     __syncthreads();
     const bool one = TK <= 1024 * kPlanBatch;                  // v still holds every id
     for (int p0 = g; p0 < TK; p0 += 1024 * kPlanBatch) {
@@ -590,16 +592,16 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
     // 425 / 462; NVFP4 198 / 345 / 422 / 500, 278 / 386 / 462 / 580, 436 / 526 /
     // 599 / 688. Four are taken for INT8 from 24 rows an expert.
     const int avg = T * K / E;
-    hipLaunchKernelGGL(k_mid_plan, dim3(1), dim3(1024), 0, s, a.sel, a.wts, a.g ? a.gam : nullptr, T, K, E, a.has_sh, mt,
-                       a.pairs, a.items, a.max_items, a.ctr + 1);
     const int dw = 64 * mid_dn_waves(I, nt);                      // columns, and threads, per down block
+    hipLaunchKernelGGL(k_mid_plan, dim3(1), dim3(1024), 0, s, a.sel, a.wts, a.g ? a.gam : nullptr, T, K, E, a.has_sh, mt,
+                       a.pairs, a.items, a.max_items, I / 64, H / dw, a.ctr);
     // (xcd_unit wants eight times the largest range: a multiple of 8)
     const dim3 g_gu((unsigned)((max_items * (I / 64) + 7) / 8 * 8)), g_dn((unsigned)((max_items * (H / dw) + 7) / 8 * 8)), b(256), bd((unsigned)dw);
 #define QFM_MID(HH, II, F4, NT, ONCE)                                                                               \
-    hipLaunchKernelGGL((k_mid_gateup<HH, II, F4, NT, ONCE>), g_gu, b, 0, s, a.items, a.ctr + 1, a.pairs,            \
+    hipLaunchKernelGGL((k_mid_gateup<HH, II, F4, NT, ONCE>), g_gu, b, 0, s, a.items, a.ctr + 3, a.pairs,            \
                        K + a.has_sh, reinterpret_cast<const uint16_t *>(a.x16), a.x16isc, a.gg, a.gu, E, a.hid,     \
                        a.hk);                                                                                       \
-    hipLaunchKernelGGL((k_mid_down<HH, II, F4, NT, ONCE>), g_dn, bd, 0, s, a.items, a.ctr + 1, a.pairs, a.hid,      \
+    hipLaunchKernelGGL((k_mid_down<HH, II, F4, NT, ONCE>), g_dn, bd, 0, s, a.items, a.ctr + 3, a.pairs, a.hid,      \
                        a.hk, a.gd, E, a.part, a.partk)
 #define QFM_MID_ONCE(HH, II, F4)                                                                                    \
     if (avg < (F4 ? 8 : 12)) { QFM_MID(HH, II, F4, 1, true); } else { QFM_MID(HH, II, F4, 1, false); }

@@ -698,7 +698,7 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
         for (int i = 0; i < EPL; i++)
             if ((cb[i] >> lane) & 1ull) s_cand[wave][pos[i]] = i * 64 + lane;
     }
-    if (overflow && renorm && w == 0 && lane == 0) atomicAdd(n_fallback, 1);
+    if (overflow && w == 0 && lane == 0) atomicAdd(n_fallback, 1);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const int nc = full ? E : total;
     float xv[NJ][4];                                     // this token's x slice, canonical lane layout

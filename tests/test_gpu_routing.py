@@ -104,3 +104,22 @@ def test_masked_experts(lib, H, T, K, finite):
         assert counters[0] == 0 and np.isin(got[0], keep).all()
     else:
         assert counters[0] == T and not got[1][:, finite:].any()
+
+
+# ------------------------------------------------------------------ counters
+@pytest.mark.parametrize("H,T,fmt,renorm,per", [(2048, 40, 0, 1, 16), (2048, 40, 1, 0, 16), (2560, 601, 1, 0, 16),
+                                                (2560, 1200, 0, 1, 16), (2048, 1300, 0, 0, 64), (2048, 2900, 0, 0, 128)])
+def test_workspace_counters(lib, H, T, fmt, renorm, per):
+    """The view's counters: the tokens with more than 64 candidates (here the
+    zero rows, whose logits all tie), with and without renormalization, and the
+    blocks of work of the two GEMMs, from the selection: items of `per` rows of
+    one expert times the weight blocks of each."""
+    K, I = 10, SHAPES[H]
+    x = orc.fill("gauss_bf16", 12, 41, orc.T_X, 0, T * H).reshape(T, H)
+    zero = [0, 7, T - 1]
+    x[zero] = 0
+    got, ref, counters = _route(lib, H, T, K, x=x, renorm=renorm, fmt=fmt)
+    _check(got, ref)
+    items = int((-(-np.bincount(got[0].ravel(), minlength=E) // per)).sum()) - (-T // per)   # and the shared expert's
+    gate_up, down = {16: (I // 64, H // 256), 64: (I // 64, H // 512), 128: (I // 128, H // 128)}[per]
+    assert counters.tolist() == [len(zero), items * gate_up, items * down]
