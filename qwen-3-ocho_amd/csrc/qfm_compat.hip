@@ -392,6 +392,79 @@ k_cx_down_part_i8(const int8_t *__restrict__ Wd, const float *__restrict__ Sd, c
     }
 }
 
+// ---- chunk tier, one row: a lane group per weight row and every load of it in
+// flight at once. Ten experts make 100 blocks of the tiles above, too few waves
+// for the latency of their chunks (whole call, us: 2048/512 23.1 against 31.0,
+// 2560/640 27.8 against 38.8; from two rows on the tiles are level or faster).
+template <int H, int I>
+__global__ void __launch_bounds__(256)
+k_cx_gateup_i8x8_row(const int8_t *__restrict__ Wg, const float *__restrict__ Sg, const int8_t *__restrict__ Wu,
+                     const float *__restrict__ Su, const int8_t *__restrict__ xq, const float *__restrict__ xs,
+                     float *__restrict__ hidden, const int *__restrict__ exp_slot, const int *__restrict__ exp_ptr,
+                     const int *__restrict__ pair_tok, const int *__restrict__ n_exp_dev) {
+    constexpr int CPR = H / 16, LPR = lpr_of(CPR), NST = CPR / LPR, RPB = 256 / LPR;
+    const int e = blockIdx.y;
+    if (e >= *n_exp_dev) return;
+    const int l = threadIdx.x % LPR, row = blockIdx.x * RPB + threadIdx.x / LPR;
+    const int slot = exp_slot[e], p1 = exp_ptr[e + 1];
+    const size_t woff = ((size_t)slot * I + row) * H;
+    uint4 wg[NST], wu[NST];
+#pragma unroll
+    for (int st = 0; st < NST; st++) {
+        wg[st] = ld_nt16(Wg + woff + (st * LPR + l) * 16);
+        wu[st] = ld_nt16(Wu + woff + (st * LPR + l) * 16);
+    }
+    const float sg = Sg[(size_t)slot * I + row], su = Su[(size_t)slot * I + row];
+    for (int p = exp_ptr[e]; p < p1; p++) {
+        const int tok = pair_tok[p];
+        float ag = 0.0f, au = 0.0f;
+#pragma unroll
+        for (int st = 0; st < NST; st++) {
+            const int c = st * LPR + l;
+            const uint4 xv = *reinterpret_cast<const uint4 *>(xq + (size_t)tok * H + c * 16);
+            const float sc = xs[(size_t)tok * (H / 32) + (c >> 1)];
+            ag = fmaf((float)dot16_i8i8(wg[st], xv), sc, ag);
+            au = fmaf((float)dot16_i8i8(wu[st], xv), sc, au);
+        }
+        ag = group_sum<LPR>(ag);
+        au = group_sum<LPR>(au);
+        if (l == 0) hidden[(size_t)p * I + row] = silu(ag * sg) * (au * su);
+    }
+}
+template <int H, int I>
+__global__ void __launch_bounds__(256)
+k_cx_down_part_i8_row(const int8_t *__restrict__ Wd, const float *__restrict__ Sd, const float *__restrict__ hidden,
+                      const float *__restrict__ pair_wt, const int *__restrict__ pair_tok,
+                      const int *__restrict__ exp_slot, const int *__restrict__ exp_ptr,
+                      const int *__restrict__ n_exp_dev, const int *__restrict__ sel, int K, float *__restrict__ part) {
+    constexpr int CPR = I / 16, LPR = lpr_of(CPR), NST = CPR / LPR, RPB = 256 / LPR;
+    const int e = blockIdx.y;
+    if (e >= *n_exp_dev) return;
+    const int l = threadIdx.x % LPR, row = blockIdx.x * RPB + threadIdx.x / LPR;
+    const int slot = exp_slot[e], p1 = exp_ptr[e + 1];
+    uint4 w[NST];
+#pragma unroll
+    for (int st = 0; st < NST; st++) w[st] = ld_nt16(Wd + ((size_t)slot * H + row) * I + (st * LPR + l) * 16);
+    const float sd = Sd[(size_t)slot * H + row];
+    for (int p = exp_ptr[e]; p < p1; p++) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int st = 0; st < NST; st++) {
+            float hv[16];
+            ld_f32x16(hidden + (size_t)p * I + (st * LPR + l) * 16, hv);
+            acc = dot16_i8f(w[st], hv, acc);
+        }
+        acc = group_sum<LPR>(acc);
+        if (l == 0) {
+            const int tok = pair_tok[p];
+            int k = 0;
+            for (int kk = K - 1; kk >= 0; kk--)
+                if (sel[(size_t)tok * K + kk] == slot) k = kk;
+            part[((size_t)tok * K + k) * H + row] = pair_wt[p] * sd * acc;
+        }
+    }
+}
+
 // y[t][i] = sum_k part[t*K + k][i], fixed k order (qf8_moe_i8.hip:312-322).
 __global__ void __launch_bounds__(256)
 k_cx_combine(const float *__restrict__ part, int K, int H, float *__restrict__ y) {
@@ -775,10 +848,19 @@ int qf8_i8_experts_chunk_ex(const Qf4ExpCache *c, const int8_t *xq, const float 
                        dim3(64 * mid_dn_waves(II, NT)), 0, s, c->i8_down, c->i8s_down, hidden, pair_wt, pair_tok,   \
                        exp_slot, exp_ptr, n_exp_dev, sel, K, part)
     QFM_SHAPE_DISPATCH({
-        hipLaunchKernelGGL((k_cx_gateup_i8x8<HH, II>), dim3(II / 64, n_exp_max), dim3(256), 0,
-                           s, c->i8_gate, c->i8s_gate, c->i8_up, c->i8s_up, xq, xs, hidden, exp_slot, exp_ptr,
-                           pair_tok, n_exp_dev);
-        if (nt == 1) { QFM_CX_DOWN(HH, II, 1); } else if (nt == 2) { QFM_CX_DOWN(HH, II, 2); } else { QFM_CX_DOWN(HH, II, 4); }
+        if (T == 1) {
+            hipLaunchKernelGGL((k_cx_gateup_i8x8_row<HH, II>), dim3(II / (256 / lpr_of(HH / 16)), n_exp_max), dim3(256),
+                               0, s, c->i8_gate, c->i8s_gate, c->i8_up, c->i8s_up, xq, xs, hidden, exp_slot, exp_ptr,
+                               pair_tok, n_exp_dev);
+            hipLaunchKernelGGL((k_cx_down_part_i8_row<HH, II>), dim3(HH / (256 / lpr_of(II / 16)), n_exp_max), dim3(256),
+                               0, s, c->i8_down, c->i8s_down, hidden, pair_wt, pair_tok, exp_slot, exp_ptr, n_exp_dev,
+                               sel, K, part);
+        } else {
+            hipLaunchKernelGGL((k_cx_gateup_i8x8<HH, II>), dim3(II / 64, n_exp_max), dim3(256), 0,
+                               s, c->i8_gate, c->i8s_gate, c->i8_up, c->i8s_up, xq, xs, hidden, exp_slot, exp_ptr,
+                               pair_tok, n_exp_dev);
+            if (nt == 1) { QFM_CX_DOWN(HH, II, 1); } else if (nt == 2) { QFM_CX_DOWN(HH, II, 2); } else { QFM_CX_DOWN(HH, II, 4); }
+        }
         hipLaunchKernelGGL(k_cx_combine, dim3((HH + 255) / 256, T), dim3(256), 0, s, part, K, HH, y);
     });
 #undef QFM_CX_DOWN

@@ -194,6 +194,48 @@ def test_experts_chunk_pair_tiles(lib, T, n_exp_max):
     L.destroy()
 
 
+@pytest.mark.parametrize("hidden,inter,T,n_exp_max", [(2048, 512, 1, 10), (2560, 640, 1, 10), (2560, 640, 2, 20),
+                                                      (2560, 640, 5, 50), (2560, 640, 17, 170), (2560, 640, 9, 10),
+                                                      (2560, 640, 21, 10), (2560, 640, 41, 10)])
+def test_experts_chunk_shapes(hidden, inter, T, n_exp_max):
+    """The chunk tier at the wider shape, whose down launch has other blocks (4, 8
+    and 4 waves for one, two and four token tiles against 4, 8 and 8) and rows of
+    640 bytes, and one row of both shapes (kernels of its own). Pairs and tolerance
+    as in test_experts_chunk_pair_tiles; one row adds -128 * sum of 16 values, with
+    at most 2^-24 * 128 of a value's rounding, to the sums: 1e-5 of the largest value
+    as well."""
+    seed, layer = 2, 6
+    _say("experts chunk H", hidden, "T", T, "bound", n_exp_max)
+    qfm.init(hidden, inter, E, K, 1, 1)
+    lib = qfm.load()
+    rng = np.random.default_rng(T)
+    sel = np.tile(rng.choice(E, K, replace=False).astype(np.int32), (T, 1))
+    for t in range(T):
+        rng.shuffle(sel[t])
+    wt = (rng.random((T, K)) + 0.1).astype(np.float32)
+    q, s = orc.x8_quant(rng.standard_normal(T * hidden).astype(np.float32))
+    q, s = q.reshape(T, hidden), s.reshape(T, hidden // 32)
+    xhat = q.astype(np.float64) * np.repeat(s.astype(np.float64), 32, axis=1)
+    L = qfm.SynthLayer(qfm.QFM_FMT_INT8, seed, layer)
+    P = T * K
+    dsel, dwt, dq, ds = _dev(sel), _dev(wt), _dev(q), _dev(s)
+    d_slot, d_ptr, d_tok, d_pw, d_cnt = (qfm.DevBuf(E * 4), qfm.DevBuf((E + 1) * 4), qfm.DevBuf(P * 4),
+                                         qfm.DevBuf(P * 4), qfm.DevBuf(8))
+    hid, part, y = qfm.DevBuf(P * inter * 4), qfm.DevBuf(P * hidden * 4), qfm.DevBuf(T * hidden * 4)
+    qfm.check(lib.qf8_i8_csr_build_ex(dsel.ptr, dwt.ptr, T, d_slot.ptr, d_ptr.ptr, d_tok.ptr, d_pw.ptr, d_cnt.ptr, None))
+    qfm.check(lib.qf8_i8_experts_chunk_ex(C.byref(L.s.arena), dq.ptr, ds.ptr, hid.ptr, None, None, d_slot.ptr, d_ptr.ptr,
+                                          d_tok.ptr, d_pw.ptr, d_cnt.ptr, n_exp_max, P, dsel.ptr, part.ptr, T, y.ptr,
+                                          None))
+    _sync(lib)
+    got = y.download(np.float32, (T, hidden))
+    w = {int(e): orc._i8_expert_arrays(seed, layer, int(e), hidden, inter) for e in sel[0]}
+    for t in range(T):
+        ref = sum(float(wt[t, k]) * orc.i8_expert(xhat[t], *w[int(sel[t, k])])[1] for k in range(K))
+        assert _rel(got[t], ref) <= 1e-5, t
+    L.destroy()
+    qfm.init(H, I, E, K, 1, 1)
+
+
 # ------------------------------------------------------------------ NVFP4 M=1
 def test_nvfp4_m1_entry_points(lib):
     seed, layer = 3, 5
