@@ -1,5 +1,6 @@
 // qfm_internal.h -- host-side internals shared by the translation units.
 #pragma once
+#include "qfm_prefill_layout.h"
 #include "../../include/qf_moe.h"
 #include <hip/hip_runtime.h>
 
@@ -131,17 +132,22 @@ struct GroupW {
     const float *s2;      // NVFP4 per-expert global scales [E]
 };
 
-// The middle path (8 < T <= mid_rows_max, qfm_mid.hip): router, selection, plan
+// The middle path (8 < T, mid_takes; qfm_mid.hip): router, selection, plan
 // and the two grouped GEMMs, up to the fp16 partials that k_pf_combine_h sums.
-// Where it ends against the prefill's 128-row tiles, us per layer, here / tiles:
-// 2048/512 INT8 1500 rows 507 / 620, 2560/640 INT8 1500 rows 841 / 932, NVFP4
-// 2048/512 458 / 686, 2560/640 723 / 991; it grows by 0.13, 0.30, 0.19 and 0.28
-// us a row, the tiles by 0.04 to 0.07.
-constexpr int mid_rows_max(int I, bool f4) { return I <= 512 ? 2800 : f4 ? 2500 : 1800; }
+// mid_takes and mid_offers_tiles (qfm_prefill_layout.h) say where it ends and
+// where its plan may leave the GEMMs to the prefill's 128-row tiles.
 // up to here the exact router of every expert (k_mid_router), beyond it
 // k_pf_select's candidates: 300 / 450 / 1021 rows 23 / 32 / 66 us, with the
 // selection 28 / 37 / 71, against 44 at 450 rows and 50 at 1021
 constexpr int kMidExactRows = 600;
+// The 128-row tiles as a middle call's other form: room in their work lists, in
+// m-tiles (0: not offered), n-tiles, and what decides. The gate/up list lies in
+// the items' region.
+struct MidTiles {
+    int max_mt, nt_gu, nt_dn;
+    int4 *items_dn;
+    MidCost cost;
+};
 struct MidArgs {
     const float *router, *bias, *g;     // g: shared-expert gate vector or nullptr
     const uint16_t *x;
@@ -151,8 +157,8 @@ struct MidArgs {
     int *sel;
     float *wts, *gam;
     uint4 *x16;                         // x as fp16 scaled by 2^k per token, 2^-k in x16isc
-    float *x16isc;
-    int *ctr;                           // {tokens with more than 64 candidates, gate/up blocks, down blocks, items, ...}
+    float *x16isc, *xsum, *x16sum;      // row sums of x and of the scaled x (the tile GEMMs' offset corrections)
+    int *ctr;                           // {tokens with more than 64 candidates, gate/up blocks, down blocks, items, tile items}
     int2 *pairs;                        // [T (K + shared)] {partial slot, weight}
     int4 *items;
     int max_items;                      // entries of items; mid_items_bound checked against it by the caller
@@ -161,6 +167,7 @@ struct MidArgs {
     uint16_t *part;                     // [T (K + shared)][H] fp16
     int8_t *partk;                      // [T (K + shared)][H / 64]
     GroupW gg, gu, gd;
+    MidTiles tiles;
 };
 int launch_mid(const MidArgs &a, hipStream_t s);
 

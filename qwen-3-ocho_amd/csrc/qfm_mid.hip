@@ -1,4 +1,4 @@
-// qfm_mid.hip -- the forward at a middle number of rows (8 < T <= mid_rows_max):
+// qfm_mid.hip -- the forward at a middle number of rows (more than 8, mid_takes):
 // weight-streaming grouped MFMA GEMMs.
 //
 // Reference behaviour: the chunk path (ocho/amd_server/qf8_moe_i8.hip:196-395)
@@ -10,10 +10,12 @@
 // Launches:
 //   k_mid_router   exact logits in the canonical fp32 order (8 token rows in
 //                  LDS at a time, two experts per wave), the shared-expert
-//                  gate, and x as fp16 scaled by 2^k per token;
+//                  gate, and x as fp16 scaled by 2^k per token with row sums;
 //   k_mid_topk     one wave per token (wave_topk);
 //   k_mid_plan     one block: the pairs grouped by expert and the work items
-//                  {group, first pair, rows <= 16 NT};
+//                  {group, first pair, rows <= 16 NT}, or the tiles of the
+//                  prefill's GEMMs where a router crowds its rows on few experts
+//                  (mid_cost; these then run in place of the next two);
 //   k_mid_gateup   hidden = silu(g) * u per item and 64 intermediate rows, as
 //                  fp16 scaled by 2^k per pair and those 64;
 //   k_mid_down     partials per item and 256 output columns, as fp16 scaled by
@@ -46,7 +48,8 @@ template <int NJ>
 __global__ void __launch_bounds__(256, NJ == 8 ? 3 : 2)
 k_mid_router(const float *__restrict__ W, const float *__restrict__ bias, const float *__restrict__ g,
              const uint16_t *__restrict__ x, int T, int E, int tg, float *__restrict__ logits,
-             float *__restrict__ gam, uint4 *__restrict__ x16, float *__restrict__ x16isc, int *__restrict__ ctr) {
+             float *__restrict__ gam, uint4 *__restrict__ x16, float *__restrict__ x16isc, float *__restrict__ xsum,
+             float *__restrict__ x16sum, int *__restrict__ ctr) {
     constexpr int H = NJ * 256;
     __shared__ __align__(16) uint16_t s_x[8 * H];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -71,6 +74,7 @@ k_mid_router(const float *__restrict__ W, const float *__restrict__ bias, const 
         const int k = amax == 0.0f ? 0 : min(113, max(-113, 141 - (int)(__float_as_uint(amax) >> 23)));
         const float sc = __uint_as_float((uint32_t)(127 + k) << 23);
         uint4 *xo = x16 + (size_t)t * (H / 8);
+        float sx = 0.0f, hs = 0.0f;
 #pragma unroll
         for (int q = 0; q < NC; q++) {
             const uint32_t d[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
@@ -78,9 +82,17 @@ k_mid_router(const float *__restrict__ W, const float *__restrict__ bias, const 
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const f16x2_t hp = {(_Float16)(bf16_lo(d[u]) * sc), (_Float16)(bf16_hi(d[u]) * sc)};
+                sx += bf16_lo(d[u]) + bf16_hi(d[u]);
+                hs += (float)hp.x + (float)hp.y;
                 o[u] = __builtin_bit_cast(uint32_t, hp);
             }
             xo[q * 64 + lane] = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+        sx = group_sum<64>(sx);
+        hs = group_sum<64>(hs);
+        if (lane == 0) {
+            xsum[t] = sx;
+            x16sum[t] = hs;
         }
         if (lane == 0) x16isc[t] = __uint_as_float((uint32_t)(127 - k) << 23);
         return;
@@ -184,14 +196,16 @@ k_mid_topk(const float *__restrict__ logits, int T, int K, int renorm, int *__re
 // items: the shared group's first, then the experts' in ascending order. The
 // selection is read in batches of 16 a thread, and a pair leaves as one 8-byte
 // store (scattered stores of three arrays and loads one at a time took 29 us at
-// 1021 rows). ctr[3] is the number of items, ctr[1] and ctr[2] the blocks that
-// gate/up (nrb an item) and down (ncb) work with (the workspace view's counters).
+// 1021 rows). ctr[3] is the number of items, ctr[4] and ctr[5] those of the tile
+// GEMMs (one pair of the three is 0), ctr[1] and ctr[2] the blocks that gate/up
+// and down work with (the workspace view's counters; nrb and ncb an item).
 constexpr int kPlanBatch = 16;
 __global__ void __launch_bounds__(1024)
 k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const float *__restrict__ gam, int T, int K,
            int E, int has_sh, int mt, int2 *__restrict__ pairs, int4 *__restrict__ items, int max_items,
-           int nrb, int ncb, int *__restrict__ ctr) {
+           int nrb, int ncb, MidTiles tp, int *__restrict__ ctr) {
     __shared__ int cnt[1024], sa[1024], sb[1024];
+    constexpr int BM = kPfTileRows;
     const int g = threadIdx.x, S = K + has_sh, TK = T * K;
     cnt[g] = 0;
     __syncthreads();
@@ -207,9 +221,9 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
     const int c = g < E ? cnt[g] : 0;
     const int mi = (c + mt - 1) / mt;
     sa[g] = c;
-    sb[g] = mi;
+    sb[g] = mi | ((c + BM - 1) / BM) << 16;                    // items, and 128-row tiles
     __syncthreads();
-    for (int st = 1; st < E; st <<= 1) {                       // inclusive scans
+    for (int st = 1; st < E; st <<= 1) {                       // inclusive scans (packed: neither half carries)
         const int a = g >= st && g < E ? sa[g - st] : 0, b = g >= st && g < E ? sb[g - st] : 0;
         __syncthreads();
         sa[g] += a;
@@ -218,17 +232,48 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
     }
     const int off = sa[g] - c, shi = has_sh ? (T + mt - 1) / mt : 0;
     cnt[g] = off;                                              // the group's next free pair
+    const int ngrp = __syncthreads_count(c > 0);
+    const int n16 = (sb[E - 1] & 0xFFFF) + shi, mtr = sb[E - 1] >> 16, mtot = mtr + (has_sh ? (T + BM - 1) / BM : 0);
+    const int gcost = (ngrp + has_sh) * tp.cost.group + (n16 - ngrp - has_sh) * tp.cost.item;
+    const bool tiles = mtot <= tp.max_mt && mtot * tp.cost.tile + tp.cost.base < gcost;   // (block-uniform)
+    if (tiles) {
+        // the work lists of k_pf_gemm, as k_pf_plan stores them: one thread per m-tile
+        const int cgu = (mtot + 7) >> 3;
+        for (int m = g; m < mtot; m += 1024) {
+            int grp = E, row0 = (m - mtr) * BM, rows = min(BM, T - row0), pb = TK + row0;
+            if (m < mtr) {
+                int lo = 0, hi = E - 1;                        // first group whose tiles end past m
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if ((sb[mid] >> 16) > m) hi = mid; else lo = mid + 1;
+                }
+                const int end = sa[lo], cl = end - (lo ? sa[lo - 1] : 0);
+                grp = lo;
+                row0 = (m - (lo ? sb[lo - 1] >> 16 : 0)) * BM;
+                rows = min(BM, cl - row0);
+                pb = end - cl + row0;
+            }
+            const int xg = m / cgu, mlg = m - xg * cgu;
+            for (int n = 0; n < tp.nt_gu; n++) items[((mlg * tp.nt_gu + n) << 3) | xg] = make_int4(grp, pb, rows, n);
+            for (int n = 0; n < tp.nt_dn; n++)
+                tp.items_dn[(((m >> 3) * tp.nt_dn + n) << 3) | (m & 7)] = make_int4(grp, pb, rows, n);
+        }
+    }
     auto item = [&](int i, int grp, int first, int rows) __attribute__((always_inline)) {
         if (i < max_items) items[i] = make_int4(grp, first, rows, 0);   // (the host's bound lies below max_items)
     };
-    if (g < E)
-        for (int i = 0; i < mi; i++) item(shi + sb[g] - mi + i, g, off + i * mt, min(mt, c - i * mt));
-    for (int i = g; i < shi; i += 1024) item(i, E, TK + i * mt, min(mt, T - i * mt));
-    if (g == E - 1) {
-        const int n = min(shi + sb[g], max_items);
-        ctr[1] = n * nrb;
-        ctr[2] = n * ncb;
+    if (!tiles) {
+        if (g < E)
+            for (int i = 0; i < mi; i++) item(shi + (sb[g] & 0xFFFF) - mi + i, g, off + i * mt, min(mt, c - i * mt));
+        for (int i = g; i < shi; i += 1024) item(i, E, TK + i * mt, min(mt, T - i * mt));
+    }
+    if (g == 0) {
+        const int n = tiles ? 0 : min(n16, max_items);
+        ctr[1] = tiles ? mtot * tp.nt_gu : n * nrb;
+        ctr[2] = tiles ? mtot * tp.nt_dn : n * ncb;
         ctr[3] = n;
+        ctr[4] = tiles ? mtot * tp.nt_gu : 0;
+        ctr[5] = tiles ? mtot * tp.nt_dn : 0;
     }
     __syncthreads();
     const bool one = TK <= 1024 * kPlanBatch;                  // v still holds every id
@@ -579,10 +624,10 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
         const unsigned g_r = (unsigned)((T + 3) / 4 + nx * ((ng + tg - 1) / tg));
         if (H == 2048)
             hipLaunchKernelGGL(k_mid_router<8>, dim3(g_r), dim3(256), 0, s, a.router, a.bias, a.g, a.x, T, E, tg, a.logits,
-                               a.gam, a.x16, a.x16isc, a.ctr);
+                               a.gam, a.x16, a.x16isc, a.xsum, a.x16sum, a.ctr);
         else
             hipLaunchKernelGGL(k_mid_router<10>, dim3(g_r), dim3(256), 0, s, a.router, a.bias, a.g, a.x, T, E, tg, a.logits,
-                               a.gam, a.x16, a.x16isc, a.ctr);
+                               a.gam, a.x16, a.x16isc, a.xsum, a.x16sum, a.ctr);
         hipLaunchKernelGGL(k_mid_topk<8>, dim3((T + 3) / 4), dim3(256), 0, s, a.logits, T, K, c.renorm, a.sel, a.wts, a.ctr);
     }
     // token tiles per item. One (16 rows) keeps three blocks on a CU, which
@@ -591,10 +636,9 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
     // four tiles: INT8 289 / 370 / 443 / 534, 321 / 373 / 466 / 589, 343 / 380 /
     // 425 / 462; NVFP4 198 / 345 / 422 / 500, 278 / 386 / 462 / 580, 436 / 526 /
     // 599 / 688. Four are taken for INT8 from 24 rows an expert.
-    const int avg = T * K / E;
     const int dw = 64 * mid_dn_waves(I, nt);                      // columns, and threads, per down block
     hipLaunchKernelGGL(k_mid_plan, dim3(1), dim3(1024), 0, s, a.sel, a.wts, a.g ? a.gam : nullptr, T, K, E, a.has_sh, mt,
-                       a.pairs, a.items, a.max_items, I / 64, H / dw, a.ctr);
+                       a.pairs, a.items, a.max_items, I / 64, H / dw, a.tiles, a.ctr);
     // (xcd_unit wants eight times the largest range: a multiple of 8)
     const dim3 g_gu((unsigned)((max_items * (I / 64) + 7) / 8 * 8)), g_dn((unsigned)((max_items * (H / dw) + 7) / 8 * 8)), b(256), bd((unsigned)dw);
 #define QFM_MID(HH, II, F4, NT, ONCE)                                                                               \
@@ -604,7 +648,7 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
     hipLaunchKernelGGL((k_mid_down<HH, II, F4, NT, ONCE>), g_dn, bd, 0, s, a.items, a.ctr + 3, a.pairs, a.hid,      \
                        a.hk, a.gd, E, a.part, a.partk)
 #define QFM_MID_ONCE(HH, II, F4)                                                                                    \
-    if (avg < (F4 ? 8 : 12)) { QFM_MID(HH, II, F4, 1, true); } else { QFM_MID(HH, II, F4, 1, false); }
+    if (mid_reads_once(T, E, K, a.f4)) { QFM_MID(HH, II, F4, 1, true); } else { QFM_MID(HH, II, F4, 1, false); }
     if (shape_2048()) {
         if (a.f4) { QFM_MID_ONCE(2048, 512, true) } else if (nt == 1) { QFM_MID_ONCE(2048, 512, false) } else { QFM_MID(2048, 512, false, 4, false); }
     } else {

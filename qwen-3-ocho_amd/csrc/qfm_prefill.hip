@@ -54,7 +54,7 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-constexpr int BM = 128, BN = 128;
+constexpr int BM = kPfTileRows, BN = 128;
 constexpr int kCandMax = 64;
 
 // bf16 bits of an exactly representable value (integers |v| <= 256): truncation is exact
@@ -119,7 +119,8 @@ __global__ void __launch_bounds__(256) k_pf_router_prep(const float *__restrict_
                                                          const uint16_t *__restrict__ x, int T,
                                                          float *__restrict__ xnorm, float *__restrict__ xsum,
                                                          uint4 *__restrict__ x16, float *__restrict__ x16sum,
-                                                         float *__restrict__ x16isc) {
+                                                         float *__restrict__ x16isc, int *__restrict__ ctr) {
+    if (blockIdx.x == 0 && threadIdx.x < 8) ctr[threadIdx.x] = 0;   // (counted into by later launches)
     if ((int)blockIdx.x >= E) {
         constexpr int kMaxCh = 5;                    // 16-byte chunks per lane: H / 512 <= 5
         const int lane = threadIdx.x & 63;
@@ -284,10 +285,10 @@ struct TileEngine {
         u32x4_t a[NA], b[NB];                     // (with uint4 the stages were promoted to LDS or scratch)
         uint32_t sc[NB];
     };
-    __device__ static void run(const uint16_t *__restrict__ A, long lda, const int *arow,
+    __device__ static void run(int tid, const uint16_t *__restrict__ A, long lda, const int *arow,
                                const char *const *bptr, int K, Lds &L, f32x4_t (&acc)[MW][4],
                                const char *const *sptr = nullptr) {
-        const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+        const int t = tid, wave = t >> 6, lane = t & 63;
         const int wm = wave / WN, wn = wave % WN;
         const uint16_t *ap[NA];
         int a_lds[NA];
@@ -499,7 +500,7 @@ k_pf_router_mfma(const uint16_t *__restrict__ x, int T, int H, const uint16_t *_
     if (threadIdx.x < BN) bptr[threadIdx.x] = reinterpret_cast<const char *>(Wb + (size_t)(e0 + threadIdx.x) * H + k0);
     __syncthreads();
     f32x4_t acc[4][4];
-    RouterEngine::run(x + k0, H, arow, bptr, Hk, lds, acc);
+    RouterEngine::run(threadIdx.x, x + k0, H, arow, bptr, Hk, lds, acc);
     float *lg_approx = lg_part + (size_t)ks * T * E;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wm = wave >> 1, wn = wave & 1;
 #pragma unroll
@@ -886,13 +887,16 @@ enum { kAllI8 = 0, kRoutedF4 = 1, kDownI8 = 2 };
 template <int MODE>
 using GemmEngine = std::conditional_t<MODE == kDownI8, DownEngineI8,
                                       std::conditional_t<MODE == kAllI8, ExpertEngine, ExpertEngineF4>>;
+// One tile: block `blk` of the grid's order, its item `it` (stored at that index
+// by k_pf_plan), nit the items of the launch. The pairs are three arrays, or
+// (pairs != nullptr) k_mid_plan's {partial slot, weight} with S slots a token.
 template <bool GATEUP, int MODE>
-__global__ void __launch_bounds__(GemmEngine<MODE>::NT)
-__attribute__((amdgpu_waves_per_eu(GemmEngine<MODE>::WavesPerSimd, GemmEngine<MODE>::WavesPerSimd)))
-k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int which, const int *__restrict__ p_tok, const int *__restrict__ p_slot, const float *__restrict__ p_wt,
-          const uint16_t *__restrict__ A, int Kdim, int Nrows, GroupW g0, GroupW g1, int E,
-          uint16_t *__restrict__ hid, uint16_t *__restrict__ part, int8_t *__restrict__ partk, int Hout, int ntiles,
-          const float *__restrict__ xsum, float *__restrict__ hsum, int nt_gu, const float *__restrict__ xisc) {
+__device__ __forceinline__ void
+pf_gemm_tile(int tid, int blk, int nit, int4 it, const int *__restrict__ p_tok, const int *__restrict__ p_slot,
+             const float *__restrict__ p_wt, const int2 *__restrict__ pairs, int S, const uint16_t *__restrict__ A,
+             int Kdim, int Nrows, const GroupW &g0, const GroupW &g1, int E, uint16_t *__restrict__ hid,
+             uint16_t *__restrict__ part, int8_t *__restrict__ partk, int Hout, int ntiles,
+             const float *__restrict__ xsum, float *__restrict__ hsum, int nt_gu, const float *__restrict__ xisc) {
     static_assert(MODE != kDownI8 || !GATEUP, "the narrow tiles are for the down GEMM");
     using Eng = GemmEngine<MODE>;
     constexpr int WN = Eng::WNc, TBN = Eng::BNt;
@@ -906,16 +910,11 @@ k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int w
     __shared__ float rsum[BM], rscl[H16 ? BM : 1];
     __shared__ int rslot[GATEUP ? 1 : BM];          // down: the owned partial slot of each row
     __shared__ float rwt[GATEUP ? 1 : BM];          // down: the routing weight of each row
-    // the tile count and this block's item (stored at the block's index by
-    // k_pf_plan) as two independent loads ahead of the first branch
-    const int nit = n_items[which];
-    const int4 it = items[blockIdx.x];
-    args_now(nit, it.x, it.y, it.z, it.w);
     int mi, ni;
     if constexpr (GATEUP) {
-        if (!xcd_tile_contig(blockIdx.x, ntiles, nit / ntiles, mi, ni)) return;
+        if (!xcd_tile_contig(blk, ntiles, nit / ntiles, mi, ni)) return;
     } else {
-        xcd_tile(blockIdx.x, ntiles, mi, ni);
+        xcd_tile(blk, ntiles, mi, ni);
         if (mi * ntiles >= nit) return;
     }
     const int grp = it.x, pbase = it.y, rows = it.z, nt = it.w;
@@ -941,25 +940,31 @@ k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int w
     // A row sums (the offset-binary correction): x rows' sums for gate/up; for
     // down, the sum of the nt_gu per-tile partial sums the gate/up epilogue
     // wrote for the pair's bf16 hidden row (fixed order: deterministic)
-    if (threadIdx.x < BM) {
-        const int r = threadIdx.x;
+    if (tid < BM) {
+        const int r = tid;
         float rs = 0.0f;
         if (GATEUP) {
-            arow[r] = r < rows ? p_tok[pbase + r] : -1;
+            arow[r] = r < rows ? (pairs ? pairs[pbase + r].x / S : p_tok[pbase + r]) : -1;
             if (r < rows) rs = xsum[arow[r]];
             if constexpr (H16) rscl[r] = r < rows ? xisc[arow[r]] : 0.0f;
         } else {
             arow[r] = r < rows ? pbase + r : -1;
             if (r < rows) {
                 for (int q = 0; q < nt_gu; q++) rs += hsum[(size_t)(pbase + r) * nt_gu + q];
-                rslot[r] = p_slot[pbase + r];
-                rwt[r] = p_wt[pbase + r];
+                if (pairs) {
+                    const int2 pr = pairs[pbase + r];
+                    rslot[r] = pr.x;
+                    rwt[r] = __int_as_float(pr.y);
+                } else {
+                    rslot[r] = p_slot[pbase + r];
+                    rwt[r] = p_wt[pbase + r];
+                }
             }
         }
         rsum[r] = rs;
     }
-    if (threadIdx.x < TBN) {
-        const int n = threadIdx.x;
+    if (tid < TBN) {
+        const int n = tid;
         if (GATEUP) {
             // wave column wn = n / 64 holds intermediate rows [(TBN / 2) nt + 32 wn, +32):
             // its n-blocks 0, 1 are their gate rows and n-blocks 2, 3 the same up rows
@@ -975,7 +980,7 @@ k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int w
     // engine geometry: MWv m-blocks of 16 rows per wave, Eng::WMc waves along the rows
     constexpr int MWv = Eng::MWc;
     constexpr int RPW = 16 * MWv;                   // rows per wave
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wm = wave / WN, wn = wave % WN;
+    const int wave = tid >> 6, lane = tid & 63, wm = wave / WN, wn = wave % WN;
     // the epilogue's column scales, loaded before the k-loop (their latency would
     // otherwise open the epilogue): gate/up columns o0 + 16 nb, down c0 + 16 nb
     const int o0 = nt * (TBN / 2) + wn * 32 + (lane & 15);
@@ -993,12 +998,12 @@ k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int w
     }
     f32x4_t acc[MWv][4];
     if constexpr (F4) {
-        if (grp < E) ExpertEngineF4::run(A, Kdim, arow, bptr, Kdim, lds, acc, sptr);
-        else SharedEngineI8::run(A, Kdim, arow, bptr, Kdim, lds, acc);
+        if (grp < E) ExpertEngineF4::run(tid, A, Kdim, arow, bptr, Kdim, lds, acc, sptr);
+        else SharedEngineI8::run(tid, A, Kdim, arow, bptr, Kdim, lds, acc);
     } else if constexpr (MODE == kDownI8) {
-        DownEngineI8::run(A, Kdim, arow, bptr, Kdim, lds, acc);
+        DownEngineI8::run(tid, A, Kdim, arow, bptr, Kdim, lds, acc);
     } else {
-        ExpertEngine::run(A, Kdim, arow, bptr, Kdim, lds, acc);
+        ExpertEngine::run(tid, A, Kdim, arow, bptr, Kdim, lds, acc);
     }
     // epilogues: the per-row values come from the LDS tables filled above (no
     // per-element global loads). The gate/up tile is staged in LDS (the
@@ -1033,7 +1038,7 @@ k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int w
         // 16-lane reduction in its fixed order (deterministic)
         constexpr int CPR = HC / 8, RPP = Eng::NT / CPR;
         static_assert(CPR == 16 && BM % RPP == 0, "16 chunks per hidden row");
-        const int cch = threadIdx.x % CPR, rr = threadIdx.x / CPR;
+        const int cch = tid % CPR, rr = tid / CPR;
 #pragma unroll
         for (int p = 0; p < BM / RPP; p++) {
             const int r = p * RPP + rr;
@@ -1114,6 +1119,45 @@ k_pf_gemm(const int4 *__restrict__ items, const int *__restrict__ n_items, int w
             }
     }
 }
+
+#define QFM_GEMM_PARAMS                                                                                              \
+    const int4 *__restrict__ items, const int *__restrict__ n_items, int which, const int *__restrict__ p_tok,         \
+        const int *__restrict__ p_slot, const float *__restrict__ p_wt, const int2 *__restrict__ pairs, int S,         \
+        const uint16_t *__restrict__ A, int Kdim, int Nrows, GroupW g0, GroupW g1, int E, uint16_t *__restrict__ hid,  \
+        uint16_t *__restrict__ part, int8_t *__restrict__ partk, int Hout, int ntiles, const float *__restrict__ xsum, \
+        float *__restrict__ hsum, int nt_gu, const float *__restrict__ xisc
+#define QFM_GEMM_TILE(BLK, IT)                                                                                       \
+    pf_gemm_tile<GATEUP, MODE>(tid, BLK, nit, IT, p_tok, p_slot, p_wt, pairs, S, A, Kdim, Nrows, g0, g1, E, hid, part,      \
+                               partk, Hout, ntiles, xsum, hsum, nt_gu, xisc)
+// a block per tile
+template <bool GATEUP, int MODE>
+__global__ void __launch_bounds__(GemmEngine<MODE>::NT)
+__attribute__((amdgpu_waves_per_eu(GemmEngine<MODE>::WavesPerSimd, GemmEngine<MODE>::WavesPerSimd)))
+k_pf_gemm(QFM_GEMM_PARAMS) {
+    // the tile count and this block's item as two independent loads ahead of the first branch
+    const int nit = n_items[which];
+    const int4 it = items[blockIdx.x];
+    args_now(nit, it.x, it.y, it.z, it.w);
+    const int tid = threadIdx.x;
+    QFM_GEMM_TILE(blockIdx.x, it);
+}
+// The same tiles over the resident blocks (a multiple of 8: blk & 7 stays the
+// block's XCD), for calls in which k_mid_plan may leave none: launched without
+// work these take 2.5 us each, a block per possible tile 7 and 10.
+template <bool GATEUP, int MODE>
+__global__ void __launch_bounds__(GemmEngine<MODE>::NT)
+__attribute__((amdgpu_waves_per_eu(GemmEngine<MODE>::WavesPerSimd, GemmEngine<MODE>::WavesPerSimd)))
+k_pf_gemm_loop(QFM_GEMM_PARAMS) {
+    const int nit = n_items[which], nblk = ((nit / ntiles + 7) & ~7) * ntiles;
+    for (int blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
+        if (blk != (int)blockIdx.x) __syncthreads();   // the previous tile's LDS is consumed
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));                  // (LDS addresses hoisted out of this loop spill)
+        QFM_GEMM_TILE(blk, items[blk]);
+    }
+}
+#undef QFM_GEMM_PARAMS
+#undef QFM_GEMM_TILE
 
 // Four sums to y as bf16 (round to nearest even), or to y32 as fp32 when
 // y32 != nullptr (y is then not written).
@@ -1242,19 +1286,39 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
         gu = GroupW{a->i8_up, a->i8s_up, L->sh_up.w, L->sh_up.s, nullptr, nullptr};
         gd = GroupW{a->i8_down, a->i8s_down, L->sh_down.w, L->sh_down.s, nullptr, nullptr};
     }
+    // the grouped GEMMs, their item counts at cnt: a block per tile, or (the middle
+    // path's other form) as many blocks as are resident
+    auto tile_gemms = [&](bool loop, const int *cnt, const int2 *pairs) {
+        const unsigned cu = 256;                           // compute units; a 512-thread block fills one
+        const dim3 nth(f4 ? ExpertEngineF4::NT : ExpertEngine::NT), nth_dn(f4 ? ExpertEngineF4::NT : DownEngineI8::NT),
+            g_gu(loop ? cu : (unsigned)(max_mt * nt_gu)), g_dn(loop ? (f4 ? cu : 2 * cu) : (unsigned)(max_mt * nt_dn));
+#define QFM_PF_GEMM(KERNEL)                                                                                          \
+    if (f4) {                                                                                                        \
+        hipLaunchKernelGGL((KERNEL<true, kRoutedF4>), g_gu, nth, 0, s, items_gu, cnt, 0, p_tok, p_slot, p_wt, pairs,  \
+                           S, x, H, I, gg, gu, E, hid, part, partk, H, nt_gu, xsum, hsum, nt_gu, nullptr);            \
+        hipLaunchKernelGGL((KERNEL<false, kRoutedF4>), g_dn, nth_dn, 0, s, items_dn, cnt, 1, p_tok, p_slot, p_wt,     \
+                           pairs, S, hid, I, H, gd, gd, E, hid, part, partk, H, nt_dn, xsum, hsum, nt_gu, nullptr);   \
+    } else {                                                                                                         \
+        hipLaunchKernelGGL((KERNEL<true, kAllI8>), g_gu, nth, 0, s, items_gu, cnt, 0, p_tok, p_slot, p_wt, pairs, S,  \
+                           reinterpret_cast<const uint16_t *>(x16), H, I, gg, gu, E, hid, part, partk, H, nt_gu,      \
+                           x16sum, hsum, nt_gu, x16isc);                                                             \
+        hipLaunchKernelGGL((KERNEL<false, kDownI8>), g_dn, nth_dn, 0, s, items_dn, cnt, 1, p_tok, p_slot, p_wt,       \
+                           pairs, S, hid, I, H, gd, gd, E, hid, part, partk, H, nt_dn, xsum, hsum, nt_gu, nullptr);   \
+    }
+        if (loop) { QFM_PF_GEMM(k_pf_gemm_loop) } else { QFM_PF_GEMM(k_pf_gemm) }
+#undef QFM_PF_GEMM
+    };
     // router and selection: exact logits of every expert up to kMidExactRows
     // rows (launch_mid), the bf16 MFMA GEMM with exact candidates beyond
-    const bool mid = T <= mid_rows_max(I, f4);
-    const int room = (int)(Lw.bytes[kPfItemsGu] / sizeof(int4));
+    const bool mid = mid_takes(T, K, I, f4), offer = mid && mid_offers_tiles(T, I);
+    const int room = (int)(Lw.bytes[kPfItemsGu] / sizeof(int4)), mid_nt = mid_token_tiles(T, E, K, I, f4);
     if (mid) {
-        const int need = mid_items_bound(T, E, K, has_sh, mid_token_tiles(T, E, K, I, f4));
+        const int need = mid_items_bound(T, E, K, has_sh, mid_nt);
         if (need > room) { set_error(-2, "mid path: %d items, room for %d", need, room); return -2; }
     }
     if (!mid || T > kMidExactRows) {
-        // zero the small counters with a fill kernel (no memset node in captured graphs)
-        launch_fill_f32(reinterpret_cast<float *>(ctr), 8, 0.0f, s);
         hipLaunchKernelGGL(k_pf_router_prep, dim3((unsigned)(E + (T + 3) / 4)), dim3(256), 0, s, L->router, E, H, wnorm,
-                           wb16, x, T, xnorm, xsum, mid || !f4 ? x16 : nullptr, x16sum, x16isc);
+                           wb16, x, T, xnorm, xsum, mid || !f4 ? x16 : nullptr, x16sum, x16isc, ctr);
         const int nks = pf_router_slices(T, E, Lw.bytes[kPfPart]);
         const bool split = pf_select_split(T, nks);
         float *lgp = nks > 1 ? reinterpret_cast<float *>(part) : lg;
@@ -1275,10 +1339,13 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
         // exponents in the hsum region, one item list, 8-byte pairs over the
         // token and slot regions)
         static_assert(kPfSlot == kPfTok + 1, "the pairs span two adjacent regions");
-        const MidArgs m{L->router, L->router_bias, g, x, T, has_sh ? 1 : 0, f4, lg, sel, wts, gam, x16, x16isc, ctr,
-                        reinterpret_cast<int2 *>(p_tok), items_gu, room, hid,
-                        reinterpret_cast<int8_t *>(hsum), part, partk, gg, gu, gd};
+        const MidTiles mtl{offer ? (int)max_mt : 0, nt_gu, nt_dn, items_dn,
+                           mid_cost(I, f4, mid_nt, mid_reads_once(T, E, K, f4))};
+        const MidArgs m{L->router, L->router_bias, g, x, T, has_sh ? 1 : 0, f4, lg, sel, wts, gam, x16, x16isc, xsum,
+                        x16sum, ctr, reinterpret_cast<int2 *>(p_tok), items_gu, room, hid,
+                        reinterpret_cast<int8_t *>(hsum), part, partk, gg, gu, gd, mtl};
         if (const int rc = launch_mid(m, s)) return rc;
+        if (offer) tile_gemms(true, ctr + 4, reinterpret_cast<const int2 *>(p_tok));
         hipLaunchKernelGGL(k_pf_combine_h, dim3((unsigned)(((size_t)T * H / 4 + 255) / 256)), dim3(256), 0, s, part,
                            partk, T, S, H, y, y32);
         return check_launch("prefill");
@@ -1288,20 +1355,7 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
                        items_gu, items_dn, ctr + 1, (int)(max_mt * nt_gu), (int)(max_mt * nt_dn));
     hipLaunchKernelGGL(k_pf_scatter, dim3((unsigned)(nblk + (has_sh ? (T + 255) / 256 : 0))), dim3(256), 0, s, sel,
                        wts, g ? gam : nullptr, T, K, E, has_sh ? 1 : 0, off, blk, p_tok, p_slot, p_wt);
-    const dim3 g_gu((unsigned)(max_mt * nt_gu)), g_dn((unsigned)(max_mt * nt_dn)),
-        nth(f4 ? ExpertEngineF4::NT : ExpertEngine::NT), nth_dn(f4 ? ExpertEngineF4::NT : DownEngineI8::NT);
-    if (f4) {
-        hipLaunchKernelGGL((k_pf_gemm<true, kRoutedF4>), g_gu, nth, 0, s, items_gu, ctr + 1, 0, p_tok, p_slot,
-                           p_wt, x, H, I, gg, gu, E, hid, part, partk, H, nt_gu, xsum, hsum, nt_gu, nullptr);
-        hipLaunchKernelGGL((k_pf_gemm<false, kRoutedF4>), g_dn, nth, 0, s, items_dn, ctr + 1, 1, p_tok, p_slot,
-                           p_wt, hid, I, H, gd, gd, E, hid, part, partk, H, nt_dn, xsum, hsum, nt_gu, nullptr);
-    } else {
-        hipLaunchKernelGGL((k_pf_gemm<true, kAllI8>), g_gu, nth, 0, s, items_gu, ctr + 1, 0, p_tok, p_slot, p_wt,
-                           reinterpret_cast<const uint16_t *>(x16), H, I, gg, gu, E, hid, part, partk, H, nt_gu, x16sum, hsum,
-                           nt_gu, x16isc);
-        hipLaunchKernelGGL((k_pf_gemm<false, kDownI8>), g_dn, nth_dn, 0, s, items_dn, ctr + 1, 1, p_tok, p_slot, p_wt,
-                           hid, I, H, gd, gd, E, hid, part, partk, H, nt_dn, xsum, hsum, nt_gu, nullptr);
-    }
+    tile_gemms(false, ctr + 1, nullptr);
     hipLaunchKernelGGL(k_pf_combine_h, dim3((unsigned)(((size_t)T * H / 4 + 255) / 256)), dim3(256), 0, s, part, partk,
                        T, S, H, y, y32);
     return check_launch("prefill");

@@ -89,6 +89,40 @@ inline int mid_items_bound(int T, int E, int K, bool has_sh, int token_tiles) {
     return (E < tk ? E : tk) + tk / mt + (has_sh ? (T + mt - 1) / mt : 0);
 }
 
+constexpr int kPfTileRows = 128;       // rows of a tile of the grouped GEMMs
+
+// The largest call of the middle path, in rows; at another top_k than 10 also in
+// pairs, as it is an expert's rows that decide. us per layer, the middle path /
+// 128-row tiles: 2048/512 INT8 1500 rows 507 / 620, 2560/640 INT8 1500 rows 841 /
+// 932, NVFP4 2048/512 458 / 686, 2560/640 723 / 991; it grows by 0.13, 0.30, 0.19
+// and 0.28 us a row, the tiles by 0.04 to 0.07. Top-16, 2800 rows of 2048/512:
+// INT8 940 / 737, NVFP4 1059 / 784.
+constexpr int mid_rows_max(int I, bool f4) { return I <= 512 ? 2800 : f4 ? 2500 : 1800; }
+inline bool mid_takes(int T, int K, int I, bool f4) {
+    return T <= mid_rows_max(I, f4) && T * K <= 10 * mid_rows_max(I, f4);
+}
+
+// Few rows an expert: weights read once, nontemporal (the figures are at ld_w).
+inline bool mid_reads_once(int T, int E, int K, bool f4) { return T * K / E < (f4 ? 8 : 12); }
+
+// Which form of the expert GEMMs a middle call runs is known once the selection
+// is: a router that crowds its rows on few experts makes many items of one
+// expert, and each reads and converts its weights again, where a 128-row tile
+// does it once. From mid_offers_tiles on the tile GEMMs are launched behind the
+// middle ones, and k_mid_plan leaves one pair of them without work (2.5 us each):
+// the tiles run where tiles * tile + base < groups * group + (items - groups) *
+// item, in units of 10 ns (groups: experts with a row, items: mid_token_tiles).
+// Fitted to calls of both forms with router biases of spread 0 to 3 and with all
+// rows on ten experts, 256 to 2800 rows; the choice is within 2% of the faster
+// form in 363 of 368 of them and within 11% in all.
+struct MidCost { int group, item, tile, base; };
+inline bool mid_offers_tiles(int T, int I) { return T >= (I > 512 ? 256 : 384); }
+inline MidCost mid_cost(int I, bool f4, int token_tiles, bool once) {
+    if (f4) return I > 512 ? MidCost{0, 30, 99, 1000} : MidCost{0, 18, 68, 1300};
+    if (I > 512) return once ? MidCost{0, 54, 67, 2400} : MidCost{0, 31, 65, 1700};
+    return token_tiles > 1 ? MidCost{45, 58, 68, -800} : once ? MidCost{10, 30, 50, 2000} : MidCost{0, 19, 41, 2200};
+}
+
 // Slices of H in the router GEMM. Few m-tiles do not fill the chip, so K is cut
 // (1021 rows: 31 -> 13 us in four). One slice writes the logits' own region;
 // more lie in the partials' region (part_bytes), which the down GEMM writes

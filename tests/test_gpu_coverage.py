@@ -257,6 +257,75 @@ def test_middle_rows_upper_edge(lib, fmt):
     st.destroy()
 
 
+def _gemm_blocks(sel, T, hidden, inter, fmt, shared, tiles):
+    """Blocks of gate/up and down work of a call with this selection: the middle
+    path's items, or 128-row tiles."""
+    cnt = np.bincount(sel.ravel(), minlength=E)
+    four = fmt == 0 and inter <= 512 and sel.size // E >= 24
+    per = 128 if tiles else 64 if four else 16
+    n = int((-(-cnt // per)).sum()) + (-(-T // per) if shared else 0)
+    if tiles:
+        return [n * (inter // 128), n * (hidden // (256 if fmt else 128))]
+    return [n * (inter // 64), n * (hidden // (512 if four else 256))]
+
+
+@pytest.mark.parametrize("hidden,inter,T,fmt,k,shared,gated,tiles", [
+    (2560, 640, 256, 0, 10, True, 1, True), (2560, 640, 257, 1, 10, True, 0, True), (2560, 640, 255, 0, 10, True, 1, False),
+    (2048, 512, 384, 1, 10, False, 1, True), (2048, 512, 511, 0, 10, True, 1, True), (2048, 512, 640, 0, 4, True, 0, True),
+    (2560, 640, 769, 0, 10, False, 1, True), (2560, 640, 895, 1, 16, True, 1, True), (2048, 512, 1281, 0, 10, True, 1, True),
+    (2048, 512, 1281, 1, 10, True, 1, True)])
+def test_middle_rows_crowded(lib, hidden, inter, T, fmt, k, shared, gated, tiles):
+    """Middle calls whose rows all go to the same k experts (a router bias of +64
+    on them): from 256 (2560/640) or 384 rows on the plan leaves such a call to the
+    128-row tiles, read from its own pairs; the groups hold T rows each, whole
+    tiles, one row more and one fewer. Below, items of 16 rows. The counters say
+    which ran. Up to 600 rows the row sums of x that the tiles correct their offsets
+    with come from k_mid_router, beyond from the MFMA router's prep launch.
+    Routing bit-exact, y within TOL of the grouped fp64 oracle; the second of two
+    calls on one workspace repeats the first bit for bit after a call with spread
+    rows in between."""
+    _say("middle rows crowded H", hidden, "T", T, "fmt", fmt, "K", k, "shared", shared, "gated", gated)
+    qfm.init(hidden, inter, E, k, 1, gated)
+    st = qfm.Stream()
+    seed, layer, xl = 4, 23, 92
+    L = qfm.SynthLayer(fmt, seed, layer, with_bias=True, stream=st)
+    st.sync()
+    bias = np.full(E, -64.0, np.float32)
+    bias[100:100 + k] = 64.0 + np.arange(k, dtype=np.float32) * 0.25
+    dbias = qfm.DevBuf.from_array(bias)
+    lay = qfm.QfmLayer.from_buffer_copy(L.s.layer)
+    if not shared:
+        lay.sh_gate, lay.sh_up, lay.sh_down, lay.sh_gate_inp = qfm.Qf8I8Mat(), qfm.Qf8I8Mat(), qfm.Qf8I8Mat(), None
+    x = orc.fill("gauss_bf16", seed, xl, orc.T_X, 0, T * hidden).reshape(T, hidden)
+    dx, dy = qfm.DevBuf.from_array(x), qfm.DevBuf(T * hidden * 2)
+    wsb = lib.qfm_workspace_bytes(T)
+    ws = qfm.DevBuf(wsb)
+    view = qfm.QfmWsView()
+    ys = []
+    for crowd in (True, False, True):
+        lay.router_bias = dbias.ptr if crowd else None
+        qfm.check(lib.qfm_moe_forward(C.byref(lay), dx.ptr, T, dy.ptr, ws.ptr, wsb, st.h), "forward")
+        st.sync()
+        lib.qfm_workspace_view(ws.ptr, T, C.byref(view))
+        sel = qfm.d2h(view.sel, np.int32, (T, k))
+        counters = qfm.d2h(view.counters, np.int32, 3).tolist()
+        assert counters[1:] == _gemm_blocks(sel, T, hidden, inter, fmt, shared, tiles and crowd), (crowd, counters)
+        ys.append(dy.download(np.uint16, (T, hidden)))
+    zero = None if shared else (np.zeros((inter, hidden)), np.zeros((inter, hidden)), np.zeros((hidden, inter)))
+    r = orc.moe_layer_grouped(hidden, inter, E, k, T, seed, layer, xl, use_bias=1, x=x, fmt=fmt, bias=bias, gated=gated,
+                              shared=zero)
+    assert np.array_equal(sel, r["sel"]) and set(np.unique(sel)) == set(range(100, 100 + k))
+    assert np.allclose(qfm.d2h(view.wts, np.float32, (T, k)), r["w"], rtol=2e-6, atol=1e-7)
+    y = orc.bf16_to_f32(ys[0])
+    rel = max(_rel(y[t], r["y"][t]) for t in range(T))
+    _say("  max rel err", rel)
+    assert rel <= TOL
+    assert np.array_equal(ys[0], ys[2])
+    L.destroy()
+    st.destroy()
+    qfm.init(H, I, E, K, 1, 1)
+
+
 # ------------------------------------------------------------------ fork rows sharing experts
 @pytest.mark.parametrize("M,fmt,boost", [(2, 0, 64.0), (8, 0, 64.0), (8, 1, 64.0), (8, 0, 1.5), (5, 1, 1.5)])
 def test_fork_rows_sharing_experts(lib, M, fmt, boost):

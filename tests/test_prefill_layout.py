@@ -209,6 +209,37 @@ def test_middle_items_never_exceed_their_bound(shim, H, I, f4, top):
                     assert items <= bound, (K, T, has_sh, items, bound)
 
 
+@pytest.mark.parametrize("H,I,f4,top", [(2048, 512, 0, 2800), (2048, 512, 1, 2800), (2560, 640, 0, 1800),
+                                        (2560, 640, 1, 2500)])
+def test_middle_path_by_pairs_and_routing(shim, H, I, f4, top):
+    """The middle path ends at `top` rows and, at a larger top_k, at as many pairs
+    as top-10 makes there. Inside, a plan that takes the 128-row tiles fits their
+    work lists whatever the routing, rows crowded on ten experts take them (from
+    the first call that offers them on), and evenly spread rows take the items up
+    to the largest call."""
+    E = 512
+    rng = np.random.default_rng(8)
+    first = 256 if I > 512 else 384
+    assert shim.mid_takes_c(top, 10, I, f4) and not shim.mid_takes_c(top + 1, 10, I, f4)
+    assert shim.mid_takes_c(top, 1, I, f4) and not shim.mid_takes_c(top + 1, 1, I, f4)
+    assert shim.mid_takes_c(10 * top // 16, 16, I, f4) and not shim.mid_takes_c(10 * top // 16 + 1, 16, I, f4)
+    assert not shim.mid_offers_tiles_c(first - 1, I) and shim.mid_offers_tiles_c(first, I)
+    for T in (first, 600, 601, 1229, top):
+        for K in (10, 16):
+            if not shim.mid_takes_c(T, K, I, f4):
+                continue
+            m = layout(shim, T, H, I, E, K, True, GU_F4 if f4 else GU_I8, GU_F4 if f4 else DN_I8)[2]
+            mt = 16 * shim.mid_token_tiles_c(T, E, K, I, f4)
+            ten, even = np.zeros(E, np.int64), np.full(E, T * K // E, np.int64)
+            ten[:K], even[:T * K % E] = T, T * K // E + 1
+            for cnt in [ten, even] + _routings(T, K, E, rng):
+                g = np.append(cnt, T)
+                n = [int((-(-g // per)).sum()) for per in (mt, BM)]
+                assert n[1] <= m["max_mt"]
+                pick = shim.mid_picks_tiles_c(int((g > 0).sum()), n[0], n[1], T, E, K, I, f4)
+                assert pick if cnt is ten else not pick if cnt is even else True, (T, K, n)
+
+
 @pytest.mark.parametrize("H,I,f4", [(2048, 512, 0), (2048, 512, 1), (2560, 640, 0), (2560, 640, 1)])
 def test_selection_waves_never_share_a_logits_buffer(shim, H, I, f4):
     """k_pf_select reads the router GEMM's slices and stores their sum plus the
