@@ -604,22 +604,23 @@ __device__ __forceinline__ uint32_t wave_kth_key(const uint32_t (&key)[EPL], con
 // Candidates, exact logits, exact top-K and the shared gate, WPT waves per
 // token. lg_part: the router GEMM's nks partial logits [nks][T][E], summed in
 // slice order; their sum goes to lg, which may be lg_part itself where nks and
-// WPT are 1 (pf_select_split): neither is __restrict__. Every wave of a token forms the bounds and
-// the candidate list itself (no barrier) and recomputes every WPT-th candidate;
-// the first wave ranks them. tau, a lower bound of the K-th largest logit, is
-// the K-th largest lower bound: first the K-th largest of the 64 lane maxima
-// (one rank pass instead of K wave-wide maxima; K distinct experts reach it),
-// then, where more than K experts reach that, the K-th largest among those.
-// The second pass matters where a router's hot experts agree modulo 64 (a lane
-// holds experts e, e + 64, ..): every candidate is a router row of 8 or 10 KiB,
-// and past 64 of them a token recomputes all 512 (32 hot experts in four lanes,
-// top-16: 2048/512 INT8 8038 rows 1909 -> 1386 us a call, 2560/640 NVFP4 4000
-// rows 1581 -> 1086; evenly spread experts the same with and without). One wave per token is bound by its chain of L2 round trips
+// WPT are 1 (pf_select_split): neither is __restrict__. Every wave of a token
+// forms the bounds and the candidate list itself (no barrier) and recomputes
+// every WPT-th candidate; the first wave ranks them. tau, a lower bound of the
+// K-th largest logit, is the K-th largest lower bound: first the K-th largest of
+// the 64 lane maxima (one rank pass instead of K wave-wide maxima; K distinct
+// experts reach it), then, where more than K experts reach that, the K-th
+// largest among those. The second pass matters where a router's hot experts
+// agree modulo 64 (a lane holds experts e, e + 64, ..): every candidate is a
+// router row of 8 or 10 KiB, and past 64 of them a token recomputes all 512 (32
+// hot experts in four lanes, top-16: 2048/512 INT8 8038 rows 1909 -> 1386 us a
+// call, 2560/640 NVFP4 4000 rows 1581 -> 1086; evenly spread experts the same
+// with and without). One wave per token is bound by its chain of L2 round trips
 // while the tokens do not fill the chip: four waves take up to kSelectSplitRows
 // (450 / 1021 / 1500 rows 19 / 23 / 36 us; K wave-wide maxima and one wave a
 // token: 25 / 30 / 31 us; 8038 rows one wave 76 -> 68 us).
 template <int NJ, int WPT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 4)
 k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, const float *__restrict__ bias,
             const float *__restrict__ g, const float *lg_part, int nks, float *lg, const float *__restrict__ xnorm,
             const float *__restrict__ wnorm, int K, int renorm, int *__restrict__ sel, float *__restrict__ wts,
@@ -701,31 +702,52 @@ k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, 
     }
     if (overflow && w == 0 && lane == 0) atomicAdd(n_fallback, 1);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int nc = full ? E : total;
     float xv[NJ][4];                                     // this token's x slice, canonical lane layout
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const u32x2_t p = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t *>(xt + j * 256 + lane * 4));
         xv[j][0] = bf16_lo(p.x); xv[j][1] = bf16_hi(p.x); xv[j][2] = bf16_lo(p.y); xv[j][3] = bf16_hi(p.y);
     }
-    constexpr int CB = 4;                                // candidates per batch of loads
-    for (int c0 = w; c0 < nc; c0 += CB * WPT) {
-        int eb[CB];
+    if (full) {
+        // every expert: one router row after the other, each of its loads replaced
+        // by the next row's as soon as it is used. A wave that recomputes all 512 is
+        // bound by the loads it has in flight; in one loop with the candidates below
+        // they were about 4 of 40, and a single such token kept a call of 2560/640
+        // NVFP4 and top-16 waiting (1200 / 2000 rows 1124 / 1423 us, 924 / 1227 so)
+        const float *wr = W + (size_t)w * H + lane * 4;
+        float4 wv[NJ];
 #pragma unroll
-        for (int q = 0; q < CB; q++) {
-            const int c = c0 + q * WPT < nc ? c0 + q * WPT : c0;   // past the end: repeat a candidate, result dropped
-            eb[q] = full ? c : s_cand[wave][c];
+        for (int j = 0; j < NJ; j++) wv[j] = *reinterpret_cast<const float4 *>(wr + j * 256);
+#pragma unroll 1
+        for (int c = w; c < E; c += WPT) {
+            if (c + WPT < E) wr += (size_t)WPT * H;      // (the last row: read again)
+            float a = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                a = __fmaf_rn(wv[j].x, xv[j][0], a);
+                a = __fmaf_rn(wv[j].y, xv[j][1], a);
+                a = __fmaf_rn(wv[j].z, xv[j][2], a);
+                a = __fmaf_rn(wv[j].w, xv[j][3], a);
+                wv[j] = *reinterpret_cast<const float4 *>(wr + j * 256);
+            }
+            a = canon_butterfly(a);
+            if (lane == 0) s_lg[tb][c] = bias ? __fadd_rn(a, bias[c]) : a;
         }
-        float lb[CB];
-        canon_dot_wave_batch<NJ, CB>(W, H, eb, xv, lane, lb);
+    } else {
+        constexpr int CB = 4;                            // candidates per batch of loads
+        for (int c0 = w; c0 < total; c0 += CB * WPT) {
+            int eb[CB];
 #pragma unroll
-        for (int q = 0; q < CB; q++) {
-            const int c = c0 + q * WPT;
-            if (c >= nc) break;
-            const float v = bias ? __fadd_rn(lb[q], bias[eb[q]]) : lb[q];
-            if (lane == 0) {
-                if (full) s_lg[tb][c] = v;
-                else s_key[tb][c] = topk_key(v, eb[q]);
+            for (int q = 0; q < CB; q++)                 // past the end: repeat a candidate, result dropped
+                eb[q] = s_cand[wave][c0 + q * WPT < total ? c0 + q * WPT : c0];
+            float lb[CB];
+            canon_dot_wave_batch<NJ, CB>(W, H, eb, xv, lane, lb);
+#pragma unroll
+            for (int q = 0; q < CB; q++) {
+                const int c = c0 + q * WPT;
+                if (c >= total) break;
+                const float v = bias ? __fadd_rn(lb[q], bias[eb[q]]) : lb[q];
+                if (lane == 0) s_key[tb][c] = topk_key(v, eb[q]);
             }
         }
     }
