@@ -616,9 +616,9 @@ __device__ __forceinline__ uint32_t wave_kth_key(const uint32_t (&key)[EPL], con
 // hot experts in four lanes, top-16: 2048/512 INT8 8038 rows 1909 -> 1386 us a
 // call, 2560/640 NVFP4 4000 rows 1581 -> 1086; evenly spread experts the same
 // with and without). One wave per token is bound by its chain of L2 round trips
-// while the tokens do not fill the chip: four waves take up to kSelectSplitRows
-// (450 / 1021 / 1500 rows 19 / 23 / 36 us; K wave-wide maxima and one wave a
-// token: 25 / 30 / 31 us; 8038 rows one wave 76 -> 68 us).
+// while the tokens do not fill the chip: four waves there (pf_select_split has
+// the figures; K wave-wide maxima in place of the rank pass took 76 us for 8038
+// rows, 68 now).
 template <int NJ, int WPT>
 __global__ void __launch_bounds__(256, 4)
 k_pf_select(const uint16_t *__restrict__ x, int T, const float *__restrict__ W, const float *__restrict__ bias,
@@ -1342,7 +1342,7 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
         hipLaunchKernelGGL(k_pf_router_prep, dim3((unsigned)(E + (T + 3) / 4)), dim3(256), 0, s, L->router, E, H, wnorm,
                            wb16, x, T, xnorm, xsum, mid || !f4 ? x16 : nullptr, x16sum, x16isc, ctr);
         const int nks = pf_router_slices(T, E, Lw.bytes[kPfPart]);
-        const bool split = pf_select_split(T, nks);
+        const bool split = pf_select_split(T, H, nks);
         float *lgp = nks > 1 ? reinterpret_cast<float *>(part) : lg;
         const int mt_router = ((T + BM - 1) / BM + 7) / 8 * 8;
         hipLaunchKernelGGL(k_pf_router_mfma, dim3(mt_router * (E / BN), nks), dim3(256), 0, s, x, T, H, wb16, E, lgp);

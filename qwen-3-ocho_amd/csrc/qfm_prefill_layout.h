@@ -132,11 +132,14 @@ inline int pf_router_slices(int T, int E, size_t part_bytes) {
     return T <= 2048 && room >= 4 ? 4 : T <= 4096 && room >= 2 ? 2 : 1;
 }
 
-// Four waves a token in k_pf_select, else one: up to kSelectSplitRows rows (the
-// figures are there), and only where its input and output logits are two
-// buffers: with one slice they are the same, and a wave would read logits that
-// another wave of its token has already stored with the bias added.
-constexpr int kSelectSplitRows = 1100;
-inline bool pf_select_split(int T, int slices) { return T <= kSelectSplitRows && slices > 1; }
+// Four waves a token in k_pf_select (a block each), else one: while the blocks of
+// all tokens are resident at once, 4 on each of the 256 CUs, and at H = 2560,
+// whose rows leave less latency to hide, up to 800 (us at 700 / 900 / 1024 / 1025
+// rows: 2048 four waves 21.3 / 23.2 / 22.6 / 27.3, one 25.6 / 24.6 / 22.4 / 22.6;
+// 2560 four 22.7 / 27.0 / 27.4 / 29.8, one 25.2 / 25.2 / 25.0 / 25.1). Only where
+// its input and output logits are two buffers: with one slice they are the same,
+// and a wave would read logits that another wave of its token has already stored
+// with the bias added.
+inline bool pf_select_split(int T, int H, int slices) { return T <= (H == 2048 ? 1024 : 800) && slices > 1; }
 
 }  // namespace qfm

@@ -18,7 +18,7 @@ extern "C" int pf_layout_c(int T, int H, int I, int E, int K, int has_sh, int gu
 extern "C" int pf_router_slices_c(int T, int E, unsigned long long part_bytes) {
     return qfm::pf_router_slices(T, E, part_bytes);
 }
-extern "C" int pf_select_split_c(int T, int slices) { return qfm::pf_select_split(T, slices); }
+extern "C" int pf_select_split_c(int T, int H, int slices) { return qfm::pf_select_split(T, H, slices); }
 extern "C" int mid_token_tiles_c(int T, int E, int K, int I, int f4) { return qfm::mid_token_tiles(T, E, K, I, f4 != 0); }
 extern "C" int mid_items_bound_c(int T, int E, int K, int has_sh, int token_tiles) {
     return qfm::mid_items_bound(T, E, K, has_sh != 0, token_tiles);

@@ -247,15 +247,15 @@ def test_selection_waves_never_share_a_logits_buffer(shim, H, I, f4):
     same token would race with the first one's stores: four waves a token only
     over two or more slices, and those fit the region that they borrow."""
     E = 512
-    assert not any(shim.pf_select_split_c(T, 1) for T in range(9, 2000))
+    assert not any(shim.pf_select_split_c(T, H, 1) for T in range(9, 2000))
     for K in (1, 2, 9, 10, 16):
         for has_sh in (True, False):
-            for T in [9, 600, 601, 1023, 1024, 1025, 1100, 1101, 2047, 2048, 2049, 4095, 4096, 4097, 16384]:
+            for T in [9, 600, 601, 800, 801, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 16384]:
                 off, by, m = layout(shim, T, H, I, E, K, has_sh, GU_F4 if f4 else GU_I8, GU_F4 if f4 else DN_I8)
                 part, lg = by[NAMES.index("part")], by[NAMES.index("lg")]
                 n = shim.pf_router_slices_c(T, E, C.c_ulonglong(int(part)))
                 assert n in (1, 2, 4) and n * T * E * 4 <= (part if n > 1 else lg)
-                assert not shim.pf_select_split_c(T, n) or n > 1
+                assert not shim.pf_select_split_c(T, H, n) or n > 1
 
 
 def test_library_sizes_match_the_layout(shim):
