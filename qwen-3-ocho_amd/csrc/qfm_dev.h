@@ -332,7 +332,6 @@ __device__ float group_max(float v) {
 }
 
 // ---- wave-wide reductions from the ROCm device library (ockl) -------------
-extern "C" __device__ __attribute__((const)) unsigned long long __ockl_wfred_max_u64(unsigned long long);
 extern "C" __device__ __attribute__((const)) float __ockl_wfred_add_f32(float);
 
 // Order-preserving 64-bit selection key of a logit: descending value, ties to

@@ -39,7 +39,7 @@ int launch_fill_f32(float *out, uint64_t cnt, float value, hipStream_t s);
 struct ShPtrs { const int8_t *qg, *qu, *qd; const float *sg, *su, *sd; };
 
 // router: W_f32 [E][H] (+ row g [H] written at column E when g != nullptr)
-// and, when sh != nullptr, the shared-expert hidden hsh[m * ld_hsh + r], in one launch.
+// and, when sh != nullptr (M > 1), the shared-expert hidden hsh[m * ld_hsh + r], in one launch.
 // With x16 != nullptr (M = 1) the launch also writes x as scaled fp16 (H / 8
 // 16-byte words) followed by a float2 (sum of the scaled values, 2^-k).
 // With tail != nullptr (2 <= M <= kTailRows, E = 512, no x16) the launch also
@@ -171,8 +171,9 @@ struct MidArgs {
 };
 int launch_mid(const MidArgs &a, hipStream_t s);
 
-// Prefill (T > 8 rows): MFMA router + exact candidate selection, grouped
-// MFMA gate/up and down over the routing inversion, owned-partial combine.
+// Every call of more than 8 rows: above kMidExactRows the MFMA router with exact
+// candidate selection; the middle path, or grouped MFMA gate/up and down over the
+// routing inversion; owned-partial combine.
 size_t prefill_ws_bytes(int T);
 // y[t] = sum of the S owned partial slots part[t*S + k][H] in slot order (bf16 out,
 // or fp32 into y32 when y32 != nullptr)

@@ -1,4 +1,7 @@
-// qfm_prefill.hip -- prefill (T tokens, T large): MFMA grouped GEMMs.
+// qfm_prefill.hip -- prefill (T tokens, T large): MFMA grouped GEMMs. The router
+// and selection serve every call above kMidExactRows rows, the experts' launches
+// the calls that the middle path (qfm_mid.hip) does not take or whose plan leaves
+// them to these tiles.
 //
 // Reference behaviour: the chunk path qf8_i8_experts_chunk
 // (ocho/amd_server/qf8_moe_i8.hip:196-322, :372-395) and Spark's
@@ -16,7 +19,7 @@
 //                      c * ||w_e|| ||x_t|| (Cauchy-Schwarz over the bf16
 //                      rounding of W, the MFMA accumulation and the canonical
 //                      fp32 order; constants below).
-//   k_pf_select        one wave per token: tau = K-th largest (logit~ - B),
+//   k_pf_select        one or four waves per token: tau = K-th largest (logit~ - B),
 //                      candidates = {e : logit~ + B >= tau} (a superset of the
 //                      exact top-K, ties included), their logits recomputed in
 //                      the canonical order, then the exact top-K among them;
@@ -514,25 +517,9 @@ k_pf_router_mfma(const uint16_t *__restrict__ x, int T, int H, const uint16_t *_
             }
 }
 
-// canonical-order dot of one router row with one token, computed by a full wave
-template <int NJ>
-__device__ __forceinline__ float canon_dot_wave(const float *__restrict__ w, const uint16_t *__restrict__ x, int lane) {
-    float a = 0.0f;
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const float4 wv = *reinterpret_cast<const float4 *>(w + j * 256 + lane * 4);
-        const uint2 p = *reinterpret_cast<const uint2 *>(x + j * 256 + lane * 4);
-        a = __fmaf_rn(wv.x, bf16_lo(p.x), a);
-        a = __fmaf_rn(wv.y, bf16_hi(p.x), a);
-        a = __fmaf_rn(wv.z, bf16_lo(p.y), a);
-        a = __fmaf_rn(wv.w, bf16_hi(p.y), a);
-    }
-    return canon_butterfly(a);
-}
-
-// The same canonical dot for CB router rows at once (x held in registers):
+// Canonical-order dots of CB router rows with one token by a full wave (x held in registers):
 // the CB rows' loads are all in flight before the first multiply and the CB
-// fma chains and butterflies are independent. Each dot keeps the order above.
+// fma chains and butterflies are independent. Each dot keeps the order of qfm_router.hip.
 template <int NJ, int CB>
 __device__ __forceinline__ void canon_dot_wave_batch(const float *__restrict__ W, int H, const int (&e)[CB],
                                                      const float (&xv)[NJ][4], int lane, float (&out)[CB]) {

@@ -37,16 +37,16 @@ __device__ __forceinline__ float canon_reduce_row(const float4 (&w)[NJ], const f
 
 // One wave per block. Blocks [0, E): router rows of W fp32 [E][H]; block E
 // (when g != nullptr): the shared-expert gate vector g [H], written to
-// column E without bias; the remaining I/2 blocks (when sh.qg != nullptr):
+// column E without bias; the remaining blocks (MR > 1, when sh.qg != nullptr):
 // two shared-expert gate/up rows each, one per half-wave, giving
 // hsh[m][r] = silu(sg_r <Qg_r, x_m>) * (su_r <Qu_r, x_m>). x is bf16 [M][H],
 // logits [M][ld]. Every output depends on x only, so one launch covers all.
 // MR rows of x are processed together: their fma chains are independent and
 // their canonical reductions share cross-lane steps (canon_reduce_rows; each
-// row keeps the canonical order). With
-// MR > 1 the shared-expert rows are also split over x rows: block (pair, mg)
-// computes rows [2 mg, 2 mg + 2) of x for its row pair, MG = ceil(M / 2) blocks
-// per pair, laid out so that one pair's blocks share an XCD (and its L2).
+// row keeps the canonical order). The shared-expert rows are also split over x
+// rows: block (pair, mg) computes rows [2 mg, 2 mg + 2) of x for its row pair,
+// MG = ceil(M / 2) blocks per pair, laid out so that one pair's blocks share an
+// XCD (and its L2).
 // With x16 != nullptr one more block (the first) writes x row 0 as scaled
 // fp16 with its (sum, 2^-k) for the M = 1 gate/up kernel.
 //
@@ -186,17 +186,13 @@ k_router_shared(const float *__restrict__ W, const float *__restrict__ bias, con
         }
         return;
     }
+    if constexpr (MR == 1) return;              // (one row's shared expert is the last job of its gate/up launch)
     // shared-expert gate/up rows
     constexpr int NST = H / 512;
     const int l = lane & 31;
     const int sb = b - E - ng;
-    int pair = sb, mlo = 0, mhi = M;
-    if (MR > 1) {
-        const int MG = (M + 1) / 2, t = sb >> 3, mg = t % MG;
-        pair = (t / MG) * 8 + (sb & 7);
-        mlo = mg * 2;
-        mhi = min(M, mlo + 2);
-    }
+    const int MG = (M + 1) / 2, t = sb >> 3, mg = t % MG, pair = (t / MG) * 8 + (sb & 7);
+    const int mlo = mg * 2, mhi = min(M, mlo + 2);
     const int r = pair * 2 + (lane >> 5);
     uint4 wg[NST], wu[NST];
 #pragma unroll
@@ -205,7 +201,7 @@ k_router_shared(const float *__restrict__ W, const float *__restrict__ bias, con
         wu[st] = ld_nt16(sh.qu + (size_t)r * H + st * 512 + l * 16);
     }
     const float sg = sh.sg[r], su = sh.su[r];
-    constexpr int SR = MR > 1 ? 2 : 1;          // x rows per pass of the shared rows
+    constexpr int SR = 2;                       // x rows per pass of the shared rows
     for (int m0 = mlo; m0 < mhi; m0 += SR) {
         float ag[SR], au[SR];
 #pragma unroll
@@ -278,7 +274,7 @@ int launch_router_shared(const float *W, const float *bias, const float *g, cons
                          const uint16_t *x, int M, float *logits, int ld, float *hsh, int ldh, hipStream_t s,
                          void *x16, const RouteTail *tail) {
     const int E = g_cfg.E, I = g_cfg.I;
-    if (sh && !hsh) { set_error(-1, "router: shared rows need an output"); return -1; }
+    if (sh && (!hsh || M == 1)) { set_error(-1, "router: shared rows need an output and more than one row"); return -1; }
     if (x16 && M != 1) { set_error(-1, "router: the fp16 x row is for M = 1"); return -1; }
     if (tail && (x16 || E != 512 || M > kTailRows || !tail->lw || !tail->ctl || !tail->sel || !tail->wts ||
                  tail->K < 1 || tail->K > 16 || (!tail->xh) != (!tail->xci))) {
@@ -288,7 +284,7 @@ int launch_router_shared(const float *W, const float *bias, const float *g, cons
     if (sh) sp = *sh;
     uint4 *xh = static_cast<uint4 *>(x16);
     float2 *xi = xh ? reinterpret_cast<float2 *>(xh + g_cfg.H / 8) : nullptr;
-    int nblk = E + (g ? 1 : 0) + (sh ? (I / 2) * (M == 1 ? 1 : (M + 1) / 2) : 0) + (xh ? 1 : 0);
+    int nblk = E + (g ? 1 : 0) + (sh ? (I / 2) * ((M + 1) / 2) : 0) + (xh ? 1 : 0);
     RouteTail tl{};
     const int tail0 = nblk - (xh ? 1 : 0);           // first tail block (counted without the fp16-row block)
     if (tail) {
@@ -312,7 +308,7 @@ int launch_router_shared(const float *W, const float *bias, const float *g, cons
         if (M == 1) { QFM_ROUTER1(8, 512); }
         else if (M <= 4) { QFM_ROUTER(8, 512, 4); }
         else { QFM_ROUTER(8, 512, 8); }
-    } else if (shape_shard() && M == 1 && !sh && !tail) {
+    } else if (shape_shard() && M == 1 && !tail) {
         QFM_ROUTER1(8, 64);
     } else if (shape_2560()) {
         if (M == 1) { QFM_ROUTER1(10, 640); }
