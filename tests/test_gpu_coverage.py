@@ -1,19 +1,23 @@
 """GPU parity on the edge cases of the decode formats and the selection:
 
 * X8 quantization on exact ties (v = (k + 1/2) s): round half to even, bit-exact;
-* prefill tokens whose x row is zero: every expert is a candidate (the
-  candidate-overflow fallback), ties go to the lowest expert index, and the
-  workspace counter reports those tokens;
+* middle-row tokens whose x row is zero: every expert is a candidate (the exact
+  form of the ranking's bound), ties go to the lowest expert index, and the
+  workspace counter reports those tokens (the MFMA router's own overflow:
+  test_gpu_routing.py);
+* middle rows around whole items, crowded on few experts (the 128-row tiles then
+  take them) and at their upper edge, and the 128-row tiles' own path from its
+  shortest calls on, at both shapes;
 * fork rows (M <= 8) whose experts coincide, all rows on the same ten experts
   or a mix of shared and private ones (each distinct expert's pair range
   staged past its first two rows);
-* prefill selection on constructed near-ties: router rows whose bf16 roundings
-  coincide, so the MFMA logits cannot order them and only the exact
-  recomputation does;
+* selection on constructed near-ties: router rows whose bf16 roundings coincide
+  (here at 33 rows through the exact router; through the MFMA logits, which cannot
+  order them: test_gpu_routing.py);
 * every E4M3 block-scale byte 0x00..0xFF (bytes >= 0x80 are large unsigned
   scales, 0x7F is +inf, as the reference decodes them) through every NVFP4
-  decode path: the fused fork-row kernels, the prefill grouped GEMMs and the
-  reference-named M=1 / M=8 tiers, against the oracle's dequantization of the
+  path: the fused fork-row kernels, the middle rows' items, the 128-row tiles and
+  the reference-named M=1 / M=8 tiers, against the oracle's dequantization of the
   same codes and scale bytes.
 """
 import ctypes as C
@@ -90,14 +94,14 @@ def test_x8_ties_bit_exact(lib):
     assert np.array_equal(gq[1:1 + ties.size], np.rint(ties).astype(np.int8))
 
 
-# ------------------------------------------------------------------ prefill: zero rows
+# ------------------------------------------------------------------ middle rows: zero rows
 @pytest.mark.parametrize("bias", [False, True])
 def test_prefill_zero_rows_fallback(lib, bias):
-    """Zero x rows: without a router bias every approximate logit is 0, all 512
-    experts become candidates (the overflow fallback), the exact logits are all
-    0 and the selection is experts 0..9 (ties to the lower index) with equal
-    weights; the counter reports exactly those rows. With a bias the logits are
-    the bias values and the selection is their top 10."""
+    """Zero x rows of a middle call (k_mid_topk): without a router bias every logit
+    is 0, all 512 experts share the ranking's prefix bound (its exact form), and the
+    selection is experts 0..9 (ties to the lower index) with equal weights; the
+    counter reports exactly those rows. With a bias the logits are the bias values
+    and the selection is their top 10."""
     T, seed, layer, xl = 40, 2, 31, 77
     zero = [0, 5, 17, 39]
     _say("prefill zero rows, bias", bias)
@@ -129,10 +133,11 @@ def test_prefill_zero_rows_fallback(lib, bias):
 def test_prefill_tile_boundaries(lib, T, fmt):
     """A router bias of +64 on experts 100..109 (and -64 elsewhere) sends every
     token to exactly those ten experts: eleven groups (with the shared one) of
-    T rows each, i.e. exactly full 128-row tiles (T = 128, 256), one spare row
-    (129), or 127 rows over (383), and 502 experts with no rows at all. Routing
-    bit-exact and every output row against the grouped fp64 oracle given the
-    same bias."""
+    T rows each, i.e. whole 16-row items (T = 128, 256), one spare row (129), or 15
+    rows over (383), and 502 experts with no rows at all (the 128-row tiles of such
+    calls begin at 384 rows: test_middle_rows_crowded, test_tiles_beyond_middle).
+    Routing bit-exact and every output row against the grouped fp64 oracle given
+    the same bias."""
     seed, layer, xl = 4, 23, 91
     _say("prefill tile boundaries T", T, "fmt", fmt)
     qfm.init(H, I, E, K, 1, 1)
@@ -281,9 +286,9 @@ def test_middle_rows_crowded(lib, hidden, inter, T, fmt, k, shared, gated, tiles
     tiles, one row more and one fewer. Below, items of 16 rows. The counters say
     which ran. Up to 600 rows the row sums of x that the tiles correct their offsets
     with come from k_mid_router, beyond from the MFMA router's prep launch.
-    Routing bit-exact, y within TOL of the grouped fp64 oracle; the second of two
-    calls on one workspace repeats the first bit for bit after a call with spread
-    rows in between."""
+    Routing bit-exact, y within TOL of the grouped fp64 oracle; crowded calls and
+    calls with spread rows in turn on one workspace, each repeats its first result
+    bit for bit."""
     _say("middle rows crowded H", hidden, "T", T, "fmt", fmt, "K", k, "shared", shared, "gated", gated)
     qfm.init(hidden, inter, E, k, 1, gated)
     st = qfm.Stream()
@@ -302,7 +307,7 @@ def test_middle_rows_crowded(lib, hidden, inter, T, fmt, k, shared, gated, tiles
     ws = qfm.DevBuf(wsb)
     view = qfm.QfmWsView()
     ys = []
-    for crowd in (True, False, True):
+    for crowd in (False, True, False, True):
         lay.router_bias = dbias.ptr if crowd else None
         qfm.check(lib.qfm_moe_forward(C.byref(lay), dx.ptr, T, dy.ptr, ws.ptr, wsb, st.h), "forward")
         st.sync()
@@ -316,11 +321,57 @@ def test_middle_rows_crowded(lib, hidden, inter, T, fmt, k, shared, gated, tiles
                               shared=zero)
     assert np.array_equal(sel, r["sel"]) and set(np.unique(sel)) == set(range(100, 100 + k))
     assert np.allclose(qfm.d2h(view.wts, np.float32, (T, k)), r["w"], rtol=2e-6, atol=1e-7)
-    y = orc.bf16_to_f32(ys[0])
+    y = orc.bf16_to_f32(ys[1])
     rel = max(_rel(y[t], r["y"][t]) for t in range(T))
     _say("  max rel err", rel)
     assert rel <= TOL
-    assert np.array_equal(ys[0], ys[2])
+    assert np.array_equal(ys[0], ys[2]) and np.array_equal(ys[1], ys[3])
+    L.destroy()
+    st.destroy()
+    qfm.init(H, I, E, K, 1, 1)
+
+
+@pytest.mark.parametrize("hidden,inter,T,fmt,shared,gated,hot", [
+    (2560, 640, 1801, 0, True, 1, 10), (2560, 640, 1919, 0, True, 0, 24), (2560, 640, 2501, 1, True, 0, 24),
+    (2560, 640, 2817, 1, False, 1, 10), (2048, 512, 2944, 0, False, 1, 10), (2048, 512, 2943, 1, True, 1, 24),
+    (2048, 512, 2945, 0, True, 0, 24)])
+def test_tiles_beyond_middle(lib, hidden, inter, T, fmt, shared, gated, hot):
+    """The shortest calls of the 128-row tiles' own path (a block per tile) and
+    row counts around whole tiles, at both shapes and formats, gated, ungated and
+    without a shared expert. A bias of +64 on `hot` experts sends every row to ten
+    of them: groups of T rows (ten) or of uneven sizes, few experts for the fp64
+    oracle. The counters say that the tiles ran."""
+    _say("tiles beyond middle H", hidden, "T", T, "fmt", fmt, "shared", shared, "gated", gated, "hot", hot)
+    qfm.init(hidden, inter, E, K, 1, gated)
+    st = qfm.Stream()
+    seed, layer, xl = 4, 24, 95
+    L = qfm.SynthLayer(fmt, seed, layer, with_bias=True, stream=st)
+    st.sync()
+    bias = np.full(E, -64.0, np.float32)
+    bias[100:100 + hot] = 64.0
+    qfm.check(lib.qfm_memcpy_h2d(L.s.layer.router_bias, bias.ctypes.data, bias.nbytes), "bias")
+    lay = qfm.QfmLayer.from_buffer_copy(L.s.layer)
+    if not shared:
+        lay.sh_gate, lay.sh_up, lay.sh_down, lay.sh_gate_inp = qfm.Qf8I8Mat(), qfm.Qf8I8Mat(), qfm.Qf8I8Mat(), None
+    x = orc.fill("gauss_bf16", seed, xl, orc.T_X, 0, T * hidden).reshape(T, hidden)
+    dx, dy = qfm.DevBuf.from_array(x), qfm.DevBuf(T * hidden * 4)
+    wsb = lib.qfm_workspace_bytes(T)
+    ws = qfm.DevBuf(wsb)
+    qfm.check(lib.qfm_moe_forward_f32(C.byref(lay), dx.ptr, T, dy.ptr, ws.ptr, wsb, st.h), "forward")
+    st.sync()
+    view = qfm.QfmWsView()
+    lib.qfm_workspace_view(ws.ptr, T, C.byref(view))
+    sel = qfm.d2h(view.sel, np.int32, (T, K))
+    assert qfm.d2h(view.counters, np.int32, 3).tolist()[1:] == _gemm_blocks(sel, T, hidden, inter, fmt, shared, True)
+    zero = None if shared else (np.zeros((inter, hidden)), np.zeros((inter, hidden)), np.zeros((hidden, inter)))
+    r = orc.moe_layer_grouped(hidden, inter, E, K, T, seed, layer, xl, use_bias=1, x=x, fmt=fmt, bias=bias, gated=gated,
+                              shared=zero)
+    assert np.array_equal(sel, r["sel"])
+    assert np.allclose(qfm.d2h(view.wts, np.float32, (T, K)), r["w"], rtol=2e-6, atol=1e-7)
+    y = dy.download(np.float32, (T, hidden))
+    rel = max(_rel(y[t], r["y"][t]) for t in range(T))
+    _say("  max rel err", rel)
+    assert rel <= TOL
     L.destroy()
     st.destroy()
     qfm.init(H, I, E, K, 1, 1)
@@ -364,9 +415,9 @@ def test_fork_rows_sharing_experts(lib, M, fmt, boost):
 # ------------------------------------------------------------------ prefill: near ties
 def test_prefill_near_ties_exact_order(lib):
     """Router rows built so that token 0's 9th..12th experts have identical bf16
-    roundings (their MFMA logits are equal) while their exact logits differ by a
-    few ulps, plus one exact duplicate (a true tie, lower index wins). The
-    prefill selection must still equal the oracle's exact top-K for every token."""
+    roundings while their exact logits differ by a few ulps, plus one exact
+    duplicate (a true tie, lower index wins). The selection of a middle call (exact
+    router) must equal the oracle's exact top-K for every token."""
     T, seed, layer, xl = 33, 3, 12, 88
     _say("prefill near ties")
     qfm.init(H, I, E, K, 1, 1)
@@ -490,8 +541,8 @@ def _paths(lib, F, x_rows, x_pf, rng):
     out = []
     g = _forward(lib, F.lay, x_rows, F.st)                       # fused fork-row kernels (M = 2)
     out.append(("fused M=2", g["y"], x_rows, g["sel"], g["wts"]))
-    p = _forward(lib, F.lay, x_pf, F.st)                         # prefill grouped GEMMs (T = 9)
-    out.append(("prefill T=9", p["y"], x_pf, p["sel"], p["wts"]))
+    p = _forward(lib, F.lay, x_pf, F.st)                         # middle rows (T = 9)
+    out.append(("middle T=9", p["y"], x_pf, p["sel"], p["wts"]))
     a = F.a
     x1 = orc.bf16_to_f32(x_rows[0]).astype(np.float32)
     sel = rng.choice(E, K, replace=False).astype(np.int32)
@@ -516,7 +567,7 @@ def f4(lib):
 def test_e4m3_every_gate_up_byte(lib, f4):
     """Each of the 255 finite scale bytes (0x7F = +inf would make every output
     NaN) in turn as the gate and up block scale of every expert, down scales 1.0:
-    the fused fork-row, prefill and reference-named M=1 paths against the
+    the fused fork-row, middle-row and reference-named M=1 paths against the
     oracle's dequantization. Bytes >= 0x80 are scales up to 2^24 * 1.875."""
     _say("e4m3 gate/up bytes")
     x_rows = orc.fill("gauss_bf16", 9, 501, orc.T_X, 0, 2 * H).reshape(2, H)
@@ -617,6 +668,59 @@ def test_e4m3_every_down_byte(lib, f4):
         _say("  ", name, "worst rel err over the 255 finite bytes", worst)
 
 
+def test_e4m3_bytes_in_tiles(lib, f4):
+    """Every finite scale byte as the gate and up block scale of every expert
+    through the 128-row tiles (384 rows crowded on ten experts), and every byte as
+    a down row's scale: three rows (the first, one in the second tile, the last)
+    against the oracle's dequantization, as the paths above."""
+    T, rows = 384, [0, 200, 383]
+    _say("e4m3 bytes in tiles")
+    x = orc.fill("gauss_bf16", 9, 506, orc.T_X, 0, T * H).reshape(T, H)
+    bias = np.full(E, -64.0, np.float32)
+    bias[100:110] = 64.0
+    db = qfm.DevBuf.from_array(bias)
+    lay = qfm.QfmLayer.from_buffer_copy(f4.lay)
+    lay.router_bias = db.ptr
+    f4.set_scales(down_rows=np.full(H, 0x38, np.uint8))
+    bytes_ = [b for b in ALL_BYTES if b != 0x7F]
+    ys = []
+    for b in bytes_:
+        f4.set_scales(gate_up_byte=b)
+        _sync(lib)
+        g = _forward(lib, lay, x, f4.st)
+        assert g["counters"].tolist()[1:] == _gemm_blocks(g["sel"], T, H, I, 1, False, True)
+        ys.append(g["y"][rows])
+    sel, wts, scales = g["sel"], g["wts"], _e4m3(np.array(bytes_))
+    X = orc.bf16_to_f32(x).astype(np.float64)
+    for q, t in enumerate(rows):
+        R = np.zeros((len(bytes_), H))
+        for k in range(K):
+            Wg, Wu, Wd = f4.unit(int(sel[t, k]))
+            gg, uu = np.outer(scales, Wg @ X[t]), np.outer(scales, Wu @ X[t])
+            with np.errstate(over="ignore", invalid="ignore"):
+                R += float(wts[t, k]) * ((gg / (1.0 + np.exp(-gg)) * uu) @ Wd.T)
+        for i, b in enumerate(bytes_):
+            if scales[i] == 0.0:
+                assert not ys[i][q].any(), hex(b)
+            else:
+                assert _rel(ys[i][q], R[i]) <= TOL, (hex(b), t)
+    bytes_c = (np.arange(H) % 256).astype(np.uint8)
+    f4.set_scales(gate_up_byte=0x38, down_rows=bytes_c)
+    _sync(lib)
+    g = _forward(lib, lay, x, f4.st)
+    srow = _e4m3(bytes_c)
+    finite = np.isfinite(srow)
+    r = f4.ref(x[rows], g["sel"][rows], g["wts"][rows], 1.0, np.where(finite, srow, 0.0))
+    y = g["y"][rows]
+    assert np.isfinite(y[:, finite]).all() and not np.isfinite(y[:, ~finite]).any()
+    for b in bytes_:
+        cols = np.nonzero(bytes_c == b)[0]
+        if srow[b] == 0.0:
+            assert not y[:, cols].any(), hex(b)
+        else:
+            assert float(np.abs(y[:, cols] - r[:, cols]).max() / np.abs(r[:, cols]).max()) <= TOL, hex(b)
+
+
 # ------------------------------------------------------------------ decode: zero rows
 @pytest.mark.parametrize("M,fmt,bias", [(1, 0, False), (3, 0, False), (1, 1, True), (5, 1, False)])
 def test_decode_zero_rows(lib, M, fmt, bias):
@@ -647,8 +751,8 @@ def test_decode_zero_rows(lib, M, fmt, bias):
 @pytest.mark.parametrize("M,fmt,shift", [(1, 0, 24), (1, 0, -24), (4, 1, 24), (4, 0, -24), (40, 0, 24), (40, 1, -24)])
 def test_input_dynamic_range(lib, M, fmt, shift):
     """x rows scaled by 2^shift (exact in bf16) through the fused decode and
-    prefill paths: the activations as fp16 scaled per token or per 16 values,
-    the hidden vectors' fp16 chunks and the prefill's scaled fp16 partials must
+    middle-row paths: the activations as fp16 scaled per token or per 16 values,
+    the hidden vectors' fp16 chunks and rows and the scaled fp16 partials must
     follow the magnitude. At 2^24 the softmax is one-hot, at 2^-24 nearly
     uniform; the routing stays bit-exact and y within the usual bound."""
     _say("dynamic range M", M, "fmt", fmt, "shift", shift)
@@ -666,6 +770,34 @@ def test_input_dynamic_range(lib, M, fmt, shift):
     assert np.allclose(g["wts"], r["w"], rtol=2e-6, atol=1e-7)
     assert np.isfinite(g["y"]).all()
     rel = max(_rel(g["y"][t], r["y"][t]) for t in range(M))
+    _say("  max rel err", rel)
+    assert rel <= TOL
+    L.destroy()
+    st.destroy()
+
+
+@pytest.mark.parametrize("T,fmt,shift", [(384, 0, 24), (385, 1, 24), (640, 0, -24), (384, 1, -24)])
+def test_input_dynamic_range_in_tiles(lib, T, fmt, shift):
+    """The same scaled rows through the 128-row tiles (rows crowded on ten experts
+    by a bias far above the logits): x as scaled fp16 (INT8) or bf16 with the row
+    sums of the offset corrections, bf16 hidden rows and the scaled fp16 partials."""
+    _say("dynamic range in tiles T", T, "fmt", fmt, "shift", shift)
+    qfm.init(H, I, E, K, 1, 1)
+    st = qfm.Stream()
+    L = qfm.SynthLayer(fmt, 7, 72, with_bias=True, stream=st)
+    st.sync()
+    bias = np.full(E, -2.0 ** 30, np.float32)
+    bias[100:110] = 2.0 ** 30
+    qfm.check(lib.qfm_memcpy_h2d(L.s.layer.router_bias, bias.ctypes.data, bias.nbytes), "bias")
+    xf = orc.bf16_to_f32(orc.fill("gauss_bf16", 7, 640, orc.T_X, 0, T * H).reshape(T, H)) * np.float32(2.0 ** shift)
+    x = (xf.view(np.uint32) >> 16).astype(np.uint16)
+    g = _forward(lib, L.s.layer, x, st)
+    assert g["counters"].tolist()[1:] == _gemm_blocks(g["sel"], T, H, I, fmt, True, True)
+    r = orc.moe_layer_grouped(H, I, E, K, T, 7, 72, 0, x=x, fmt=fmt, use_bias=1, bias=bias)
+    assert np.array_equal(g["sel"], r["sel"])
+    assert np.allclose(g["wts"], r["w"], rtol=2e-6, atol=1e-7)
+    assert np.isfinite(g["y"]).all()
+    rel = max(_rel(g["y"][t], r["y"][t]) for t in range(T))
     _say("  max rel err", rel)
     assert rel <= TOL
     L.destroy()

@@ -7,9 +7,10 @@ give the bits of the eager run of the same chain (the kernels write each
 output once, in a fixed order, so eager and replayed results are identical).
 The chain covers M = 1 (the single-row INT8 kernels), M = 8 (the fork-row
 kernels, INT8 and NVFP4) and M = 4 NVFP4 (the selection in the router launch
-and the combine in the down launch, whose tags advance on every replay), and
-a prefill (T = 37: the counters cleared by a fill kernel, never by a memset
-node).
+and the combine in the down launch, whose tags advance on every replay), middle
+rows (37; their counters are cleared by the router launch, never by a memset
+node), and a captured middle call whose plan picks another form of the expert
+GEMMs when the routing changes between replays.
 """
 import ctypes as C
 import sys
@@ -83,4 +84,59 @@ def test_graph_replays_match_eager(lib, M, fmt, nl):
     assert lib.qfm_graph_destroy(g) == 0
     for L in layers:
         L.destroy()
+    st.destroy()
+
+
+@pytest.mark.parametrize("T,fmt", [(512, 0), (700, 1), (1300, 0)])
+def test_graph_form_follows_the_routing(lib, T, fmt):
+    """One captured middle call, replayed with its rows spread, crowded on ten
+    experts (128-row tiles) and spread again by what the router bias buffer holds:
+    every replay equals the eager call's bits, and the counters those of its form."""
+    _say("graph form T", T, "fmt", fmt)
+    qfm.init(H, 512, 512, 10, 1, 1)
+    st = qfm.Stream()
+    L = qfm.SynthLayer(fmt, 0, 44, with_bias=True, stream=st)
+    st.sync()
+    crowd = np.full(512, -64.0, np.float32)
+    crowd[100:110] = 64.0
+    x, y = qfm.DevBuf(T * H * 2), qfm.DevBuf(T * H * 2)
+    qfm.check(lib.qfm_gen_input_rows(x.ptr, T, 0, 510, 0, st.h), "x")
+    wsb = lib.qfm_workspace_bytes(T)
+    ws = qfm.DevBuf(wsb)
+
+    def fwd():
+        qfm.check(lib.qfm_moe_forward(C.byref(L.s.layer), x.ptr, T, y.ptr, ws.ptr, wsb, st.h), "fwd")
+
+    def result():
+        st.sync()
+        view = qfm.QfmWsView()
+        lib.qfm_workspace_view(ws.ptr, T, C.byref(view))
+        return y.download(np.uint16, (T, H)), qfm.d2h(view.counters, np.int32, 3)
+
+    def set_bias(b):
+        qfm.check(lib.qfm_memcpy_h2d(L.s.layer.router_bias, b.ctypes.data, b.nbytes), "bias")
+        y.zero()
+
+    biases = [np.zeros(512, np.float32), crowd]
+    ref = []
+    for b in biases:
+        set_bias(b)
+        fwd()
+        ref.append(result())
+    assert not np.array_equal(ref[0][1], ref[1][1])
+    qfm.check(lib.qfm_graph_capture_begin(st.h), "capture")
+    fwd()
+    g = lib.qfm_graph_capture_end(st.h)
+    assert g, lib.qfm_last_error().decode()
+    for rep, i in enumerate((0, 1, 0, 1, 1)):
+        set_bias(biases[i])
+        qfm.check(lib.qfm_graph_launch(g, st.h), "launch")
+        got = result()
+        assert np.array_equal(got[0], ref[i][0]) and np.array_equal(got[1], ref[i][1]), rep
+        set_bias(biases[1 - i])                              # eager work of the other form between the replays
+        fwd()
+        got = result()
+        assert np.array_equal(got[0], ref[1 - i][0]) and np.array_equal(got[1], ref[1 - i][1]), rep
+    assert lib.qfm_graph_destroy(g) == 0
+    L.destroy()
     st.destroy()

@@ -494,10 +494,10 @@ def _run_prefill(lib, T, seed, layer, x_layer, bias=True, fmt=qfm.QFM_FMT_INT8, 
 @pytest.mark.parametrize("T,bias,fmt,renorm", [(9, True, 0, 1), (37, True, 0, 1), (300, True, 0, 1), (129, False, 0, 1), (37, True, 1, 1),
                                                (300, True, 1, 1), (9, False, 1, 1), (37, True, 0, 0), (129, False, 1, 0)])
 def test_prefill_small(lib, T, bias, fmt, renorm):
-    """Prefill path (T > 8): MFMA router + exact candidate selection, grouped GEMMs
-    on INT8 (fmt 0) or NVFP4 (fmt 1) routed experts (the shared expert is INT8).
-    renorm 0 divides by the softmax denominator over all 512 logits, which the
-    selection recomputes exactly (weights at the same 2e-6 as renorm 1)."""
+    """Middle rows (more than 8): exact router, weight-streaming grouped GEMMs on
+    INT8 (fmt 0) or NVFP4 (fmt 1) routed experts (the shared expert is INT8).
+    renorm 0 divides by the softmax denominator over all 512 logits (weights at the
+    same 2e-6 as renorm 1; beyond 600 rows: test_gpu_routing.py)."""
     _say("prefill", T, bias, "int8" if fmt == 0 else "nvfp4", "renorm", renorm)
     _cfg(lib, renorm=renorm)
     g = _run_prefill(lib, T, 1, 2, 600 + T, bias, fmt)
@@ -534,8 +534,8 @@ def test_prefill_config4_routing_and_sample(lib):
 
 @pytest.mark.parametrize("T,fmt,gated", [(37, 0, 1), (20, 1, 0)])
 def test_prefill_reference_shape(lib, T, fmt, gated):
-    """Prefill at the reference's own shape (H=2560, I=640): router tiles of
-    K=2560, five gate/up n-tiles, ten down n-tiles."""
+    """Middle rows at the reference's own shape (H=2560, I=640): ten gate/up and ten
+    down blocks an item (its 128-row tiles: test_tiles_beyond_middle)."""
     _say("prefill 2560/640", T, fmt, gated)
     _cfg(lib, H=2560, I=640, gated=gated)
     g = _run_prefill(lib, T, 2, 5, 900 + T, True, fmt, H=2560)

@@ -106,9 +106,37 @@ def test_masked_experts(lib, H, T, K, finite):
         assert counters[0] == T and not got[1][:, finite:].any()
 
 
+@pytest.mark.parametrize("H,T,bias", [(2048, 601, False), (2048, 1200, True), (2560, 601, True), (2560, 1200, False),
+                                      (2560, 2100, True), (2560, 4200, False)])
+def test_near_ties_exact_order(lib, H, T, bias):
+    """Router rows whose bf16 roundings coincide, so that the MFMA logits of the
+    9th..12th experts of token 0 are equal while the exact ones differ by a few
+    ulps, with an exact duplicate (the lower index wins): only the exact
+    recomputation orders them. Four slices of H and four waves a token, four and
+    one, two and one, one and one."""
+    rng = np.random.default_rng(T)
+    W = orc.fill("gauss", 12, 7, orc.T_ROUTER, 0, E * H, 0.02).reshape(E, H).copy()
+    x = orc.fill("gauss_bf16", 12, 40, orc.T_X, 0, T * H).reshape(T, H)
+    b = np.zeros(E, np.float32)
+    if bias:
+        b[:] = rng.choice([0.0, 0.25, 0.5], E)
+    order = np.argsort(-orc.router_logits(W, x[:1], b)[0].astype(np.float64), kind="stable")
+    base, near = int(order[8]), [int(e) for e in order[20:24]]
+    k = int(np.argmax(np.abs(orc.bf16_to_f32(x[0]))))
+    for j, e in enumerate(near):
+        W[e], b[e] = W[base], b[base]
+        for _ in range(j):                                   # near[0]: the duplicate
+            W[e, k] = np.nextafter(W[e, k], np.float32(np.inf if j % 2 else -np.inf))
+    bits = lambda a: (a.view(np.uint32) + 0x7FFF + ((a.view(np.uint32) >> 16) & 1)) >> 16
+    assert all(np.array_equal(bits(W[e]), bits(W[base])) for e in near)
+    got, ref, _ = _route(lib, H, T, 10, bias=b if bias else None, x=x, router=W)
+    _check(got, ref)
+
+
 # ------------------------------------------------------------------ counters
 @pytest.mark.parametrize("H,T,fmt,renorm,per", [(2048, 40, 0, 1, 16), (2048, 40, 1, 0, 16), (2560, 601, 1, 0, 16),
-                                                (2560, 1200, 0, 1, 16), (2048, 1300, 0, 0, 64), (2048, 2900, 0, 0, 128)])
+                                                (2048, 601, 1, 1, 16), (2560, 1200, 0, 1, 16), (2048, 1300, 0, 0, 64),
+                                                (2048, 2900, 0, 0, 128), (2560, 1801, 0, 0, 128), (2560, 2501, 1, 1, 256)])
 def test_workspace_counters(lib, H, T, fmt, renorm, per):
     """The view's counters: the tokens with more than 64 candidates (here the
     zero rows, whose logits all tie), with and without renormalization, and the
@@ -120,6 +148,7 @@ def test_workspace_counters(lib, H, T, fmt, renorm, per):
     x[zero] = 0
     got, ref, counters = _route(lib, H, T, K, x=x, renorm=renorm, fmt=fmt)
     _check(got, ref)
-    items = int((-(-np.bincount(got[0].ravel(), minlength=E) // per)).sum()) - (-T // per)   # and the shared expert's
-    gate_up, down = {16: (I // 64, H // 256), 64: (I // 64, H // 512), 128: (I // 128, H // 128)}[per]
+    rows = min(per, 128)                                 # (256: NVFP4 tiles of 128 rows, 256 down columns)
+    items = int((-(-np.bincount(got[0].ravel(), minlength=E) // rows)).sum()) - (-T // rows)   # and the shared expert's
+    gate_up, down = {16: (I // 64, H // 256), 64: (I // 64, H // 512), 128: (I // 128, H // 128), 256: (I // 128, H // 256)}[per]
     assert counters.tolist() == [len(zero), items * gate_up, items * down]
