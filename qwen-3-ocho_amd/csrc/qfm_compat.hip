@@ -172,11 +172,15 @@ __device__ __forceinline__ void ld_f32x16(const float *p, float *v) {
 // one 32-value X8 block (exact), scaled by the token's block scale into fp32.
 // Weights stream 16 bytes a lane, two 256-value chunks in flight, and become
 // fragments through wave-private LDS (as the middle path's gate/up); an
-// expert's further pairs read them again, from L2. Bound by the weight stream;
-// the form before it (a lane group per row, four tokens a pass) lost the
-// stream's rate to its dots from ~2 rows an expert on (2560/640, 64 / 128 / 256 /
-// 1024 rows, whole call with the down launch below: 514 / 846 / 1410 / 4704 us
-// against 317 / 420 / 503 / 1286).
+// expert's further pairs read them again (nontemporally too, the first ones being
+// most of the bytes). Bound by the weight stream; the form before it (a lane group
+// per row, four tokens a pass) lost the stream's rate to its dots from ~2 rows an
+// expert on. Whole call with the down launch below, us, before / now at 2 / 4 / 8 /
+// 16 rows: 2048/512 44 / 34, 65 / 44, 111 / 65, 187 / 96, 2560/640 43 / 43, 64 / 57,
+// 106 / 89, 176 / 139; 2560/640 at 64 / 128 / 256 / 1024 rows 514 / 846 / 1410 / 4704
+// against 317 / 420 / 503 / 1286; 64 rows all on ten experts 363 against 164, and
+// 202 where the caller's bound says 512 experts (one token tile a down pass in
+// place of four).
 struct ChunkGuLds {
     uint8_t w[4][32 * 256];                       // per wave: 16 gate and 16 up rows of one chunk
     uint8_t x[2][16 * 256];                       // 16 tokens' codes, two chunks
@@ -278,8 +282,9 @@ k_cx_gateup_i8x8(const int8_t *__restrict__ Wg, const float *__restrict__ Sg, co
 // (qf8_moe_i8.hip:263-311). grid (H / CW, n_exp_max), CW columns a block.
 // MFMA tiles of 16 weight rows by 16 columns (mid_dn_body), a pair's fp32 hidden row as three
 // of the columns: the value times 2^k (k per 64 values) split into three fp16
-// pieces of 11 bits, which leaves nothing of the 24 out (2^-39 of the group's
-// largest value at most), so the dots are the fp32 ones; the three sums are
+// pieces of 11 bits. Values from 2^-15 of their group's largest on keep all 24
+// bits, smaller ones what lies above 2^-39 of it, far below the sums' own rounding
+// (error against 64 bits 2.8e-7, 3.0e-7 with fp32 dots); the three sums are
 // added per row. Five pairs a token tile; an expert's further pairs read its
 // weights again (from L2). Bound by the weight stream; the form before it (a
 // lane group per weight row, each reading the pairs' rows from L2) waited for

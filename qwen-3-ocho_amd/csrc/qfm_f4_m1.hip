@@ -11,8 +11,9 @@
 // row before, rank it in the router launch's tail and pass partials as tagged
 // words: two cross-XCD hand-offs, which one row need not pay. Bound by the three
 // dependent launches and the selection (~1.3 us), then the weight streams.
-// us per layer (8 layers, graph), the fork-row kernels -> these: 2048/512 17.3 ->
-// 14.4, 2560/640 21.3 -> 18.7 (per launch: router 6.3 -> 3.9, gate/up 8.3 -> 9.5
+// us per layer (8 layers, one graph over and over; with other inputs between the
+// passes 2560/640 21.6 -> 19.1), the fork-row kernels -> these: 2048/512 17.3 ->
+// 14.3, 2560/640 21.5 -> 18.7 (per launch: router 6.3 -> 3.9, gate/up 8.3 -> 9.5
 // with the selection and the shared expert in it, down 7.2 -> 7.2; 2048/512 down
 // 4.7).
 #include "qfm_dev.h"

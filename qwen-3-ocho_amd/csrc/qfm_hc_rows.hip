@@ -13,7 +13,11 @@
 // us per call, two launches -> three (H = 2048): T = 2 12.0 -> 18.5, 4 15.1 ->
 // 18.8, 5 18.6 -> 18.9, 6 18.8 -> 19.0, 8 23.3 -> 19.1, 16 37.6 -> 19.9, 129
 // 252 -> 26.6, 256 497 -> 31.3; H = 2560: T = 4 19.6 -> 21.2, 5 22.6 -> 21.3,
-// 129 347 -> 30.1, 256 683 -> 36.6. Hence kHcFewRows = 4.
+// 129 347 -> 30.1, 256 683 -> 36.6. These calls find the 6.7 or 10.5 MB of weights
+// in the caches; over 24 layers, us per layer: H = 2048 T = 4 15.7 (two launches), 5
+// 19.4 -> 19.1, 6 19.9 -> 19.1, 8 24.2 -> 19.2, H = 2560 T = 5 23.5 -> 21.8; a call whose
+// weights and rows were never read, 129 rows at H = 2560: 376 -> 53. Hence
+// kHcFewRows = 4.
 #include "qfm_internal.h"
 #include "qfm_x8.h"
 

@@ -92,7 +92,8 @@ __device__ __forceinline__ float exp2i(int k) { return __uint_as_float((uint32_t
 // gate/up + down at 37 / 300 rows 154 -> 136 / 288 -> 262 us, 6.4 TB/s), plain
 // where an expert's further items read them again (1021 rows: 264 + 167 us
 // nontemporal, 244 + 144 plain; NVFP4 at 2560/640 395 + 255 against 304 + 240;
-// at 700 rows no difference).
+// at 700 rows no difference; whole calls at 600 rows 2560/640 INT8 evenly spread
+// 543 nontemporal, 561 plain, all on ten experts 356 and 270).
 template <bool ONCE>
 __device__ __forceinline__ u32x4_t ld_w(const uint8_t *p) {
     const u32x4_t *v = reinterpret_cast<const u32x4_t *>(p);

@@ -40,7 +40,8 @@ namespace qfm {
 
 // ---- router ---------------------------------------------------------------------
 // Blocks [0, ceil(T / 4)): a wave per token writes x as fp16 scaled by 2^k
-// (largest magnitude in [2^14, 2^15): bf16 values exact) and 2^-k. The others:
+// (largest magnitude in [2^14, 2^15): bf16 values from 2^-28 of the row's largest
+// on exact, smaller ones to 2^-39 of it) and 2^-k. The others:
 // 8 router rows (two per wave, held in registers) x tg groups of 8 tokens,
 // whose x rows go through LDS; block row E / 8 is the shared-expert gate
 // vector. Every dot keeps the canonical order (canon_reduce_rows).
@@ -630,12 +631,15 @@ int launch_mid(const MidArgs &a, hipStream_t s) {
                                a.gam, a.x16, a.x16isc, a.xsum, a.x16sum, a.ctr);
         hipLaunchKernelGGL(k_mid_topk<8>, dim3((T + 3) / 4), dim3(256), 0, s, a.logits, T, K, c.renorm, a.sel, a.wts, a.ctr);
     }
-    // token tiles per item. One (16 rows) keeps three blocks on a CU, which
-    // streams best, and an expert's further items find its weights in L2:
-    // gate/up + down, us, at 300 / 1021 / 1500 / 2000 rows with one, two and
-    // four tiles: INT8 289 / 370 / 443 / 534, 321 / 373 / 466 / 589, 343 / 380 /
-    // 425 / 462; NVFP4 198 / 345 / 422 / 500, 278 / 386 / 462 / 580, 436 / 526 /
-    // 599 / 688. Four are taken for INT8 from 24 rows an expert.
+    // token tiles per item. With one (16 rows) LDS and registers leave three
+    // blocks on a CU (down at 2560/640: two), and an expert's further items find
+    // its weights in L2: gate/up + down, us, at 300 / 1021 / 1500 / 2000 rows with
+    // one, two and four tiles: INT8 289 / 370 / 443 / 534, 321 / 373 / 466 / 589,
+    // 343 / 380 / 425 / 462; NVFP4 198 / 345 / 422 / 500, 278 / 386 / 462 / 580, 436 /
+    // 526 / 599 / 688. Two and four tiles also read their weights in chunks half as
+    // long (mid_kc), and NVFP4's LDS is sized for the INT8 shared expert's rows: the
+    // figures compare these forms, not wider items alone. Four are taken for INT8
+    // from 24 rows an expert.
     const int dw = 64 * mid_dn_waves(I, nt);                      // columns, and threads, per down block
     hipLaunchKernelGGL(k_mid_plan, dim3(1), dim3(1024), 0, s, a.sel, a.wts, a.g ? a.gam : nullptr, T, K, E, a.has_sh, mt,
                        a.pairs, a.items, a.max_items, I / 64, H / dw, a.tiles, a.ctr);

@@ -157,7 +157,8 @@ __global__ void __launch_bounds__(256) k_pf_router_prep(const float *__restrict_
         }
         if (x16) {
             // the row as fp16 scaled by 2^k (largest magnitude in [2^14, 2^15): no
-            // overflow, bf16 values exact), with the sum of the scaled values and 2^-k
+            // overflow; bf16 values from 2^-28 of the row's largest on exact, smaller
+            // ones to 2^-39 of it), with the sum of the scaled values and 2^-k
             float amax = 0.0f;
 #pragma unroll
             for (int q = 0; q < kMaxCh; q++) {
