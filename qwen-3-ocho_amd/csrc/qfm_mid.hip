@@ -221,7 +221,8 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
     __syncthreads();
     const int c = g < E ? cnt[g] : 0;
     const int mi = (c + mt - 1) / mt;
-    sa[g] = c;
+    constexpr int kGroup = 1 << 20;                            // (above every pair count)
+    sa[g] = c | (c > 0 ? kGroup : 0);                          // pairs, and groups
     sb[g] = mi | ((c + BM - 1) / BM) << 16;                    // items, and 128-row tiles
     __syncthreads();
     for (int st = 1; st < E; st <<= 1) {                       // inclusive scans (packed: neither half carries)
@@ -231,11 +232,10 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
         sb[g] += b;
         __syncthreads();
     }
-    const int off = sa[g] - c, shi = has_sh ? (T + mt - 1) / mt : 0;
+    const int off = (sa[g] & (kGroup - 1)) - c, shi = has_sh ? (T + mt - 1) / mt : 0;
     cnt[g] = off;                                              // the group's next free pair
-    const int ngrp = __syncthreads_count(c > 0);
     const int n16 = (sb[E - 1] & 0xFFFF) + shi, mtr = sb[E - 1] >> 16, mtot = mtr + (has_sh ? (T + BM - 1) / BM : 0);
-    const int gcost = (ngrp + has_sh) * tp.cost.group + (n16 - ngrp - has_sh) * tp.cost.item;
+    const int ngrp = sa[E - 1] / kGroup + has_sh, gcost = ngrp * tp.cost.group + (n16 - ngrp) * tp.cost.item;
     const bool tiles = mtot <= tp.max_mt && mtot * tp.cost.tile + tp.cost.base < gcost;   // (block-uniform)
     if (tiles) {
         // the work lists of k_pf_gemm, as k_pf_plan stores them: one thread per m-tile
@@ -248,7 +248,7 @@ k_mid_plan(const int *__restrict__ sel, const float *__restrict__ wts, const flo
                     const int mid = (lo + hi) >> 1;
                     if ((sb[mid] >> 16) > m) hi = mid; else lo = mid + 1;
                 }
-                const int end = sa[lo], cl = end - (lo ? sa[lo - 1] : 0);
+                const int end = sa[lo] & (kGroup - 1), cl = end - (lo ? sa[lo - 1] & (kGroup - 1) : 0);
                 grp = lo;
                 row0 = (m - (lo ? sb[lo - 1] >> 16 : 0)) * BM;
                 rows = min(BM, cl - row0);
