@@ -108,7 +108,10 @@ inline bool mid_reads_once(int T, int E, int K, bool f4) { return T * K / E < (f
 // Which form of the expert GEMMs a middle call runs is known once the selection
 // is: a router that crowds its rows on few experts makes many items of one
 // expert, and each reads and converts its weights again, where a 128-row tile
-// does it once. From mid_offers_tiles on the tile GEMMs are launched behind the
+// does it once. The tiles hold the hidden rows in 8 bits (bf16), the items in 11;
+// a bf16 result rounds to about the same (error against 64 bits 0.0024 and
+// 0.0017), an fp32 result does not (0.0017 and 0.0003) and keeps the items. For
+// bf16 results, from mid_offers_tiles on, the tile GEMMs are launched behind the
 // middle ones, and k_mid_plan leaves one pair of them without work (2.5 us each):
 // the tiles run where tiles * tile + base < groups * group + (items - groups) *
 // item, in units of 10 ns (groups: experts with a row, items: mid_token_tiles).

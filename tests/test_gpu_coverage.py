@@ -284,7 +284,7 @@ def test_middle_rows_crowded(lib, hidden, inter, T, fmt, k, shared, gated, tiles
     on them): from 256 (2560/640) or 384 rows on the plan leaves such a call to the
     128-row tiles, read from its own pairs; the groups hold T rows each, whole
     tiles, one row more and one fewer. Below, items of 16 rows. The counters say
-    which ran. Up to 600 rows the row sums of x that the tiles correct their offsets
+    which ran; an fp32 result keeps the items. Up to 600 rows the row sums of x that the tiles correct their offsets
     with come from k_mid_router, beyond from the MFMA router's prep launch.
     Routing bit-exact, y within TOL of the grouped fp64 oracle; crowded calls and
     calls with spread rows in turn on one workspace, each repeats its first result
@@ -326,6 +326,17 @@ def test_middle_rows_crowded(lib, hidden, inter, T, fmt, k, shared, gated, tiles
     _say("  max rel err", rel)
     assert rel <= TOL
     assert np.array_equal(ys[0], ys[2]) and np.array_equal(ys[1], ys[3])
+    dy32 = qfm.DevBuf(T * hidden * 4)
+    qfm.check(lib.qfm_moe_forward_f32(C.byref(lay), dx.ptr, T, dy32.ptr, ws.ptr, wsb, st.h), "forward f32")
+    st.sync()
+    counters = qfm.d2h(view.counters, np.int32, 3).tolist()
+    assert counters[1:] == _gemm_blocks(sel, T, hidden, inter, fmt, shared, False)
+    y = dy32.download(np.float32, (T, hidden)).astype(np.float64)
+    err = float(np.linalg.norm(y - r["y"]) / np.linalg.norm(r["y"]))
+    _say("  fp32 result: error (2-norm)", err)
+    # hidden rows rounded to 11 bits (2^-12 of a value) and partials to 11 bits of their
+    # 64 columns' largest, 3 times the root mean square: 4 x 2^-12 (bf16 hidden rows: 1.7e-3)
+    assert err <= 4 * 2.0 ** -12
     L.destroy()
     st.destroy()
     qfm.init(H, I, E, K, 1, 1)
