@@ -1320,7 +1320,7 @@ int launch_prefill(const qfm_layer *L, const uint16_t *x, int T, uint16_t *y, fl
     };
     // router and selection: exact logits of every expert up to kMidExactRows
     // rows (launch_mid), the bf16 MFMA GEMM with exact candidates beyond
-    const bool mid = mid_takes(T, K, I, f4), offer = mid && !y32 && mid_offers_tiles(T, I);
+    const bool f32 = y32 != nullptr, mid = mid_takes(T, K, I, f4, f32), offer = mid && mid_offers_tiles(T, I, f32);
     const int room = (int)(Lw.bytes[kPfItemsGu] / sizeof(int4)), mid_nt = mid_token_tiles(T, E, K, I, f4);
     if (mid) {
         const int need = mid_items_bound(T, E, K, has_sh, mid_nt);

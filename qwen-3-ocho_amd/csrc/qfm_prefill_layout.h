@@ -91,15 +91,16 @@ inline int mid_items_bound(int T, int E, int K, bool has_sh, int token_tiles) {
 
 constexpr int kPfTileRows = 128;       // rows of a tile of the grouped GEMMs
 
-// The largest call of the middle path, in rows; at another top_k than 10 also in
-// pairs, as it is an expert's rows that decide. us per layer, the middle path /
+// The largest call of the middle path, in rows; at a larger top_k than 10 also in
+// pairs, as it is an expert's rows that decide, unless the result is fp32, which
+// keeps the items' hidden rows (below) as long as the rows allow. us per layer, the middle path /
 // 128-row tiles: 2048/512 INT8 1500 rows 507 / 620, 2560/640 INT8 1500 rows 841 /
 // 932, NVFP4 2048/512 458 / 686, 2560/640 723 / 991; it grows by 0.13, 0.30, 0.19
 // and 0.28 us a row, the tiles by 0.04 to 0.07. Top-16, 2800 rows of 2048/512:
 // INT8 940 / 737, NVFP4 1059 / 784.
 constexpr int mid_rows_max(int I, bool f4) { return I <= 512 ? 2800 : f4 ? 2500 : 1800; }
-inline bool mid_takes(int T, int K, int I, bool f4) {
-    return T <= mid_rows_max(I, f4) && T * K <= 10 * mid_rows_max(I, f4);
+inline bool mid_takes(int T, int K, int I, bool f4, bool f32) {
+    return T <= mid_rows_max(I, f4) && (f32 || T * K <= 10 * mid_rows_max(I, f4));
 }
 
 // Few rows an expert: weights read once, nontemporal (the figures are at ld_w).
@@ -119,7 +120,7 @@ inline bool mid_reads_once(int T, int E, int K, bool f4) { return T * K / E < (f
 // rows on ten experts, 256 to 2800 rows; the choice is within 2% of the faster
 // form in 363 of 368 of them and within 11% in all.
 struct MidCost { int group, item, tile, base; };
-inline bool mid_offers_tiles(int T, int I) { return T >= (I > 512 ? 256 : 384); }
+inline bool mid_offers_tiles(int T, int I, bool f32) { return !f32 && T >= (I > 512 ? 256 : 384); }
 inline MidCost mid_cost(int I, bool f4, int token_tiles, bool once) {
     if (f4) return I > 512 ? MidCost{0, 30, 99, 1000} : MidCost{0, 18, 68, 1300};
     if (I > 512) return once ? MidCost{0, 54, 67, 2400} : MidCost{0, 31, 65, 1700};

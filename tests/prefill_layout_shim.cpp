@@ -23,8 +23,8 @@ extern "C" int mid_token_tiles_c(int T, int E, int K, int I, int f4) { return qf
 extern "C" int mid_items_bound_c(int T, int E, int K, int has_sh, int token_tiles) {
     return qfm::mid_items_bound(T, E, K, has_sh != 0, token_tiles);
 }
-extern "C" int mid_takes_c(int T, int K, int I, int f4) { return qfm::mid_takes(T, K, I, f4 != 0); }
-extern "C" int mid_offers_tiles_c(int T, int I) { return qfm::mid_offers_tiles(T, I); }
+extern "C" int mid_takes_c(int T, int K, int I, int f4, int f32) { return qfm::mid_takes(T, K, I, f4 != 0, f32 != 0); }
+extern "C" int mid_offers_tiles_c(int T, int I, int f32) { return qfm::mid_offers_tiles(T, I, f32 != 0); }
 extern "C" int mid_picks_tiles_c(int groups, int items, int tiles, int T, int E, int K, int I, int f4) {
     const qfm::MidCost c =
         qfm::mid_cost(I, f4 != 0, qfm::mid_token_tiles(T, E, K, I, f4 != 0), qfm::mid_reads_once(T, E, K, f4 != 0));

@@ -388,6 +388,39 @@ def test_tiles_beyond_middle(lib, hidden, inter, T, fmt, shared, gated, hot):
     qfm.init(H, I, E, K, 1, 1)
 
 
+@pytest.mark.parametrize("hidden,inter,T,fmt", [(2048, 512, 2800, 0), (2560, 640, 1800, 0), (2560, 640, 2500, 1)])
+def test_middle_rows_fp32_top16(lib, hidden, inter, T, fmt):
+    """The largest fp32 middle calls at top-16, where a bf16 result runs the tiles:
+    both forms of one call on the same rows, by the counters; routing the same, y
+    apart by the tiles' 8-bit hidden rows and the bf16 result (2^-9 each)."""
+    _say("middle rows fp32 top-16 H", hidden, "T", T, "fmt", fmt)
+    qfm.init(hidden, inter, E, 16, 1, 1)
+    st = qfm.Stream()
+    L = qfm.SynthLayer(fmt, 8, 3, stream=st)
+    x = orc.fill("gauss_bf16", 8, 62, orc.T_X, 0, T * hidden).reshape(T, hidden)
+    dx, dy = qfm.DevBuf.from_array(x), qfm.DevBuf(T * hidden * 4)
+    wsb = lib.qfm_workspace_bytes(T)
+    ws = qfm.DevBuf(wsb)
+    view = qfm.QfmWsView()
+    got = []
+    for f32 in (False, True):
+        fwd = lib.qfm_moe_forward_f32 if f32 else lib.qfm_moe_forward
+        qfm.check(fwd(C.byref(L.s.layer), dx.ptr, T, dy.ptr, ws.ptr, wsb, st.h), "forward")
+        st.sync()
+        lib.qfm_workspace_view(ws.ptr, T, C.byref(view))
+        sel = qfm.d2h(view.sel, np.int32, (T, 16))
+        counters = qfm.d2h(view.counters, np.int32, 3).tolist()
+        assert counters[1:] == _gemm_blocks(sel, T, hidden, inter, fmt, True, not f32)
+        got.append((sel, dy.download(np.float32, (T, hidden)) if f32 else orc.bf16_to_f32(dy.download(np.uint16, (T, hidden)))))
+    assert np.array_equal(got[0][0], got[1][0])
+    err = float(np.linalg.norm(got[0][1] - got[1][1]) / np.linalg.norm(got[1][1]))
+    _say("  2-norm difference", err)
+    assert err <= 2 * 2.0 ** -9
+    L.destroy()
+    st.destroy()
+    qfm.init(H, I, E, K, 1, 1)
+
+
 # ------------------------------------------------------------------ fork rows sharing experts
 @pytest.mark.parametrize("M,fmt,boost", [(2, 0, 64.0), (8, 0, 64.0), (8, 1, 64.0), (8, 0, 1.5), (5, 1, 1.5)])
 def test_fork_rows_sharing_experts(lib, M, fmt, boost):

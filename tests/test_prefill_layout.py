@@ -212,21 +212,25 @@ def test_middle_items_never_exceed_their_bound(shim, H, I, f4, top):
 @pytest.mark.parametrize("H,I,f4,top", [(2048, 512, 0, 2800), (2048, 512, 1, 2800), (2560, 640, 0, 1800),
                                         (2560, 640, 1, 2500)])
 def test_middle_path_by_pairs_and_routing(shim, H, I, f4, top):
-    """The middle path ends at `top` rows and, at a larger top_k, at as many pairs
-    as top-10 makes there. Inside, a plan that takes the 128-row tiles fits their
+    """The middle path ends at `top` rows and, at a larger top_k and for bf16
+    results, at as many pairs as top-10 makes there. Inside, a plan that takes the 128-row tiles fits their
     work lists whatever the routing, rows crowded on ten experts take them (from
     the first call that offers them on), and evenly spread rows take the items up
     to the largest call."""
     E = 512
     rng = np.random.default_rng(8)
     first = 256 if I > 512 else 384
-    assert shim.mid_takes_c(top, 10, I, f4) and not shim.mid_takes_c(top + 1, 10, I, f4)
-    assert shim.mid_takes_c(top, 1, I, f4) and not shim.mid_takes_c(top + 1, 1, I, f4)
-    assert shim.mid_takes_c(10 * top // 16, 16, I, f4) and not shim.mid_takes_c(10 * top // 16 + 1, 16, I, f4)
-    assert not shim.mid_offers_tiles_c(first - 1, I) and shim.mid_offers_tiles_c(first, I)
+    for f32 in (0, 1):
+        assert shim.mid_takes_c(top, 10, I, f4, f32) and not shim.mid_takes_c(top + 1, 10, I, f4, f32)
+        assert shim.mid_takes_c(top, 1, I, f4, f32) and not shim.mid_takes_c(top + 1, 1, I, f4, f32)
+        assert shim.mid_takes_c(10 * top // 16, 16, I, f4, f32)
+        assert bool(shim.mid_takes_c(10 * top // 16 + 1, 16, I, f4, f32)) == bool(f32)   # fp32 results: by rows alone
+        assert not shim.mid_takes_c(top + 1, 16, I, f4, f32)
+    assert not shim.mid_offers_tiles_c(first - 1, I, 0) and shim.mid_offers_tiles_c(first, I, 0)
+    assert not shim.mid_offers_tiles_c(first, I, 1) and not shim.mid_offers_tiles_c(top, I, 1)
     for T in (first, 600, 601, 1229, top):
         for K in (10, 16):
-            if not shim.mid_takes_c(T, K, I, f4):
+            if not shim.mid_takes_c(T, K, I, f4, 0):
                 continue
             m = layout(shim, T, H, I, E, K, True, GU_F4 if f4 else GU_I8, GU_F4 if f4 else DN_I8)[2]
             mt = 16 * shim.mid_token_tiles_c(T, E, K, I, f4)
